@@ -1041,7 +1041,6 @@ int awamd_device_info(char *buf, int n) { return device_info(buf, n); }
 struct AwBatch {
     Batch batch;
     int tb_warm = BatchOptions().tile_warm;
-    int tb_opts = BatchOptions().tile_opts;
     int tb_tail = BatchOptions().tail_tile_cols;
 };
 
@@ -1084,7 +1083,6 @@ int awamd_batch_run_opts(void *b, int precision, int tile_cols, int traceback, i
     opt.prec = precision == 1 ? Precision::FP32 : Precision::FP64;
     opt.tile_cols = tile_cols;
     opt.tile_warm = ab.tb_warm;
-    opt.tile_opts = ab.tb_opts;
     opt.tail_tile_cols = ab.tb_tail;
     opt.traceback = traceback != 0;
     opt.fixup = fixup != 0;
@@ -1113,7 +1111,6 @@ int awamd_batch_set_traceback(void *b, int warm, int options)
         return -1;
     }
     ab.tb_warm = warm;
-    ab.tb_opts = options;
     return 0;
 }
 
@@ -1140,7 +1137,6 @@ int awamd_batch_run_ex(void *b, int precision, int tile_cols, int traceback, int
     opt.prec = precision == 1 ? Precision::FP32 : Precision::FP64;
     opt.tile_cols = tile_cols;
     opt.tile_warm = ab.tb_warm;
-    opt.tile_opts = ab.tb_opts;
     opt.tail_tile_cols = ab.tb_tail;
     opt.traceback = traceback != 0;
     opt.fixup = fixup != 0;
@@ -1163,7 +1159,7 @@ int awamd_batch_tune(void *b, int precision, const int *cand, int ncand, double 
 {
     AwBatch &ab = *reinterpret_cast<AwBatch *>(b);
     return ab.batch.tune_tiles(precision == 1 ? Precision::FP32 : Precision::FP64, cand, ncand,
-                               ms_out, ab.tb_warm, ab.tb_opts);
+                               ms_out, ab.tb_warm);
 }
 
 int awamd_batch_tune_forward(void *b, const int *tiles, const int *warms, int ncand, double tol,

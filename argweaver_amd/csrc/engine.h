@@ -54,6 +54,7 @@ struct DevInst {
     int last_state;           // the state of the last column when given, else -1 (sampled)
     int hostprep;             // the per-block inputs come from the host (internal threading)
     int *ldet;                // [B*RW] deterministic switch target of block b-1's states
+    unsigned short *pred;     // [B*RW] likeliest source in block b-1 of every state of block b
     double *lprior;           // [RW] first-column prior
     double *vemit;            // [nvar*RW] emissions of variant columns
     // outputs
@@ -105,7 +106,6 @@ struct RunStats {
     int nvar = 0;
     int tb_passes = 0;            // re-run passes of the tiled traceback
     long long tb_rerun_cols = 0;  // columns re-sampled by those passes
-    int tb_adopted = 0;           // tiles that took an alternative option
     double ms_fw_main = 0;        // the main forward launch (without re-runs and checks)
     int fw_tiles = 0;             // forward tiles launched
     int fw_reruns = 0;            // forward tiles re-run from their boundary column
@@ -131,21 +131,18 @@ struct HostInstance {
 
 // Schedule of a batch run.  The forward runs one wave per instance over
 // all of its columns, or, in FP32, one wave per forward tile (checked
-// speculative starts); the traceback runs one wave per option of a column
-// tile.
+// speculative starts); the traceback runs one workgroup per column tile.
 struct BatchOptions {
     Precision prec = Precision::FP64;
     int tile_cols = 0;       // traceback tile length (0: one tile per instance)
     int tile_warm = 256;     // warm-up columns of a speculative tile start
-    int tile_opts = 3;       // options per traceback tile (1 .. 4): the
-                             // speculative chain and its alternatives
     // traceback tile length of the instances whose FP32 forward tiles are
     // re-run: their traceback runs after the forward, when the rest of the
     // batch is done or on the other stream, so shorter tiles spread it over
     // more of the device (0: tile_cols)
     int tail_tile_cols = 4000;
     bool traceback = true;
-    bool fixup = true;       // false: speculative option-0 paths only (diagnostics)
+    bool fixup = true;       // false: speculative paths only (diagnostics)
     // FP32 forward tiles: long instances are split into tiles (counting the
     // warm-up) of fw_tile columns at a column cost of 0.94 us, scaled by
     // the column cost of the instance's states per lane, that run
@@ -190,10 +187,10 @@ public:
     // the traceback alone for each candidate tile length (0: one tile per
     // instance) on the resident tables; returns the fastest (ms per
     // candidate in ms_out when given), -1 on error.  Leaves the batch with
-    // the path of the last candidate.  warm / opts: the tiles' warm-up and
-    // options (BatchOptions::tile_warm, tile_opts).
+    // the path of the last candidate.  warm: the tiles' warm-up
+    // (BatchOptions::tile_warm).
     int tune_tiles(Precision prec, const int *cand, int ncand, double *ms_out = nullptr,
-                   int warm = BatchOptions().tile_warm, int opts = BatchOptions().tile_opts);
+                   int warm = BatchOptions().tile_warm);
     // FP32 forward-tile autotuner: times the forward (with its checks and
     // re-runs) for each (tile, warm-up) candidate and returns the index of
     // the fastest (-1 on error)

@@ -24,17 +24,12 @@
 //                  table, the result reaching each state by ds_bpermute; a
 //                  column costs O(S + T^2) and rows are written coalesced.
 //   k_lnl_b        per-instance sum of log normalisers (FP64)
-//   k_tb_spec      one wave per option of a column tile, every tile in one
-//                  launch: FP64 weights and CDF (DPP wave scan), rows
-//                  staged through LDS in double-buffered batches.  A tile
-//                  before the last runs a speculative chain (a state
-//                  sampled from a column past its end and a warm-up) and
-//                  alternative chains from the neighbouring states of that
-//                  chain's branch; once the true state at the tile's end is
-//                  known the option that started from it is exact
-//   k_tb_rerun     a tile no option fits, re-sampled from its true state
-//                  until it coalesces with an option's path (identical from
-//                  there on)
+//   traceback      one workgroup per column tile (traceback.hip).  A tile
+//                  before the last runs a speculative chain (a state sampled
+//                  from a column past its end and a warm-up); a tile whose
+//                  true state at its end proves to be another is re-run from
+//                  it until it meets the chain's path (identical from there
+//                  on)
 //
 // The forward kernel is a template over the table type: double is the
 // drop-in arithmetic (the reference's forward table to ~1e-15), float keeps
@@ -55,109 +50,11 @@
 #include <vector>
 
 #include "engine.h"
+#include "forward.h"
+#include "kernel_util.h"
+#include "traceback.h"
 
 namespace aw {
-
-#define HIP_OK(x)                                                                       \
-    do {                                                                                \
-        hipError_t e_ = (x);                                                            \
-        if (e_ != hipSuccess) {                                                         \
-            fprintf(stderr, "argweaver_amd: HIP error %s at %s:%d\n", hipGetErrorString(e_), \
-                    __FILE__, __LINE__);                                                \
-            return 1;                                                                   \
-        }                                                                               \
-    } while (0)
-
-// Pointers read out of DevInst are generic; accesses through them compile to
-// flat instructions, which count against the LDS wait counter too, so every
-// LDS wait would also drain outstanding HBM stores.  gp() restores the
-// global address space so loads and stores become global_* instructions.
-#define AW_GLOBAL __attribute__((address_space(1)))
-template <class X>
-__device__ inline AW_GLOBAL X *gp(X *p)
-{
-    return (AW_GLOBAL X *)p;
-}
-
-// Read-only data indexed by wave-uniform values (block bounds, uniforms)
-// goes through the constant address space so it is fetched with scalar loads.
-#define AW_CONST __attribute__((address_space(4)))
-template <class X>
-__device__ inline AW_CONST const X *cp(const X *p)
-{
-    return (AW_CONST const X *)p;
-}
-
-// LDS operations of one wave are performed in order, so inside a
-// single-wave workgroup only the compiler's order matters; every LDS access
-// of a kernel goes through one dynamic shared array, so accesses that may
-// overlap are never reordered.  This marks the places that rely on it.
-__device__ inline void lds_order() {}
-
-// index i such that off[i] <= x < off[i+1]
-template <class PT, class X>
-__device__ inline int find_owner(PT off, int n, X x)
-{
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (off[mid] <= x) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
-
-//===========================================================================
-// cross-lane moves (DPP).  A lane whose source is outside the wave (wave
-// shifts) or outside its 16-lane row (row shifts) receives 0.
-
-constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114,
-              DPP_ROW_SHR8 = 0x118, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138,
-              DPP_QUAD_SWAP1 = 0xB1;   // quad_perm [1,0,3,2]: lanes 2k and 2k+1 swap
-
-template <int CTRL>
-__device__ __forceinline__ int dpp_i(int x)
-{
-    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_r(float x)
-{
-    return __int_as_float(dpp_i<CTRL>(__float_as_int(x)));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp_r(double x)
-{
-    const long long v = __double_as_longlong(x);
-    const unsigned lo = (unsigned)dpp_i<CTRL>((int)v);
-    const unsigned hi = (unsigned)dpp_i<CTRL>((int)(v >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-__device__ __forceinline__ double readlane_d(double x, int l)
-{
-    const long long v = __double_as_longlong(x);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// inclusive prefix sum over the 64 lanes: Hillis-Steele inside each 16-lane
-// row, then the totals of the rows before
-__device__ __forceinline__ double wave_incl_scan(double v)
-{
-    v += dpp_r<DPP_ROW_SHR1>(v);
-    v += dpp_r<DPP_ROW_SHR2>(v);
-    v += dpp_r<DPP_ROW_SHR4>(v);
-    v += dpp_r<DPP_ROW_SHR8>(v);
-    const double t0 = readlane_d(v, 15), t1 = readlane_d(v, 31), t2 = readlane_d(v, 47);
-    const int row = threadIdx.x >> 4;
-    double off = 0.0;
-    if (row >= 1) off = t0;
-    if (row >= 2) off += t1;
-    if (row >= 3) off += t2;
-    return v + off;
-}
 
 //===========================================================================
 // column classification
@@ -810,563 +707,6 @@ __global__ __launch_bounds__(64) void k_var_emit_b(const DevInst *__restrict__ D
     }
 }
 
-//===========================================================================
-// forward recursion, one wave per instance (arghmm_forward_alg,
-// sample_thread.cpp:394-460; arghmm_forward_block :186-296;
-// arghmm_forward_switch :345-389)
-
-// NT1 is a compile-time bound on the T-1 time bins (19 for the usual 20
-// time points), so the per-time loops are fully unrolled without padding.
-//
-// Per block, each lane keeps in registers the factor planes of its R
-// states, two 0/1 factors per state (not the first / not the last state of
-// its branch: they cut the prefix and suffix sums), and whether the lane
-// holds a branch start / end (the carry stops there).  Per state it also
-// keeps its time, which gives both the lane holding the other-branch term
-// of its time and where its value goes in the per-time partial sums;
-// padding states use time bin 31, whose term is 0, so they come out 0 with
-// no mask.  The 0/1 factors are floats in both precisions: FP64 runs apply
-// them as selects, which keeps their registers at one per state.
-template <class Real, int R, int NT1>
-struct FwLane {
-    Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R];
-    float nf[R], nl[R];
-    int boff[R];     // 4 * time: ds_bpermute address of the lane holding TF[time]
-    Real m1, m2;
-    Real tmc[NT1];   // lane b < T-1: column b of the (a,b) table (FP32)
-};
-
-// x times a 0/1 factor m (a select in FP64: the same value)
-template <class Real>
-__device__ __forceinline__ Real keep(Real x, float m)
-{
-    if constexpr (sizeof(Real) == 4) return x * m;
-    else return (m != 0.f) ? x : Real(0);
-}
-
-// The (a,b) table lives in registers (lane b holds column b) for FP32 and
-// in LDS for FP64, where registers are short.
-template <class Real>
-constexpr bool tm_in_lds()
-{
-    return sizeof(Real) == 8;
-}
-
-// Per-time sums are accumulated in GCOPY copies of the 32 time bins, one
-// copy per group of 64 / GCOPY consecutive lanes, so that the LDS atomics of
-// one instruction seldom meet at one address (colliding atomics are
-// serialised).  Bin a, copy c sits at GP[a * GCOPY + c].  The sums are FP64
-// in both precisions: ds_add_f64 is much faster than ds_add_f32 here.
-constexpr int GCOPY = 16;
-
-template <class Real>
-__device__ __forceinline__ const AW_GLOBAL Real *planes(const DevInst &d, int b, int RW)
-{
-    if (sizeof(Real) == 4)
-        return (const AW_GLOBAL Real *)(gp(d.lcoef32) + (size_t)b * NCOEF * RW);
-    return (const AW_GLOBAL Real *)(gp(d.lcoef) + (size_t)b * NCOEF * RW);
-}
-
-template <class Real, int R, int NT1>
-__device__ __forceinline__ void fw_load_block(const DevInst &d, int b, FwLane<Real, R, NT1> &fl,
-                                              Real *TMS)
-{
-    constexpr int RW = 64 * R;
-    const int lane = threadIdx.x, T1 = d.T - 1;
-    // uniform bases, per-lane index: loads use the scalar-base address form
-    const AW_GLOBAL Real *coef = planes<Real>(d, b, RW);
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    int ti[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int x = r * 64 + lane;
-        fl.cf[r] = coef[CF * RW + x];
-        fl.cd[r] = coef[CD * RW + x];
-        fl.cg[r] = coef[CG * RW + x];
-        fl.ck[r] = coef[CK * RW + x];
-        fl.cj[r] = coef[CJ * RW + x];
-        fl.ce[r] = coef[CE * RW + x];
-        ti[r] = info[x];
-    }
-    bool first = false, last = false;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int t = ti[r] & INFO_TIME;
-        fl.nf[r] = (ti[r] & INFO_FIRST) ? 0.f : 1.f;
-        fl.nl[r] = (ti[r] & INFO_LAST) ? 0.f : 1.f;
-        fl.boff[r] = t * 4;
-        first |= (ti[r] & INFO_FIRST) != 0;
-        last |= (ti[r] & INFO_LAST) != 0;
-    }
-    fl.m1 = first ? Real(0) : Real(1);
-    fl.m2 = last ? Real(0) : Real(1);
-    // Loaded values go straight into their registers: selecting or copying
-    // a value whose load is still in flight makes the compiler wait for it
-    // at once.  Indices are clamped instead; entries a >= T-1 meet a zero
-    // per-time sum and lanes >= T-1 compute terms nobody uses.
-    const AW_GLOBAL double *tmb = gp(d.tm) + (size_t)b * T1 * T1;
-    const int lc = min(lane, T1 - 1);
-    if (tm_in_lds<Real>()) {
-        // TMS[a * 32 + b] = P(a -> b); lanes 32..63 duplicate lanes 0..31
-        double t[NT1];
-#pragma unroll
-        for (int a = 0; a < NT1; a++) t[a] = tmb[min(a, T1 - 1) * T1 + lc];
-#pragma unroll
-        for (int a = 0; a < NT1; a++)
-            if (lane < 32) TMS[a * 32 + lane] = (Real)t[a];
-    } else {
-#pragma unroll
-        for (int a = 0; a < NT1; a++) fl.tmc[a] = (Real)tmb[min(a, T1 - 1) * T1 + lc];
-    }
-}
-
-// variant row v, clamped to the last row (an instance without variant
-// columns has one allocated row that is never used)
-template <int R>
-__device__ __forceinline__ void vrow_load(const DevInst &d, int v, double (&ev)[R])
-{
-    constexpr int RW = 64 * R;
-    const AW_GLOBAL double *row = gp(d.vemit) + (size_t)max(min(v, d.nvar - 1), 0) * RW;
-#pragma unroll
-    for (int r = 0; r < R; r++) ev[r] = row[r * 64 + threadIdx.x];
-}
-
-// 1 / x: FP32 tables use the hardware reciprocal (within 1 ulp; the
-// normaliser itself, and so the log-likelihood, is kept exactly), FP64
-// tables the correctly rounded division
-__device__ __forceinline__ float recip(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double recip(double x) { return 1.0 / x; }
-
-template <class Real>
-__device__ __forceinline__ void lds_add(Real *p, Real v)
-{
-    (void)atomicAdd(p, v);
-}
-
-__device__ __forceinline__ float readlane_r(float x, int l)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
-}
-__device__ __forceinline__ double readlane_r(double x, int l)
-{
-    return readlane_d(x, l);
-}
-
-// x of the lane addr / 4 (ds_bpermute)
-__device__ __forceinline__ float bperm_r(float x, int addr)
-{
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
-}
-__device__ __forceinline__ double bperm_r(double x, int addr)
-{
-    const long long v = __double_as_longlong(x);
-    const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)v);
-    const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)(v >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// variant rows staged per LDS refill (at most 16 KB of them), and rows per
-// load batch of a refill (bounded by the registers they take)
-template <class Real, int R>
-constexpr int fw_vst()
-{
-    return (16384 / (64 * R * (int)sizeof(Real))) < 8 ? (16384 / (64 * R * (int)sizeof(Real))) : 8;
-}
-template <class Real, int R>
-constexpr int fw_vch()
-{
-    return (32 / R) < 2 ? 2 : (32 / R) > fw_vst<Real, R>() ? fw_vst<Real, R>() : (32 / R);
-}
-
-// LDS of the forward kernel, in Reals: partial sums, the previous column in
-// state order, the switch targets (plus one dummy slot per lane), staged
-// variant rows, the (a,b) table
-template <class Real, int R>
-constexpr int fw_lds_reals()
-{
-    return 32 * GCOPY * (int)(sizeof(double) / sizeof(Real)) + 64 * R + (64 * R + 64) +
-           fw_vst<Real, R>() * 64 * R + 31 * 32;
-}
-
-// A forward tile: columns [c0, c1) of an instance computed by one wave.
-// mode 0 starts from the prior at column 0.  mode 1 starts at c0 from a
-// uniform vector and stores nothing before cs (a warm-up: the filter
-// forgets its start).  mode 2 starts at c0 from the column held in boundary
-// slot bin (written by the tile before).  A tile with bout >= 0 also
-// computes column c1 into boundary slot bout, for the check of the next
-// tile's start.
-struct FwTile {
-    int inst;
-    int c0, cs, c1;
-    int mode;
-    int bout, bin;
-};
-constexpr int BND_STRIDE = 64 * 32;   // Reals per boundary slot (the largest row)
-
-// wave-wide maximum
-__device__ __forceinline__ double wave_max(double x)
-{
-    for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off));
-    return x;
-}
-
-// columns between the checks of a re-run tile against its stored columns
-constexpr int FW_RECHECK = 128;
-
-template <class Real, int R, int NT1>
-__device__ __forceinline__ void fw_instance(const DevInst d, Real *sm, const FwTile tile,
-                                            AW_GLOBAL Real *bnd, AW_GLOBAL double *bnorm,
-                                            double tol, AW_GLOBAL int *early)
-{
-    constexpr int RW = 64 * R;
-    constexpr int VST = fw_vst<Real, R>();
-    constexpr int VCH = fw_vch<Real, R>();
-    const int lane = threadIdx.x;
-    const int T1 = d.T - 1, L = d.L;
-    // carry steps: a branch has at most T-1 states, so it reaches back at
-    // most ceil((T-2)/R) lanes from the lane holding its last state
-    const int K = (T1 - 1 + R - 1) / R;
-    double *GP = (double *)sm;       // 32 x GCOPY: per-time partial sums
-    // byte offset of this lane's copy within a time bin's GCOPY copies
-    const int gslot = (lane / (64 / GCOPY)) * (int)sizeof(double);
-    // the half of bin lane>>1 that this lane reduces, and its read rotation
-    double *gq = GP + (lane >> 1) * GCOPY + (lane & 1) * (GCOPY / 2);
-    const int grot = (lane >> 1) & (GCOPY / 2 - 1);
-    Real *XS = (Real *)(GP + 32 * GCOPY);   // RW: previous column in state order (switch)
-    Real *NW = XS + RW;              // RW + 64: switch targets, then a dummy slot per lane
-    Real *VS = NW + RW + 64;         // VST rows: staged variant-column emissions
-    Real *TMS = VS + VST * RW;       // 31 x 32: the (a,b) table (FP64)
-    AW_GLOBAL Real *alpha = (AW_GLOBAL Real *)d.alpha;
-    auto norms = gp(d.norms);
-
-    const int c0 = tile.c0, cs = tile.cs;
-    // the last column computed: c1 - 1, or c1 into the boundary slot
-    const int clast = tile.bout >= 0 ? tile.c1 : tile.c1 - 1;
-    FwLane<Real, R, NT1> fl;
-    int b = find_owner(cp(d.bstart), d.B, c0);
-    int bend = cp(d.bstart)[b] + cp(d.blen)[b];
-    fw_load_block<Real, R, NT1>(d, b, fl, TMS);
-#pragma unroll
-    for (int k = 0; k < 32 * GCOPY / 64; k++) GP[k * 64 + lane] = 0.0;
-    // Column classes of a window of 64 columns, one per lane, read with
-    // readlane; the next window's are loaded a window ahead.  vmcnt counts
-    // the table stores too, so any wait on a load inside the column loop
-    // would also wait for the stores of the column before: the windows are
-    // an outer loop, and the one wait per window is taken there.
-    const AW_GLOBAL int *clsg = gp(d.cls);
-    int wb = c0 & ~63;
-    int clsv = clsg[min(wb + lane, L - 1)];
-    int clsn = clsg[min(wb + 64 + lane, L - 1)];
-    // Variant rows (row index = the column's class) are consumed in order
-    // and staged in LDS, VST at a time, so that a refill costs a few waits
-    // and the columns read their row from LDS.
-    int vbase = 0, vend = 0;
-
-    Real x[R], tfs[R], v[R];
-    Real sc = Real(1);   // the previous column is x * sc
-
-    // A re-run tile (mode 2) stops once a column it computes agrees with
-    // the column stored by its speculative run (relative tolerance tol):
-    // the filter is contractive, so the stored columns after it, the
-    // normalisers and the boundary column stay within tolerance.
-    bool rejoined = false;
-
-    // per-time sums, normaliser, stored row, other-branch term of the next
-    // column
-    auto finish = [&](int col, bool first) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-            lds_add((double *)((char *)GP + fl.boff[r] * (2 * GCOPY) + gslot), (double)v[r]);
-        // lane l takes the copies of bin l>>1 in its half (l&1), leaving 0
-        // (one exchange each; the LDS operations of one wave run in order).
-        // Step k reads copy (k + l/2) mod 8 of the half: the lanes of one
-        // step then spread over the banks (copy k of every bin would sit in
-        // two banks), which also fixes each lane's summation order
-        double q[GCOPY / 2];
-#pragma unroll
-        for (int k = 0; k < GCOPY / 2; k++)
-            q[k] = __longlong_as_double((long long)__hip_atomic_exchange(
-                (unsigned long long *)(gq + ((k + grot) & (GCOPY / 2 - 1))), 0ull,
-                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-#pragma unroll
-        for (int w = 1; w < GCOPY / 2; w *= 2)
-#pragma unroll
-            for (int k = 0; k < GCOPY / 2; k += 2 * w) q[k] += q[k + w];
-        const Real g = (Real)(q[0] + dpp_r<DPP_QUAD_SWAP1>(q[0]));   // lanes 2a, 2a+1: G[a]
-        // four interleaved partial sums keep the dependency chains short
-        Real nq[4] = {Real(0), Real(0), Real(0), Real(0)};
-        Real tq[4] = {Real(0), Real(0), Real(0), Real(0)};
-#pragma unroll
-        for (int a = 0; a < NT1; a++) {
-            const Real ga = readlane_r(g, 2 * a);
-            nq[a & 3] += ga;
-            tq[a & 3] += ga * (tm_in_lds<Real>() ? TMS[a * 32 + (lane & 31)] : fl.tmc[a]);
-        }
-        const Real norm = (nq[0] + nq[1]) + (nq[2] + nq[3]);
-        const Real t = (tq[0] + tq[1]) + (tq[2] + tq[3]);
-        // column 0 is stored unnormalised (scale 1); a restarted tile's first
-        // column is the boundary column as stored by the tile before
-        const Real nsc = (col == 0 || (first && tile.mode == 2)) ? Real(1) : recip(norm);
-        if (col >= cs && col < tile.c1) {
-            AW_GLOBAL Real *row = alpha + (size_t)col * RW;
-            if (tile.mode == 2 && !first && (col - tile.c0) % FW_RECHECK == 0) {
-                double dmax = 0.0, amax = 0.0;
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const double nv = (double)(v[r] * nsc), ov = (double)row[r * 64 + lane];
-                    dmax = fmax(dmax, fabs(nv - ov));
-                    amax = fmax(amax, fabs(nv));
-                }
-                dmax = wave_max(dmax);
-                amax = wave_max(amax);
-                rejoined = dmax <= tol * amax;
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) row[r * 64 + lane] = v[r] * nsc;
-            if (lane == 0) {
-                double nv = (col == 0) ? ((L == 1) ? (double)norm : 1.0) : (double)norm;
-                if (first && tile.mode == 2) nv = bnorm[tile.bin];
-                norms[col] = nv;
-            }
-        } else if (col == tile.c1) {
-            AW_GLOBAL Real *row = bnd + (size_t)tile.bout * BND_STRIDE;
-#pragma unroll
-            for (int r = 0; r < R; r++) row[r * 64 + lane] = v[r] * nsc;
-            if (lane == 0) bnorm[tile.bout] = (double)norm;
-        }
-        // TF[b] lives in lane b; lanes >= T-1 (padding bin 31) hold 0
-        const Real tv = (lane < T1) ? t * nsc : Real(0);
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            tfs[r] = bperm_r(tv, fl.boff[r]);
-            x[r] = v[r];
-        }
-        sc = nsc;
-    };
-
-    // first column.  mode 0: the unnormalised prior, not multiplied by the
-    // emission (calc_state_priors, trans.cpp:785-831); padding positions
-    // hold 0.  mode 1: 1 on every state.  mode 2: the boundary column.
-    if (tile.mode == 0) {
-        const AW_GLOBAL double *pr = gp(d.lprior);
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = (Real)pr[r * 64 + lane];
-    } else if (tile.mode == 1) {
-        const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = (lane * R + r < S) ? Real(1) : Real(0);
-    } else {
-        const AW_GLOBAL Real *src = bnd + (size_t)tile.bin * BND_STRIDE;
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = src[r * 64 + lane];
-    }
-    finish(c0, true);
-
-    // an empty asm reading the register makes the compiler complete its
-    // load here rather than at a use inside the column loop
-    asm volatile("" : "+v"(clsv));
-    int col = c0 + 1;
-    while (col <= clast && !rejoined) {
-        if (col >= wb + 64) {
-            wb += 64;
-            clsv = clsn;
-            asm volatile("" : "+v"(clsv));
-            clsn = clsg[min(wb + 64 + lane, L - 1)];
-        }
-        const int wend = min(wb + 63, clast);
-    for (; col <= wend; col++) {
-        const int cls = __builtin_amdgcn_readlane(clsv, col & 63);
-        const bool var = cls >= 0;
-        Real ev[R];
-        if (var) {
-            if (cls >= vend) {
-                vbase = cls;
-                vend = min(cls + VST, d.nvar);
-#pragma unroll
-                for (int k0 = 0; k0 < VST; k0 += VCH) {
-                    // VST need not be a multiple of VCH
-                    double buf[VCH][R];
-#pragma unroll
-                    for (int k = 0; k < VCH; k++)
-                        if (k0 + k < VST) vrow_load<R>(d, vbase + k0 + k, buf[k]);
-#pragma unroll
-                    for (int k = 0; k < VCH; k++)
-#pragma unroll
-                        for (int r = 0; r < R; r++)
-                            if (k0 + k < VST) VS[(k0 + k) * RW + r * 64 + lane] = (Real)buf[k][r];
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) ev[r] = VS[(cls - vbase) * RW + r * 64 + lane];
-        }
-
-        if (col == bend) {
-            // switch column: deterministic transitions scattered into NW
-            // (the recombination and recoalescence sources excluded), then
-            // the two dense rows.  Every load of the column is issued before
-            // the first use, branch-free, so the column waits once.
-            const int nb = b + 1;
-            const int so0 = cp(d.soff)[b], so1 = cp(d.soff)[nb];
-            const int S1 = so1 - so0, S2 = cp(d.soff)[nb + 1] - so1;
-            const int rs = cp(d.srcs)[2 * nb], cs = cp(d.srcs)[2 * nb + 1];
-            const AW_GLOBAL Real *swn = planes<Real>(d, nb, RW);
-            const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)nb * RW;
-            int dt[R];
-            Real dpv[R], rr[R], cr[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int x = r * 64 + lane;
-                dt[r] = detn[x];
-                dpv[r] = swn[CDP * RW + x];
-                rr[r] = swn[CRR * RW + x];
-                cr[r] = swn[CCR * RW + x];
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                XS[lane * R + r] = x[r];   // padding slots (s >= S1) are never read
-                NW[r * 64 + lane] = Real(0);
-            }
-            b = nb;
-            bend += cp(d.blen)[nb];
-            fw_load_block<Real, R, NT1>(d, b, fl, TMS);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int s = lane * R + r;
-                const bool ok = s < S1 && dt[r] >= 0 && s != rs && s != cs;
-                lds_add(&NW[ok ? dt[r] : RW + lane], ok ? x[r] * dpv[r] : Real(0));
-            }
-            const Real prs = (rs != -1) ? XS[max(rs, 0)] * sc : Real(0);
-            const Real pcs = (cs != -1) ? XS[max(cs, 0)] * sc : Real(0);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int s = lane * R + r;
-                const Real e = var ? ev[r] : (cls == -1) ? fl.ce[r] : Real(1);
-                Real acc = (s < S2) ? NW[s] * sc : Real(0);
-                if (rs != -1 && rr[r] > Real(0)) acc += prs * rr[r];
-                if (cs != -1 && cr[r] > Real(0)) acc += pcs * cr[r];
-                v[r] = (s < S2) ? acc * e : Real(0);
-            }
-        } else {
-            // same-branch prefix sums (younger states) with the carry from
-            // the lanes before, suffix sums (older states) with the carry
-            // from the lanes after
-            Real P[R], Q[R];
-            Real p = Real(0);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                P[r] = keep(p, fl.nf[r]);
-                p = fl.cf[r] * x[r] + P[r];
-            }
-            Real q = Real(0);
-#pragma unroll
-            for (int r = R - 1; r >= 0; r--) {
-                Q[r] = keep(q, fl.nl[r]);
-                q = fl.cd[r] * x[r] + Q[r];
-            }
-            Real c1 = Real(0), c2 = Real(0);
-            for (int k = 0; k < K; k++) {
-                c1 = dpp_r<DPP_WAVE_SHR1>(fl.m1 * c1 + p);
-                c2 = dpp_r<DPP_WAVE_SHL1>(fl.m2 * c2 + q);
-            }
-            // the carry reaches the slots before the lane's first branch
-            // start (prefix) / after its last branch end (suffix)
-            Real f1 = Real(1);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                f1 = keep(f1, fl.nf[r]);
-                P[r] += c1 * f1;
-            }
-            Real f2 = Real(1);
-#pragma unroll
-            for (int r = R - 1; r >= 0; r--) {
-                f2 = keep(f2, fl.nl[r]);
-                Q[r] += c2 * f2;
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const Real e = var ? ev[r] : (cls == -1) ? fl.ce[r] : Real(1);
-                const Real same = (fl.cg[r] * P[r] + fl.ck[r] * Q[r]) + fl.cj[r] * x[r];
-                v[r] = e * (tfs[r] + sc * same);
-            }
-        }
-        finish(col, false);
-        if (rejoined) break;
-    }
-    }
-    // the column after the one that rejoined (never 0), else 0
-    if (early && lane == 0) *early = rejoined ? col + 1 : 0;
-}
-
-// One launch covers every instance of a batch, whatever its states-per-lane
-// count: waves of different R run side by side from the start, with no
-// dependence on how streams map to hardware queues.
-// REDO marks the launches of re-run tiles (a separate symbol, so that
-// profiles report the main forward launch on its own).  BIG: the instances
-// with 32 states per lane (blocks of 1025-2048 states) run in a symbol of
-// their own, launched over the same tiles, so that their register demand
-// (spilled to AGPRs and scratch) does not weigh on the others.
-template <class Real, int NT1, bool REDO, bool BIG>
-__global__ __launch_bounds__(64) void k_fw_all(const DevInst *__restrict__ D,
-                                               const FwTile *__restrict__ tiles,
-                                               Real *__restrict__ bnd, double *__restrict__ bnorm,
-                                               double tol, int *__restrict__ early)
-{
-    extern __shared__ __align__(16) double fw_dyn[];
-    const FwTile t = tiles[blockIdx.x];
-    const DevInst &d = D[t.inst];
-    Real *sm = (Real *)fw_dyn;
-    AW_GLOBAL Real *bg = (AW_GLOBAL Real *)bnd;
-    AW_GLOBAL double *ng = (AW_GLOBAL double *)bnorm;
-    AW_GLOBAL int *eg = early ? (AW_GLOBAL int *)(early + blockIdx.x) : nullptr;
-    if ((d.R > 16) != BIG) return;   // the other symbol's tile
-    if constexpr (BIG) {
-        fw_instance<Real, 32, NT1>(d, sm, t, bg, ng, tol, eg);
-    } else {
-        switch (d.R) {
-        case 1: fw_instance<Real, 1, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 2: fw_instance<Real, 2, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 4: fw_instance<Real, 4, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 6: fw_instance<Real, 6, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 8: fw_instance<Real, 8, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 12: fw_instance<Real, 12, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        default: fw_instance<Real, 16, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        }
-    }
-}
-
-// Check of a speculative forward tile's start: the boundary column computed
-// by the tile before (slot bin) against the tile's own stored column c0,
-// both normalised.  flag = 1 when they differ by more than tol relative to
-// the column's largest entry, or the normalisers by more than tol.
-template <class Real>
-__global__ __launch_bounds__(64) void k_fw_check(const DevInst *__restrict__ D,
-                                                 const FwTile *__restrict__ tiles,
-                                                 const int *__restrict__ idx,
-                                                 const Real *__restrict__ bnd,
-                                                 const double *__restrict__ bnorm, double tol,
-                                                 int *__restrict__ flags)
-{
-    const FwTile t = tiles[idx[blockIdx.x]];
-    const DevInst &d = D[t.inst];
-    const int RW = 64 * d.R, lane = threadIdx.x;
-    const Real *a = (const Real *)d.alpha + (size_t)t.cs * RW;
-    const Real *q = bnd + (size_t)t.bin * BND_STRIDE;
-    double dmax = 0.0, amax = 0.0;
-    for (int x = lane; x < RW; x += 64) {
-        dmax = fmax(dmax, fabs((double)a[x] - (double)q[x]));
-        amax = fmax(amax, fabs((double)q[x]));
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        dmax = fmax(dmax, __shfl_xor(dmax, off));
-        amax = fmax(amax, __shfl_xor(amax, off));
-    }
-    if (lane == 0) {
-        const double n0 = gp(d.norms)[t.cs], n1 = bnorm[t.bin];
-        const bool bad = !(dmax <= tol * amax) || !(fabs(n0 - n1) <= tol * fabs(n1));
-        flags[blockIdx.x] = bad ? 1 : 0;
-    }
-}
-
 // log-likelihood: sum of log column normalisers
 __global__ __launch_bounds__(256) void k_lnl_b(const DevInst *__restrict__ D,
                                                const int *__restrict__ list)
@@ -1382,544 +722,6 @@ __global__ __launch_bounds__(256) void k_lnl_b(const DevInst *__restrict__ D,
         __syncthreads();
     }
     if (threadIdx.x == 0) *d.lnl = part[0];
-}
-
-//===========================================================================
-// stochastic traceback (stochastic_traceback, sample_thread.cpp:522-569;
-// sample_hmm_posterior_step :506-519; sample, common.h:272-290)
-
-struct Chunk {
-    int inst, c0, c1;        // columns [c0, c1) of instance inst
-    int cw;                  // column where the speculative chain starts (>= c1)
-    int first, last;         // first / last tile of its instance
-    long long coff;          // the tile's alternative paths in the option buffer
-};
-
-// Options of a traceback tile.  Option 0 is the speculative chain: a state
-// sampled from column cw alone, a warm-up back to column c1 (not stored),
-// then the tile's columns into the path.  Options 1 .. K-1 are chains of the
-// same tile started at column c1 from the other states of the branch that
-// option 0 holds there (the most probable first, by the forward column):
-// two backward chains on one branch at neighbouring times can run side by
-// side for tens of thousands of columns with the same uniforms, and one of
-// them is then the true chain.  Each option records the state it starts
-// from at c1 and the state it reaches at c0; once the true state at c1 is
-// known, an option that started from it is the tile's exact path.
-constexpr int TB_KMAX = 4;
-
-template <int R>
-struct TbLane {
-    int ti[R];
-    int node[R];   // node of the state (info_node)
-    int off1[R];   // a * (T-1): other-branch entry P(a -> b) at off1 + b
-    int off2[R];   // same-branch entry P(a -> b) at off2 + b
-    int dt[R];     // deterministic switch target into the next block
-    double dp[R];  // and its weight
-};
-
-// LDS tables of block b: the (a,b) table followed by the (c,a,b) table, in
-// the run's precision, copied with every load of a lane in flight at once
-// (TCP per round)
-template <class Real, int R>
-__device__ __forceinline__ void tb_load_block(const DevInst &d, int b, TbLane<R> &tl, Real *tab)
-{
-    constexpr int RW = 64 * R;
-    const int lane = threadIdx.x, T1 = d.T - 1, TT = T1 * T1;
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    // switch into block b+1 from this block's states (the last block
-    // re-reads its own entries, never used)
-    const int bn = min(b + 1, d.B - 1);
-    const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)bn * RW;
-    const AW_GLOBAL Real *dpn = planes<Real>(d, bn, RW) + CDP * RW;
-    const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * TT;
-    const AW_GLOBAL double *tm2 = gp(d.tm2s) + (size_t)b * d.TC;
-    const int n = TT + d.TC;
-    constexpr int TCP = sizeof(Real) == 4 ? 48 : 24;
-    for (int base = 0; base < n; base += 64 * TCP) {
-        double t[TCP];
-#pragma unroll
-        for (int k = 0; k < TCP; k++) {
-            const int x = min(base + k * 64 + lane, n - 1);
-            const AW_GLOBAL double *src = (x < TT) ? tm + x : tm2 + (x - TT);
-            t[k] = *src;
-        }
-        if (base == 0) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                tl.ti[r] = info[r * 64 + lane];
-                tl.dt[r] = detn[r * 64 + lane];
-                tl.dp[r] = dpn[r * 64 + lane];
-            }
-        }
-        // entries past the end repeat the last one (same index, same value):
-        // a per-entry condition would become a branch per store
-#pragma unroll
-        for (int k = 0; k < TCP; k++) tab[min(base + k * 64 + lane, n - 1)] = (Real)t[k];
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        // padding slots carry time bin 31: clamp so their (zero-weighted)
-        // table reads stay inside the tables
-        const int a = min(tl.ti[r] & INFO_TIME, T1 - 1), c = info_age(tl.ti[r]);
-        tl.node[r] = info_node(tl.ti[r]);
-        tl.off1[r] = a * T1;
-        tl.off2[r] = TT + tc_base(c, T1) + (a - c) * (T1 - c) - c;
-    }
-}
-
-// First index k of the lane-run weights (lane l holds states l*R..l*R+R-1)
-// whose cumulative sum reaches u * total; S-1 if none does.  Returns k and
-// the info word of state k in kinfo.  pre[r] = w[0] + ... + w[r] of the
-// lane.  Branch-free: the owner lane counts the prefixes below the pick.
-template <int R>
-__device__ __forceinline__ int lane_sample(const double (&pre)[R], const int (&ti)[R], int S,
-                                           double u, int &kinfo)
-{
-    const int lane = threadIdx.x;
-    const double loc = pre[R - 1];
-    const double inc = wave_incl_scan(loc);
-    const double excl = dpp_r<DPP_WAVE_SHR1>(inc);
-    const double total = readlane_d(inc, 63);
-    const double pick = u * total;
-    const bool has = lane * R < S;
-    const unsigned long long m = __ballot(has && excl + loc >= pick);
-    const int owner = m ? (int)__ffsll((long long)m) - 1 : (S - 1) / R;
-    const int nloc = min(R, S - lane * R);
-    const double thr = pick - excl;
-    int cnt = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) cnt += (pre[r] < thr) ? 1 : 0;
-    const int rsel = m ? min(cnt, nloc - 1) : nloc - 1;
-    // select ti[rsel] with masks (a compare-and-branch form becomes a
-    // dynamically indexed scratch array)
-    int inf = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) inf |= ti[r] & -(int)(r == rsel);
-    kinfo = __builtin_amdgcn_readlane(inf, owner);
-    return __builtin_amdgcn_readlane(lane * R + rsel, owner);
-}
-
-// forward-table rows staged per traceback batch: about TB_ROWREG registers
-// of a lane hold the next batch.  Fewer rows per batch mean less LDS per
-// tile: at 48 an FP32 tile with 20 time points takes about 35 KB, so four
-// tiles fit on a CU (three at 64); at 32 the batches of R = 12 and 16 are
-// too short to hide the row loads.
-constexpr int TB_ROWREG = 48;
-template <class Real, int R>
-constexpr int tb_batch()
-{
-    return (TB_ROWREG / (R * (int)(sizeof(Real) / 4))) > 16 ? 16
-         : (TB_ROWREG / (R * (int)(sizeof(Real) / 4))) < 2 ? 2
-                                                           : (TB_ROWREG / (R * (int)(sizeof(Real) / 4)));
-}
-// host mirror of tb_batch
-inline int tb_batch_host(int R, size_t rsz)
-{
-    return std::max(2, std::min(16, TB_ROWREG / (R * (int)(rsz / 4))));
-}
-
-template <class Real, int R>
-__device__ __forceinline__ void row_load(AW_GLOBAL const Real *alpha, int col, Real (&rv)[R])
-{
-    constexpr int RW = 64 * R;
-    AW_GLOBAL const Real *row = alpha + (size_t)col * RW;
-#pragma unroll
-    for (int r = 0; r < R; r++) rv[r] = row[r * 64 + threadIdx.x];
-}
-
-// The state of a backward chain: the state k sampled at the column last
-// visited, its info word, and the block of that column.
-struct Chain {
-    int k, info, blk;
-};
-
-// Stored paths a re-run compares its samples with (option 0 in the path,
-// the alternatives in the option buffer), each indexed by column; null for
-// an option not compared.
-struct Cmp {
-    const AW_GLOBAL int *p[TB_KMAX];
-};
-
-// Sample columns hi, hi-1, .., lo given the chain's state at column hi+1,
-// storing the samples of columns <= whi through dst (dst[c] for column c;
-// nothing when dst is null).  The walk stops at the first column whose
-// sample equals a compared stored path o (the chains have coalesced: the
-// rest is that path) and returns it with opt = o; else it returns -1 with
-// the chain at column lo.  The uniform of column col is u[L-1-col].
-//
-// Rows come through LDS in batches of BT columns, double-buffered: the
-// loads of the next batch are issued when a batch starts and written to
-// LDS when it ends, so the column loop itself never waits on HBM (vmcnt
-// orders loads behind stores, so a per-column prefetch would not hide it).
-// The uniforms and the stored paths come 64 columns at a time, one per
-// lane, read with readlane.
-template <class Real, int R>
-__device__ __forceinline__ int tb_range(const DevInst &d, Real *tab, Real *rows, int hi, int lo,
-                                        Chain &chn, AW_GLOBAL int *dst, int whi, const Cmp &cmp,
-                                        int &opt)
-{
-    constexpr int RW = 64 * R;
-    constexpr int BT = tb_batch<Real, R>();
-    const int lane = threadIdx.x, L = d.L;
-    AW_GLOBAL const Real *alpha = (AW_GLOBAL const Real *)d.alpha;
-    const AW_GLOBAL double *ug = gp(d.u);
-    opt = -1;
-    if (hi < lo) return -1;
-    int knext = chn.k, kinfo = chn.info, kblk = chn.blk;
-    int bc = find_owner(cp(d.bstart), d.B, hi);
-    int bc_start = cp(d.bstart)[bc];
-    int S = cp(d.soff)[bc + 1] - cp(d.soff)[bc];
-    TbLane<R> tl;
-    tb_load_block<Real, R>(d, bc, tl, tab);
-    // window of 64 columns w0, w0-1, .., w0-63: lane j holds column w0-j
-    // (its uniform, the stored paths, and the sampled state, which is
-    // stored once per window: per-column stores would make every later load
-    // wait for them, vmcnt being in order)
-    int w0 = hi;
-    double uw = ug[min(L - 1 - (w0 - lane), L - 1)];
-    // stored paths are read within the walked columns [lo, hi] only
-    int pw[TB_KMAX];
-#pragma unroll
-    for (int o = 0; o < TB_KMAX; o++) pw[o] = cmp.p[o] ? cmp.p[o][max(w0 - lane, lo)] : -1;
-    int pnew = 0;
-    // store the sampled states of the window's columns w0 .. clo
-    auto flush = [&](int clo) {
-        const int c = w0 - lane;
-        if (dst && c >= clo && c <= min(w0, whi)) dst[c] = pnew;
-    };
-    Real nxt[BT][R];
-#pragma unroll
-    for (int k = 0; k < BT; k++) row_load<Real, R>(alpha, max(hi - k, lo), nxt[k]);
-#pragma unroll
-    for (int k = 0; k < BT; k++)
-#pragma unroll
-        for (int r = 0; r < R; r++) rows[k * RW + r * 64 + lane] = nxt[k][r];
-    int buf = 0;
-    for (int top = hi; top >= lo; top -= BT) {
-        const int bot = max(top - BT + 1, lo);
-#pragma unroll
-        for (int k = 0; k < BT; k++) row_load<Real, R>(alpha, max(top - BT - k, lo), nxt[k]);
-        const Real *rb = rows + buf * BT * RW;
-        for (int col = top; col >= bot; col--) {
-            if (w0 - col >= 64) {
-                flush(col + 1);
-                w0 = col;
-                uw = ug[min(L - 1 - (w0 - lane), L - 1)];
-#pragma unroll
-                for (int o = 0; o < TB_KMAX; o++)
-                    if (cmp.p[o]) pw[o] = cmp.p[o][max(w0 - lane, lo)];
-            }
-            const double uval = readlane_d(uw, w0 - col);
-            const Real *row = rb + (top - col) * RW;
-            // every load first, then the weights: per-slot conditions around
-            // a load would give each load its own wait
-            Real rv[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) rv[r] = row[r * 64 + lane];
-            Real tr[R];
-            if (bc != kblk) {
-                // col is the last column of block bc: switch into kblk = bc+1
-                // (TransMatrixSwitch::get, trans.h:201-209)
-                const int rs = cp(d.srcs)[2 * kblk], cs = cp(d.srcs)[2 * kblk + 1];
-                const int pk = lane_pos(knext, R);
-                const AW_GLOBAL Real *cn = planes<Real>(d, kblk, RW);
-                const double rrk = cn[CRR * RW + pk], crk = cn[CCR * RW + pk];
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const int s = lane * R + r;
-                    tr[r] = (Real)((s == cs) ? crk : (s == rs) ? rrk : (tl.dt[r] == knext ? tl.dp[r] : 0.0));
-                }
-            } else {
-                const int nk = info_node(kinfo), bk = kinfo & INFO_TIME;
-#pragma unroll
-                for (int r = 0; r < R; r++) tr[r] = tab[(tl.node[r] == nk ? tl.off2[r] : tl.off1[r]) + bk];
-            }
-            // padding slots hold 0 in the table, so their weights are 0; the
-            // product is in the table's precision, the cumulative sums FP64
-            double pre[R];
-            double acc = 0.0;
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                acc += (double)(rv[r] * tr[r]);
-                pre[r] = acc;
-            }
-            knext = lane_sample<R>(pre, tl.ti, S, uval, kinfo);
-            kblk = bc;
-            int hit = -1;
-#pragma unroll
-            for (int o = TB_KMAX - 1; o >= 0; o--)
-                if (cmp.p[o] && __builtin_amdgcn_readlane(pw[o], w0 - col) == knext) hit = o;
-            if (hit >= 0) {
-                flush(col + 1);
-                chn = Chain{knext, kinfo, kblk};
-                opt = hit;
-                return col;
-            }
-            pnew = (lane == w0 - col) ? knext : pnew;
-            if (col - 1 < bc_start && col - 1 >= lo) {
-                bc--;
-                bc_start = cp(d.bstart)[bc];
-                S = cp(d.soff)[bc + 1] - cp(d.soff)[bc];
-                tb_load_block<Real, R>(d, bc, tl, tab);
-            }
-        }
-        buf ^= 1;
-        Real *wb = rows + buf * BT * RW;
-#pragma unroll
-        for (int k = 0; k < BT; k++)
-#pragma unroll
-            for (int r = 0; r < R; r++) wb[k * RW + r * 64 + lane] = nxt[k][r];
-        lds_order();
-    }
-    flush(lo);
-    chn = Chain{knext, kinfo, kblk};
-    return -1;
-}
-
-// state sampled from column col alone (the last column, or the speculative
-// start of a tile)
-template <class Real, int R>
-__device__ __forceinline__ Chain tb_column(const DevInst &d, int col, double uval)
-{
-    constexpr int RW = 64 * R;
-    AW_GLOBAL const Real *alpha = (AW_GLOBAL const Real *)d.alpha;
-    const int b = find_owner(cp(d.bstart), d.B, col);
-    const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    Real rv[R];
-    row_load<Real, R>(alpha, col, rv);
-    int ti[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) ti[r] = info[r * 64 + threadIdx.x];
-    double pre[R];
-    double acc = 0.0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        acc += (double)rv[r];   // padding slots hold 0
-        pre[r] = acc;
-    }
-    Chain c;
-    c.k = lane_sample<R>(pre, ti, S, uval, c.info);
-    c.blk = b;
-    return c;
-}
-
-// The alternative start of option o >= 1 at column col: among the other
-// states of the branch of state k0 (block b), the one of rank o - 1 by the
-// forward column (ties by state index); -1 when the branch has too few.
-// Lane l looks at state k0 - 31 + l: a branch has fewer than 32 states.
-template <class Real, int R>
-__device__ __forceinline__ int tb_alternative(const DevInst &d, int col, int b, int k0, int o)
-{
-    constexpr int RW = 64 * R;
-    const int lane = threadIdx.x;
-    const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    AW_GLOBAL const Real *row = (AW_GLOBAL const Real *)d.alpha + (size_t)col * RW;
-    const int node = info_node(info[lane_pos(k0, R)]);
-    const int x = k0 - 31 + lane;
-    const bool ok = x >= 0 && x < S && x != k0 && info_node(info[lane_pos(min(max(x, 0), S - 1), R)]) == node;
-    const double v = ok ? (double)row[lane_pos(min(max(x, 0), S - 1), R)] : -1.0;
-    // rank among the candidates: those with a larger value, or an equal
-    // value and a smaller index
-    int rank = 0;
-    for (int j = 0; j < 64; j++) {
-        const double vj = readlane_d(v, j);
-        rank += (vj > v || (vj == v && j < lane)) ? 1 : 0;
-    }
-    const unsigned long long m = __ballot(ok && rank == o - 1);
-    if (!m) return -1;
-    return __builtin_amdgcn_readlane(x, (int)__ffsll((long long)m) - 1);
-}
-
-// The option buffer column c of option o >= 1 of tile ch (dst[c] / src[c]).
-__device__ __forceinline__ AW_GLOBAL int *opt_path(int *obuf, const Chunk &ch, int o)
-{
-    return (AW_GLOBAL int *)obuf + ch.coff + (long long)(o - 1) * (ch.c1 - ch.c0) - ch.c0;
-}
-
-// One option of a tile (the speculative launch).  ostart / oend receive the
-// option's state at column c1 (-1: no such option) and at column c0.
-template <class Real, int R>
-__device__ __forceinline__ void tb_option(const DevInst d, const Chunk &ch, int o, int K, int *obuf,
-                                          int *ostart, int *oend, void *lds)
-{
-    Real *tab = (Real *)lds;
-    Real *rows = tab + (d.T - 1) * (d.T - 1) + d.TC;
-    constexpr int RW = 64 * R;
-    const int L = d.L;
-    AW_GLOBAL int *path = gp(d.path);
-    const Cmp none{{nullptr, nullptr, nullptr, nullptr}};
-    int dummy;
-    Chain c;
-    if (ch.last) {
-        // the last tile is exact: option 0 only
-        if (o > 0) {
-            if (threadIdx.x == 0) *ostart = *oend = -1;
-            return;
-        }
-        if (d.last_state >= 0) {
-            // conditioned on the last column's state
-            c.blk = d.B - 1;
-            c.k = d.last_state;
-            c.info = gp(d.linfo)[(size_t)c.blk * RW + lane_pos(c.k, R)];
-        } else {
-            c = tb_column<Real, R>(d, L - 1, cp(d.u)[0]);
-        }
-        if (threadIdx.x == 0) path[L - 1] = c.k;
-        tb_range<Real, R>(d, tab, rows, L - 2, ch.c0, c, path, L - 2, none, dummy);
-        if (threadIdx.x == 0) {
-            *ostart = -1;
-            *oend = c.k;
-        }
-        return;
-    }
-    // the speculative chain's warm-up, the same in every option
-    c = tb_column<Real, R>(d, ch.cw, cp(d.u)[L - 1 - ch.cw]);
-    tb_range<Real, R>(d, tab, rows, ch.cw - 1, ch.c1, c, nullptr, -1, none, dummy);
-    AW_GLOBAL int *dst = path;
-    if (o > 0) {
-        const int k = tb_alternative<Real, R>(d, ch.c1, c.blk, c.k, o);
-        if (k < 0) {
-            if (threadIdx.x == 0) *ostart = *oend = -1;
-            return;
-        }
-        c.k = k;
-        c.info = gp(d.linfo)[(size_t)c.blk * RW + lane_pos(k, R)];
-        dst = opt_path(obuf, ch, o);
-    }
-    const int start = c.k;
-    tb_range<Real, R>(d, tab, rows, ch.c1 - 1, ch.c0, c, dst, ch.c1 - 1, none, dummy);
-    if (threadIdx.x == 0) {
-        *ostart = start;
-        *oend = c.k;
-    }
-    (void)K;
-}
-
-// Re-run of a tile from its true state at column c1 until it coalesces with
-// one of its options' stored paths; the path then follows that option (an
-// alternative's columns are copied in).  res: the column of coalescence (-1
-// for none), the option, and the state at column c0.
-template <class Real, int R>
-__device__ __forceinline__ void tb_rerun(const DevInst d, const Chunk &ch, int k1, int K, int *obuf,
-                                         const int *ostart, int *res, void *lds)
-{
-    Real *tab = (Real *)lds;
-    Real *rows = tab + (d.T - 1) * (d.T - 1) + d.TC;
-    constexpr int RW = 64 * R;
-    AW_GLOBAL int *path = gp(d.path);
-    Cmp cmp{{path, nullptr, nullptr, nullptr}};
-#pragma unroll
-    for (int o = 1; o < TB_KMAX; o++)
-        if (o < K && ostart[o] >= 0) cmp.p[o] = opt_path(obuf, ch, o);
-    Chain c;
-    c.blk = find_owner(cp(d.bstart), d.B, ch.c1);
-    c.k = k1;
-    c.info = gp(d.linfo)[(size_t)c.blk * RW + lane_pos(k1, R)];
-    int hit;
-    const int col = tb_range<Real, R>(d, tab, rows, ch.c1 - 1, ch.c0, c, path, ch.c1 - 1, cmp, hit);
-    int end = c.k;
-    const int o = (col >= 0) ? hit : -1;
-    if (col >= 0) {
-        if (o > 0) {
-            // the rest of the tile is the alternative's
-            const AW_GLOBAL int *src = opt_path(obuf, ch, o);
-            for (int cc = ch.c0 + (int)threadIdx.x; cc <= col; cc += 64) path[cc] = src[cc];
-            end = src[ch.c0];
-        } else {
-            end = path[ch.c0];
-        }
-    }
-    if (threadIdx.x == 0) {
-        res[0] = col;
-        res[1] = o;
-        res[2] = end;
-    }
-}
-
-// Launch of the speculative options of the tiles list[0..nlist): block
-// (jj, o) of tile list[jj], option o sits at 8 * (K * (jj / 8) + o) + jj % 8,
-// so the options of a tile run on one XCD (blocks go round-robin over the
-// eight) and share its L2 for their rows.
-// BIG: the tiles of instances with 32 states per lane (a symbol of their own,
-// as for the forward)
-template <class Real, bool BIG>
-__global__ __launch_bounds__(64) void k_tb_spec(const DevInst *__restrict__ D,
-                                                const Chunk *__restrict__ chunks,
-                                                const int *__restrict__ list, int nlist, int K,
-                                                int *__restrict__ obuf, int *__restrict__ ostart,
-                                                int *__restrict__ oend)
-{
-    extern __shared__ double tb_dyn[];
-    const int bx = blockIdx.x;
-    const int jj = (bx / (8 * K)) * 8 + bx % 8, o = (bx / 8) % K;
-    if (jj >= nlist) return;
-    const int j = list[jj];
-    const Chunk ch = chunks[j];
-    const DevInst &d = D[ch.inst];
-    int *os = ostart + (size_t)j * K + o, *oe = oend + (size_t)j * K + o;
-    if ((d.R > 16) != BIG) return;   // the other symbol's tile
-    if constexpr (BIG) {
-        tb_option<Real, 32>(d, ch, o, K, obuf, os, oe, tb_dyn);
-    } else {
-        switch (d.R) {
-        case 1: tb_option<Real, 1>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        case 2: tb_option<Real, 2>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        case 4: tb_option<Real, 4>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        case 6: tb_option<Real, 6>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        case 8: tb_option<Real, 8>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        case 12: tb_option<Real, 12>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        default: tb_option<Real, 16>(d, ch, o, K, obuf, os, oe, tb_dyn); break;
-        }
-    }
-}
-
-// Re-runs: block x re-samples tile idx[x] from state k1[x] at its column c1.
-template <class Real, bool BIG>
-__global__ __launch_bounds__(64) void k_tb_rerun(const DevInst *__restrict__ D,
-                                                 const Chunk *__restrict__ chunks,
-                                                 const int *__restrict__ idx,
-                                                 const int *__restrict__ k1, int K,
-                                                 int *__restrict__ obuf,
-                                                 const int *__restrict__ ostart,
-                                                 int *__restrict__ res)
-{
-    extern __shared__ double tb_dyn[];
-    const int j = idx[blockIdx.x];
-    const Chunk ch = chunks[j];
-    const DevInst &d = D[ch.inst];
-    const int *os = ostart + (size_t)j * K;
-    int *rs = res + 3 * blockIdx.x;
-    const int k = k1[blockIdx.x];
-    if ((d.R > 16) != BIG) return;   // the other symbol's tile
-    if constexpr (BIG) {
-        tb_rerun<Real, 32>(d, ch, k, K, obuf, os, rs, tb_dyn);
-    } else {
-        switch (d.R) {
-        case 1: tb_rerun<Real, 1>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        case 2: tb_rerun<Real, 2>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        case 4: tb_rerun<Real, 4>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        case 6: tb_rerun<Real, 6>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        case 8: tb_rerun<Real, 8>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        case 12: tb_rerun<Real, 12>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        default: tb_rerun<Real, 16>(d, ch, k, K, obuf, os, rs, tb_dyn); break;
-        }
-    }
-}
-
-// Adopted alternatives: block x copies option opt[x] of tile idx[x] into the
-// path over the tile's columns.
-__global__ __launch_bounds__(256) void k_tb_adopt(const DevInst *__restrict__ D,
-                                                  const Chunk *__restrict__ chunks,
-                                                  const int *__restrict__ idx,
-                                                  const int *__restrict__ opt,
-                                                  int *__restrict__ obuf)
-{
-    const Chunk ch = chunks[idx[blockIdx.x]];
-    AW_GLOBAL int *path = gp(D[ch.inst].path);
-    const AW_GLOBAL int *src = opt_path(obuf, ch, opt[blockIdx.x]);
-    for (int c = ch.c0 + (int)threadIdx.x; c < ch.c1; c += 256) path[c] = src[c];
 }
 
 //===========================================================================
@@ -1973,8 +775,8 @@ std::recursive_mutex &device_mutex()
 #define DEVICE_LOCK std::lock_guard<std::recursive_mutex> device_lock_(device_mutex())
 
 // The batch's streams: main carries every stage; side carries only the
-// traceback of the instances whose forward is final (their options,
-// re-runs and adoptions, driven by a helper host thread) while the forward
+// traceback of the instances whose forward is final (their chains and
+// re-runs, driven by a helper host thread) while the forward
 // re-runs of others continue on main.  The two are joined by the host
 // (stream synchronisation), never by a stream waiting on an event.
 struct Streams {
@@ -2069,20 +871,7 @@ int lanes_per_state_r(int Smax)
     return -1;
 }
 
-// LDS bytes / size of Real of the forward kernel for R states per lane
-int fw_lds_reals_r(bool fp32, int R)
-{
-    switch (R) {
-    case 1: return fp32 ? fw_lds_reals<float, 1>() : fw_lds_reals<double, 1>();
-    case 2: return fp32 ? fw_lds_reals<float, 2>() : fw_lds_reals<double, 2>();
-    case 4: return fp32 ? fw_lds_reals<float, 4>() : fw_lds_reals<double, 4>();
-    case 6: return fp32 ? fw_lds_reals<float, 6>() : fw_lds_reals<double, 6>();
-    case 8: return fp32 ? fw_lds_reals<float, 8>() : fw_lds_reals<double, 8>();
-    case 12: return fp32 ? fw_lds_reals<float, 12>() : fw_lds_reals<double, 12>();
-    case 16: return fp32 ? fw_lds_reals<float, 16>() : fw_lds_reals<double, 16>();
-    default: return fp32 ? fw_lds_reals<float, 32>() : fw_lds_reals<double, 32>();
-    }
-}
+}  // namespace
 
 // The dynamic-LDS limit of a kernel only ever rises, under one lock: a
 // batch on another host thread that set a larger limit for the same kernel
@@ -2099,30 +888,6 @@ int set_lds_limit(const void *kern, size_t sh)
     return 0;
 }
 
-template <class Real, bool BIG = false>
-int launch_fw(const DevInst *dD, const FwTile *tiles, int cnt, void *bnd, double *bnorm,
-              size_t sh, hipStream_t st, int T1max, double tol = 0.0, int *early = nullptr)
-{
-    auto kern = early ? ((T1max <= 19) ? k_fw_all<Real, 19, true, BIG> : k_fw_all<Real, MAXT - 1, true, BIG>)
-                      : ((T1max <= 19) ? k_fw_all<Real, 19, false, BIG> : k_fw_all<Real, MAXT - 1, false, BIG>);
-    if (set_lds_limit((const void *)kern, sh)) return 1;
-    hipLaunchKernelGGL(kern, dim3(cnt), dim3(64), sh, st, dD, tiles, (Real *)bnd, bnorm, tol, early);
-    HIP_OK(hipGetLastError());
-    return 0;
-}
-
-// launch of a traceback kernel with sh bytes of dynamic LDS
-template <class Kern, class... Args>
-int launch_lds(Kern kern, int grid, size_t sh, hipStream_t st, Args... args)
-{
-    if (set_lds_limit((const void *)kern, sh)) return 1;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), sh, st, args...);
-    HIP_OK(hipGetLastError());
-    return 0;
-}
-
-}  // namespace
-
 struct Batch::Impl {
     std::vector<HostInstance> hosts;
     std::vector<std::vector<double>> us, priors;
@@ -2133,7 +898,7 @@ struct Batch::Impl {
     std::vector<double> lnl;
     std::vector<int> nvar;
     std::vector<Chunk> chunks;
-    std::vector<int> tlist0, tlist1;   // host tile lists of the option launches
+    std::vector<int> tlist0, tlist1;   // host tile lists of the two launches
     DevBuf in, work, tab, aux, vbuf, tiles, fwb;
     Arena arena;   // base == nullptr: buffers come from hipMalloc
     std::vector<std::vector<float>> staged32;   // FP32 planes of host-prepared instances
@@ -2141,16 +906,15 @@ struct Batch::Impl {
     DevInst *dD = nullptr;
     long long *d_coloff = nullptr;
     int *d_blkoff = nullptr, *d_voff = nullptr, *d_nvar = nullptr, *d_list = nullptr;
-    // traceback options: start / end states [nch * K], alternative paths,
-    // re-run lists and results, adopted alternatives
-    int *d_ostart = nullptr, *d_oend = nullptr, *d_obuf = nullptr;
-    int *d_ridx = nullptr, *d_rk1 = nullptr, *d_rres = nullptr, *d_aidx = nullptr, *d_aopt = nullptr;
-    int *d_tlist = nullptr;   // [2 nch] tile lists of the two option launches
-    int tb_opts = 1;
+    // traceback tiles: start / end states of their chains, re-run lists and
+    // results
+    int *d_ostart = nullptr, *d_oend = nullptr;
+    int *d_ridx = nullptr, *d_rk1 = nullptr, *d_rres = nullptr;
+    int *d_tlist = nullptr;   // [2 nch] tile lists of the two launches
     // instances with 32 states per lane run in kernel symbols of their own;
     // the LDS bytes of those symbols' forward and traceback launches
     bool any_big = false;
-    size_t shf_big = 0, sht_big = 0;
+    size_t shf_big = 0, sht = 0, sht_big = 0;
     Chunk *d_chunks = nullptr;
     FwTile *d_fwt = nullptr, *d_fwre = nullptr;
     char *d_bnd = nullptr;
@@ -2350,52 +1114,34 @@ int Batch::upload()
     return 0;
 }
 
-// FP32 traceback column cost (us) by states per lane, measured on one
-// instance per R (20 time points) on MI355X.
-inline double tb_cost_model(int R)
-{
-    return R <= 1 ? 0.50 : R == 2 ? 0.52 : R == 4 ? 0.63 : R == 6 ? 0.75 : R == 8 ? 0.86 : R == 12 ? 1.05 : 1.25;
-}
-
-// Traceback tiles of every instance: about tile_cols columns (0: one per
-// instance; scaled by the column cost of the instance's R), tail_cols for
-// the instances with tail[inst] set, the instances with the most states per
-// lane first, K options per tile.  Copies the tile list to the device on the
-// main stream; returns the LDS size of the tile kernels (sht).
-static int plan_tiles(Batch::Impl &m, bool fp32, int tile_cols, int warm, int K, size_t &sht,
+// Traceback tiles of every instance: tile_cols columns (0: one per
+// instance), tail_cols for the instances with tail[inst] set, the instances
+// with the most states per lane first.  Copies the tile list to the device
+// on the main stream.
+static int plan_tiles(Batch::Impl &m, int tile_cols, int warm,
                       const std::vector<char> *tail = nullptr, int tail_cols = 0)
 {
     const int n = (int)m.h.size();
-    const size_t rsz = fp32 ? sizeof(float) : sizeof(double);
     std::vector<Chunk> &chs = m.chunks;
     chs.clear();
-    m.sht_big = 0;
     // The tail instances' tiles run when the rest of the device is idle:
-    // tail_cols long, or longer when that would give more option waves
-    // than the device has SIMDs (each wave a SIMD to itself), since a
-    // second round of waves costs more than longer tiles do
+    // tail_cols long, or longer when that would give more workgroups than
+    // the device has CUs
     if (tail && tail_cols > 0) {
         double cols = 0;
         for (int i = 0; i < n; i++)
-            if ((*tail)[i]) cols += (double)m.h[i].L * tb_cost_model(m.h[i].R) / tb_cost_model(12);
-        const double simds = 4.0 * std::max(1, ctx().prop.multiProcessorCount);
-        tail_cols = std::max(tail_cols, (int)std::ceil(cols * K / simds));
+            if ((*tail)[i]) cols += m.h[i].L;
+        const double cus = std::max(1, ctx().prop.multiProcessorCount);
+        tail_cols = std::max(tail_cols, (int)std::ceil(cols / cus));
     }
-    // tiles of the instances with the most states per lane (the slowest
-    // columns) are dispatched first
     std::vector<int> byr(n);
     std::iota(byr.begin(), byr.end(), 0);
     std::stable_sort(byr.begin(), byr.end(), [&](int a, int b) { return m.h[a].R > m.h[b].R; });
-    sht = 0;
-    long long ocols = 0;   // columns of the tiles that have alternatives
+    m.sht = m.sht_big = 0;
     for (int i : byr) {
         const DevInst &d = m.h[i];
-        // tile_cols columns at R = 12's column cost; instances with cheaper
-        // columns get proportionally longer tiles (fewer tiles, the same
-        // time per tile)
         const int tc = (tail && (*tail)[i] && tail_cols > 0) ? tail_cols : tile_cols;
-        const int tile =
-            tc > 0 ? std::max(64, (int)(tc * tb_cost_model(12) / tb_cost_model(d.R))) : d.L;
+        const int tile = tc > 0 ? std::max(64, tc) : d.L;
         const int nt = (d.L + tile - 1) / tile;
         for (int t = 0; t < nt; t++) {
             Chunk k;
@@ -2405,31 +1151,22 @@ static int plan_tiles(Batch::Impl &m, bool fp32, int tile_cols, int warm, int K,
             k.first = (t == 0);
             k.last = (t == nt - 1);
             k.cw = k.last ? d.L - 1 : std::min(d.L - 1, k.c1 + std::max(warm, 0));
-            k.coff = k.last ? 0 : (long long)(K - 1) * ocols;
-            if (!k.last) ocols += k.c1 - k.c0;
             chs.push_back(k);
         }
-        // (a,b) and (c,a,b) tables, then two row batches
-        const int T1 = d.T - 1;
-        const int bt = tb_batch_host(d.R, rsz);
-        size_t &sh = d.R > 16 ? m.sht_big : sht;
-        sh = std::max(sh, rsz * ((size_t)T1 * T1 + d.TC) + rsz * 2 * bt * 64 * (size_t)d.R);
+        size_t &sh = d.R > 16 ? m.sht_big : m.sht;
+        sh = std::max(sh, tb_lds_bytes(d.R));
     }
     const int nch = (int)chs.size();
-    m.tb_opts = K;
     for (int pass = 0; pass < 2; pass++) {
         Plan p;
         p.base = pass ? m.tiles.p : nullptr;
         m.d_chunks = p.take<Chunk>(nch);
-        m.d_ostart = p.take<int>((size_t)nch * K);
-        m.d_oend = p.take<int>((size_t)nch * K);
+        m.d_ostart = p.take<int>(nch);
+        m.d_oend = p.take<int>(nch);
         m.d_ridx = p.take<int>(2 * (size_t)nch);
         m.d_rk1 = p.take<int>(2 * (size_t)nch);
-        m.d_rres = p.take<int>(6 * (size_t)nch);
-        m.d_aidx = p.take<int>(2 * (size_t)nch);
-        m.d_aopt = p.take<int>(2 * (size_t)nch);
+        m.d_rres = p.take<int>(4 * (size_t)nch);
         m.d_tlist = p.take<int>(2 * (size_t)nch);
-        m.d_obuf = p.take<int>((size_t)std::max(1LL, (long long)(K - 1) * ocols));
         if (pass == 0 && m.tiles.ensure(p.used + 4096)) return 1;
     }
     HIP_OK(hipMemcpyAsync(m.d_chunks, chs.data(), sizeof(Chunk) * nch, hipMemcpyHostToDevice,
@@ -2437,81 +1174,50 @@ static int plan_tiles(Batch::Impl &m, bool fp32, int tile_cols, int warm, int K,
     return 0;
 }
 
-// The speculative launch on stream s: every option of the tiles of the
-// instances with take[inst] set (all when take is null); slot 0 or 1 of the
-// device tile lists.
-static int launch_options(Batch::Impl &m, bool fp32, size_t sht, const std::vector<char> *take,
-                          int slot, hipStream_t s)
+// The chains of the tiles of the instances with take[inst] set (all when
+// take is null) on stream s; slot 0 or 1 of the device tile lists.
+static int launch_chains(Batch::Impl &m, bool fp32, const std::vector<char> *take, int slot,
+                         hipStream_t s)
 {
-    const int nch = (int)m.chunks.size(), K = m.tb_opts;
+    const int nch = (int)m.chunks.size();
     std::vector<int> &list = slot ? m.tlist1 : m.tlist0;
     list.clear();
     // the tiles of the 32-states-per-lane instances after the others (a
     // launch of their own symbol)
-    for (int big = 0; big < 2; big++)
+    int nn = 0;
+    for (int big = 0; big < 2; big++) {
         for (int j = 0; j < nch; j++)
             if ((!take || (*take)[m.chunks[j].inst]) && (m.h[m.chunks[j].inst].R > 16) == (big == 1))
                 list.push_back(j);
+        if (!big) nn = (int)list.size();
+    }
     const int nl = (int)list.size();
     if (!nl) return 0;
-    int nn = 0;
-    while (nn < nl && m.h[m.chunks[list[nn]].inst].R <= 16) nn++;
     int *dl = m.d_tlist + (size_t)slot * nch;
     HIP_OK(hipMemcpyAsync(dl, list.data(), sizeof(int) * nl, hipMemcpyHostToDevice, s));
-    if (nn > 0) {
-        const int grid = (nn + 7) / 8 * 8 * K;
-        if (fp32 ? launch_lds(k_tb_spec<float, false>, grid, sht, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)dl, nn, K, m.d_obuf,
-                              m.d_ostart, m.d_oend)
-                 : launch_lds(k_tb_spec<double, false>, grid, sht, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)dl, nn, K, m.d_obuf,
-                              m.d_ostart, m.d_oend))
-            return 1;
-    }
-    if (nl > nn) {
-        const int nb = nl - nn, grid = (nb + 7) / 8 * 8 * K;
-        if (fp32 ? launch_lds(k_tb_spec<float, true>, grid, m.sht_big, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)(dl + nn), nb, K, m.d_obuf,
-                              m.d_ostart, m.d_oend)
-                 : launch_lds(k_tb_spec<double, true>, grid, m.sht_big, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)(dl + nn), nb, K, m.d_obuf,
-                              m.d_ostart, m.d_oend))
-            return 1;
-    }
-    return 0;
+    if (nn > 0 && launch_tb_spec(fp32, false, m.dD, m.d_chunks, dl, nn, m.sht, m.d_ostart, m.d_oend, s))
+        return 1;
+    return nl > nn && launch_tb_spec(fp32, true, m.dD, m.d_chunks, dl + nn, nl - nn, m.sht_big,
+                                     m.d_ostart, m.d_oend, s);
 }
 
 // Resolution of the tiles, right to left within each instance.  A tile
-// whose true state at c1 is the start of one of its options takes that
-// option's path (option 0 is in place; an alternative is copied in at the
-// end) and passes that option's end state on as the true state of the
-// tile before.  The first tile that no option fits is re-run from its true
-// state, and in the same pass every tile before it whose predicted start
-// (the end of the next tile's option 0, or of the option its own
-// prediction fits) fits none of its options is re-run from that
-// prediction.  A re-run replaces option 0 by the chain from its start (the
-// samples until it coalesces with a stored option, then that option), so a
-// right prediction leaves the tile decided for the next pass.
+// whose true state at c1 is the start of its chain keeps that chain's path
+// and passes the chain's end state on as the true state of the tile before.
+// The first tile that does not fit is re-run from its true state, and in the
+// same pass every tile before it whose predicted start (the end of the next
+// tile's chain) is not its own is re-run from that prediction.  A re-run
+// replaces the tile's chain by the one from its start (the samples until it
+// meets the stored path, then that path), so a right prediction leaves the
+// tile decided for the next pass.
 // take: the instances to resolve (all when null); slot 0 or 1 of the
 // device lists, so that two resolutions of disjoint instances can run at
 // once on two streams.
-static int resolve_tiles(Batch::Impl &m, bool fp32, size_t sht, RunStats &rs, hipStream_t s,
+static int resolve_tiles(Batch::Impl &m, bool fp32, RunStats &rs, hipStream_t s,
                          const std::vector<char> *take, int slot)
 {
     const std::vector<Chunk> &chs = m.chunks;
-    const int nch = (int)chs.size(), K = m.tb_opts;
-    int *ridx = m.d_ridx + (size_t)slot * nch, *rk1 = m.d_rk1 + (size_t)slot * nch;
-    int *rres = m.d_rres + (size_t)slot * 3 * nch;
-    int *aidx = m.d_aidx + (size_t)slot * nch, *aopt = m.d_aopt + (size_t)slot * nch;
-    std::vector<int> os((size_t)nch * K), oe((size_t)nch * K);
-    HIP_OK(hipMemcpyAsync(os.data(), m.d_ostart, sizeof(int) * os.size(), hipMemcpyDeviceToHost, s));
-    HIP_OK(hipMemcpyAsync(oe.data(), m.d_oend, sizeof(int) * oe.size(), hipMemcpyDeviceToHost, s));
-    HIP_OK(hipStreamSynchronize(s));
-    auto match = [&](int j, int b) {
-        for (int o = 0; o < K; o++)
-            if (os[(size_t)j * K + o] == b) return o;
-        return -1;
-    };
+    const int nch = (int)chs.size();
     // per instance: its first tile, the rightmost undecided tile and the
     // true state at that tile's column c1
     struct Walk {
@@ -2522,96 +1228,67 @@ static int resolve_tiles(Batch::Impl &m, bool fp32, size_t sht, RunStats &rs, hi
         if (chs[j].last && !chs[j].first && (!take || (*take)[chs[j].inst])) {
             int f = j;
             while (!chs[f].first) f--;
-            ws.push_back(Walk{f, j - 1, oe[(size_t)j * K]});
+            ws.push_back(Walk{f, j - 1, 0});
         }
-    std::vector<int> aj, ao, pj, pk, res;
+    if (ws.empty()) return 0;
+    int *ridx = m.d_ridx + (size_t)slot * nch, *rk1 = m.d_rk1 + (size_t)slot * nch;
+    int *rres = m.d_rres + (size_t)slot * 2 * nch;
+    std::vector<int> os(nch), oe(nch);
+    HIP_OK(hipMemcpyAsync(os.data(), m.d_ostart, sizeof(int) * nch, hipMemcpyDeviceToHost, s));
+    HIP_OK(hipMemcpyAsync(oe.data(), m.d_oend, sizeof(int) * nch, hipMemcpyDeviceToHost, s));
+    HIP_OK(hipStreamSynchronize(s));
+    for (Walk &w : ws) w.b = oe[w.r + 1];
+    std::vector<int> pj, pk, res;
     while (true) {
         pj.clear();
         pk.clear();
         for (Walk &w : ws) {
-            while (w.r >= w.f) {
-                const int o = match(w.r, w.b);
-                if (o < 0) break;
-                if (o > 0) {
-                    aj.push_back(w.r);
-                    ao.push_back(o);
-                }
-                w.b = oe[(size_t)w.r * K + o];
-                w.r--;
-            }
+            while (w.r >= w.f && os[w.r] == w.b) w.b = oe[w.r--];
             if (w.r < w.f) continue;
-            pj.push_back(w.r);
-            pk.push_back(w.b);
-            int g = oe[(size_t)w.r * K];
-            for (int j = w.r - 1; j >= w.f; j--) {
-                const int o = match(j, g);
-                if (o >= 0) {
-                    g = oe[(size_t)j * K + o];
-                    continue;
+            int g = w.b;
+            for (int j = w.r; j >= w.f; j--) {
+                if (os[j] != g) {
+                    pj.push_back(j);
+                    pk.push_back(g);
                 }
-                pj.push_back(j);
-                pk.push_back(g);
-                g = oe[(size_t)j * K];
+                g = oe[j];
             }
         }
         if (pj.empty()) break;
         const int np = (int)pj.size();
         HIP_OK(hipMemcpyAsync(ridx, pj.data(), sizeof(int) * np, hipMemcpyHostToDevice, s));
         HIP_OK(hipMemcpyAsync(rk1, pk.data(), sizeof(int) * np, hipMemcpyHostToDevice, s));
-        if (fp32 ? launch_lds(k_tb_rerun<float, false>, np, sht, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)ridx,
-                              (const int *)rk1, K, m.d_obuf, (const int *)m.d_ostart, rres)
-                 : launch_lds(k_tb_rerun<double, false>, np, sht, s, (const DevInst *)m.dD,
-                              (const Chunk *)m.d_chunks, (const int *)ridx,
-                              (const int *)rk1, K, m.d_obuf, (const int *)m.d_ostart, rres))
+        if (m.sht && launch_tb_rerun(fp32, false, m.dD, m.d_chunks, ridx, rk1, np, m.sht, rres, s))
             return 1;
-        if (m.any_big &&
-            (fp32 ? launch_lds(k_tb_rerun<float, true>, np, m.sht_big, s, (const DevInst *)m.dD,
-                               (const Chunk *)m.d_chunks, (const int *)ridx,
-                               (const int *)rk1, K, m.d_obuf, (const int *)m.d_ostart, rres)
-                  : launch_lds(k_tb_rerun<double, true>, np, m.sht_big, s, (const DevInst *)m.dD,
-                               (const Chunk *)m.d_chunks, (const int *)ridx,
-                               (const int *)rk1, K, m.d_obuf, (const int *)m.d_ostart, rres)))
+        if (m.sht_big &&
+            launch_tb_rerun(fp32, true, m.dD, m.d_chunks, ridx, rk1, np, m.sht_big, rres, s))
             return 1;
-        res.resize(3 * (size_t)np);
+        res.resize(2 * (size_t)np);
         HIP_OK(hipMemcpyAsync(res.data(), rres, sizeof(int) * res.size(), hipMemcpyDeviceToHost, s));
         HIP_OK(hipStreamSynchronize(s));
         rs.tb_passes++;
         for (int x = 0; x < np; x++) {
             const int j = pj[x];
-            rs.tb_rerun_cols += chs[j].c1 - (res[3 * x] < 0 ? chs[j].c0 : res[3 * x]);
-            os[(size_t)j * K] = pk[x];
-            oe[(size_t)j * K] = res[3 * x + 2];
+            rs.tb_rerun_cols += chs[j].c1 - (res[2 * x] < 0 ? chs[j].c0 : res[2 * x]);
+            os[j] = pk[x];
+            oe[j] = res[2 * x + 1];
         }
     }
-    if (!aj.empty()) {
-        const int na = (int)aj.size();
-        HIP_OK(hipMemcpyAsync(aidx, aj.data(), sizeof(int) * na, hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(aopt, ao.data(), sizeof(int) * na, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(k_tb_adopt, dim3(na), dim3(256), 0, s, (const DevInst *)m.dD,
-                           (const Chunk *)m.d_chunks, (const int *)aidx, (const int *)aopt,
-                           m.d_obuf);
-        HIP_OK(hipGetLastError());
-    }
-    rs.tb_adopted = (int)aj.size();
     return 0;
 }
 
 // The traceback of every instance whose forward table is resident: the
-// options of every tile in one launch, then the resolution (re-runs where
-// no option fits).  resolve = false leaves the speculative option-0 paths
+// chains of every tile in one launch, then the resolution (re-runs of the
+// tiles that do not fit).  opt.fixup = false leaves the speculative paths
 // (diagnostics).
 static int traceback_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt, RunStats &rs)
 {
-    size_t sht;
-    const int K = std::max(1, std::min(opt.tile_opts, TB_KMAX));
-    if (plan_tiles(m, fp32, opt.tile_cols, opt.tile_warm, K, sht)) return 1;
-    if (launch_options(m, fp32, sht, nullptr, 0, m.st.main)) return 1;
-    return opt.fixup ? resolve_tiles(m, fp32, sht, rs, m.st.main, nullptr, 0) : 0;
+    if (plan_tiles(m, opt.tile_cols, opt.tile_warm)) return 1;
+    if (launch_chains(m, fp32, nullptr, 0, m.st.main)) return 1;
+    return opt.fixup ? resolve_tiles(m, fp32, rs, m.st.main, nullptr, 0) : 0;
 }
 
-int Batch::tune_tiles(Precision prec, const int *cand, int ncand, double *ms_out, int warm,
-                      int opts)
+int Batch::tune_tiles(Precision prec, const int *cand, int ncand, double *ms_out, int warm)
 {
     BATCH_LOCK;
     BatchOptions opt;
@@ -2630,7 +1307,6 @@ int Batch::tune_tiles(Precision prec, const int *cand, int ncand, double *ms_out
         topt.prec = prec;
         topt.tile_cols = cand[i];
         topt.tile_warm = warm;
-        topt.tile_opts = opts;
         if (traceback_stage(m, fp32, topt, rs)) return -1;
         (void)hipEventRecord(c.ev[7], c.main);
         HIP_OK(hipStreamSynchronize(c.main));
@@ -2768,8 +1444,8 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
             return 1;
     }
     (void)hipEventRecord(c.ev[6], s);
-    if (fp32 ? launch_fw<float>(m.dD, m.d_fwt, nt, m.d_bnd, m.d_bnorm, shf, s, t1max)
-             : launch_fw<double>(m.dD, m.d_fwt, nt, m.d_bnd, m.d_bnorm, shf, s, t1max))
+    if (fp32 ? launch_fw<float, false>(m.dD, m.d_fwt, nt, m.d_bnd, m.d_bnorm, shf, s, t1max)
+             : launch_fw<double, false>(m.dD, m.d_fwt, nt, m.d_bnd, m.d_bnorm, shf, s, t1max))
         return 1;
     (void)hipEventRecord(c.ev[7], s);
     if (m.any_big) HIP_OK(hipStreamSynchronize(c.side));
@@ -2782,13 +1458,8 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
     while (!chk.empty()) {
         const int nc = (int)chk.size();
         HIP_OK(hipMemcpyAsync(m.d_fidx, chk.data(), sizeof(int) * nc, hipMemcpyHostToDevice, s));
-        if (fp32)
-            hipLaunchKernelGGL(k_fw_check<float>, dim3(nc), dim3(64), 0, s, m.dD, m.d_fwt, m.d_fidx,
-                               (const float *)m.d_bnd, m.d_bnorm, opt.fw_tol, m.d_fflag);
-        else
-            hipLaunchKernelGGL(k_fw_check<double>, dim3(nc), dim3(64), 0, s, m.dD, m.d_fwt, m.d_fidx,
-                               (const double *)m.d_bnd, m.d_bnorm, opt.fw_tol, m.d_fflag);
-        HIP_OK(hipGetLastError());
+        if (launch_fw_check(m.dD, m.d_fwt, m.d_fidx, nc, m.d_bnd, m.d_bnorm, opt.fw_tol, m.d_fflag, s))
+            return 1;
         flags.resize(nc);
         HIP_OK(hipMemcpyAsync(flags.data(), m.d_fflag, sizeof(int) * nc, hipMemcpyDeviceToHost, s));
         HIP_OK(hipStreamSynchronize(s));
@@ -2822,16 +1493,11 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
         const int nr = (int)sub.size();
         HIP_OK(hipMemcpyAsync(m.d_fwt, tl.data(), sizeof(FwTile) * nt, hipMemcpyHostToDevice, s));
         HIP_OK(hipMemcpyAsync(m.d_fwre, sub.data(), sizeof(FwTile) * nr, hipMemcpyHostToDevice, s));
-        if (fp32 ? launch_fw<float>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, shf, s, t1max,
-                                    opt.fw_tol, m.d_fflag)
-                 : launch_fw<double>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, shf, s, t1max,
-                                     opt.fw_tol, m.d_fflag))
+        if (launch_fw<float, false>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, shf, s, t1max,
+                                    opt.fw_tol, m.d_fflag))
             return 1;
-        if (m.any_big &&
-            (fp32 ? launch_fw<float, true>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, m.shf_big, s,
-                                           t1max, opt.fw_tol, m.d_fflag)
-                  : launch_fw<double, true>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, m.shf_big, s,
-                                            t1max, opt.fw_tol, m.d_fflag)))
+        if (m.any_big && launch_fw<float, true>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, m.shf_big,
+                                                s, t1max, opt.fw_tol, m.d_fflag))
             return 1;
         // a tile that rejoined its stored columns kept its boundary column;
         // the tile after one that ran to its end is checked again
@@ -2897,6 +1563,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
             d.lcoef = fp32 ? nullptr : p.take<double>((size_t)B * NCOEF * RW);
             d.lcoef32 = fp32 ? p.take<float>((size_t)B * NCOEF * RW) : nullptr;
             d.ldet = p.take<int>((size_t)B * RW);
+            d.pred = p.take<unsigned short>((size_t)B * RW);
             d.lprior = p.take<double>(RW);
             d.norms = p.take<double>(L);
             d.path = p.take<int>(L);
@@ -3009,6 +1676,9 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
                            m.d_voff, n, nmax);
     }
     HIP_OK(hipGetLastError());
+    int rmax = 1;
+    for (int i = 0; i < n; i++) rmax = std::max(rmax, m.h[i].R);
+    if (launch_tb_pred(m.dD, m.d_blkoff, n, blkoff[n], rmax, s)) return 1;
     (void)hipEventRecord(c.ev[3], s);
 
     // forward: one wave per tile, all tiles in one launch, the longest
@@ -3028,34 +1698,32 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         const DevInst &d = m.h[i];
         t1max = std::max(t1max, d.T - 1);
         size_t &sh = d.R > 16 ? m.shf_big : shf;
-        sh = std::max(sh, rsz * (size_t)fw_lds_reals_r(fp32, d.R));
+        sh = std::max(sh, fw_lds_bytes(fp32, d.R));
         m.any_big |= d.R > 16;
     }
     RunStats rs;
     // Once the first check of the forward tiles has shown which instances
-    // are re-run, the traceback options of all the others go to the side
+    // are re-run, the traceback chains of all the others go to the side
     // stream and run while the re-runs continue on the main stream.
     // A helper host thread then resolves those instances' tiles on the side
     // stream (its re-runs too), while this thread drives the forward re-runs
     // and then the re-run instances' traceback on the main stream.
-    size_t sht = 0;
     std::vector<char> busy, done;
-    const int K = std::max(1, std::min(opt.tile_opts, TB_KMAX));
     std::thread helper;
     RunStats rs_side;
     int rc_side = 0;
     auto early_tb = [&](const std::vector<char> &b) -> int {
         if (!opt.traceback || std::find(b.begin(), b.end(), 1) == b.end()) return 0;
         busy = b;
-        if (plan_tiles(m, fp32, opt.tile_cols, opt.tile_warm, K, sht, &b, opt.tail_tile_cols))
+        if (plan_tiles(m, opt.tile_cols, opt.tile_warm, &b, opt.tail_tile_cols))
             return 1;
         HIP_OK(hipStreamSynchronize(s));   // the tile list is on the device
         done.assign(n, 0);
         for (int i = 0; i < n; i++) done[i] = !b[i];
-        if (launch_options(m, fp32, sht, &done, 0, c.side)) return 1;
+        if (launch_chains(m, fp32, &done, 0, c.side)) return 1;
         if (opt.fixup)
             helper = std::thread([&] {
-                rc_side = resolve_tiles(m, fp32, sht, rs_side, c.side, &done, 1);
+                rc_side = resolve_tiles(m, fp32, rs_side, c.side, &done, 1);
                 (void)hipEventRecord(c.ev[8], c.side);
             });
         return 0;
@@ -3072,20 +1740,19 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     (void)hipEventRecord(c.ev[4], s);
     hipLaunchKernelGGL(k_lnl_b, dim3(n), dim3(256), 0, s, m.dD, m.d_list);
     HIP_OK(hipGetLastError());
-    // traceback tiles: the options of every tile, then their resolution
+    // traceback tiles: the chains of every tile, then their resolution
     if (opt.traceback) {
         if (busy.empty()) {
             if (traceback_stage(m, fp32, opt, rs)) return 1;
         } else {
-            if (launch_options(m, fp32, sht, &busy, 1, s)) return 1;
-            if (opt.fixup && resolve_tiles(m, fp32, sht, rs, s, &busy, 0)) return 1;
+            if (launch_chains(m, fp32, &busy, 1, s)) return 1;
+            if (opt.fixup && resolve_tiles(m, fp32, rs, s, &busy, 0)) return 1;
             (void)hipEventRecord(c.ev[9], s);
             if (helper.joinable()) helper.join();
             HIP_OK(hipStreamSynchronize(c.side));
             if (rc_side) return 1;
             rs.tb_passes = std::max(rs.tb_passes, rs_side.tb_passes);
             rs.tb_rerun_cols += rs_side.tb_rerun_cols;
-            rs.tb_adopted += rs_side.tb_adopted;
         }
     }
     (void)hipEventRecord(c.ev[5], s);
@@ -3357,3 +2024,4 @@ int run_instance_noalloc(const HostInstance &hi, const double *u, int *path, dou
 }
 
 }  // namespace aw
+

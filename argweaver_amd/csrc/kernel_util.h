@@ -1,0 +1,150 @@
+// kernel_util.h -- device helpers shared by the kernels (address spaces,
+// cross-lane moves, coefficient planes) and the launch helpers.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+
+#include "engine.h"
+
+namespace aw {
+
+#define HIP_OK(x)                                                                       \
+    do {                                                                                \
+        hipError_t e_ = (x);                                                            \
+        if (e_ != hipSuccess) {                                                         \
+            fprintf(stderr, "argweaver_amd: HIP error %s at %s:%d\n", hipGetErrorString(e_), \
+                    __FILE__, __LINE__);                                                \
+            return 1;                                                                   \
+        }                                                                               \
+    } while (0)
+
+// Pointers read out of DevInst are generic; accesses through them compile to
+// flat instructions, which count against the LDS wait counter too, so every
+// LDS wait would also drain outstanding HBM stores.  gp() restores the
+// global address space so loads and stores become global_* instructions.
+#define AW_GLOBAL __attribute__((address_space(1)))
+template <class X>
+__device__ inline AW_GLOBAL X *gp(X *p)
+{
+    return (AW_GLOBAL X *)p;
+}
+
+// Read-only data indexed by wave-uniform values (block bounds, uniforms)
+// goes through the constant address space so it is fetched with scalar loads.
+#define AW_CONST __attribute__((address_space(4)))
+template <class X>
+__device__ inline AW_CONST const X *cp(const X *p)
+{
+    return (AW_CONST const X *)p;
+}
+
+// LDS operations of one wave are performed in order, so inside a
+// single-wave workgroup only the compiler's order matters; every LDS access
+// of a kernel goes through one dynamic shared array, so accesses that may
+// overlap are never reordered.  This marks the places that rely on it.
+__device__ inline void lds_order() {}
+
+// index i such that off[i] <= x < off[i+1]
+template <class PT, class X>
+__device__ inline int find_owner(PT off, int n, X x)
+{
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        int mid = (lo + hi + 1) >> 1;
+        if (off[mid] <= x) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+//===========================================================================
+// cross-lane moves (DPP).  A lane whose source is outside the wave (wave
+// shifts) or outside its 16-lane row (row shifts) receives 0.
+
+constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114,
+              DPP_ROW_SHR8 = 0x118, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138,
+              DPP_QUAD_SWAP1 = 0xB1;   // quad_perm [1,0,3,2]: lanes 2k and 2k+1 swap
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_i(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_r(float x)
+{
+    return __int_as_float(dpp_i<CTRL>(__float_as_int(x)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_r(double x)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = (unsigned)dpp_i<CTRL>((int)v);
+    const unsigned hi = (unsigned)dpp_i<CTRL>((int)(v >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+__device__ __forceinline__ double readlane_d(double x, int l)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, l);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// inclusive prefix sum over the 64 lanes: Hillis-Steele inside each 16-lane
+// row, then the totals of the rows before
+__device__ __forceinline__ double wave_incl_scan(double v)
+{
+    v += dpp_r<DPP_ROW_SHR1>(v);
+    v += dpp_r<DPP_ROW_SHR2>(v);
+    v += dpp_r<DPP_ROW_SHR4>(v);
+    v += dpp_r<DPP_ROW_SHR8>(v);
+    const double t0 = readlane_d(v, 15), t1 = readlane_d(v, 31), t2 = readlane_d(v, 47);
+    const int row = threadIdx.x >> 4;
+    double off = 0.0;
+    if (row >= 1) off = t0;
+    if (row >= 2) off += t1;
+    if (row >= 3) off += t2;
+    return v + off;
+}
+
+
+template <class Real>
+__device__ __forceinline__ const AW_GLOBAL Real *planes(const DevInst &d, int b, int RW)
+{
+    if (sizeof(Real) == 4)
+        return (const AW_GLOBAL Real *)(gp(d.lcoef32) + (size_t)b * NCOEF * RW);
+    return (const AW_GLOBAL Real *)(gp(d.lcoef) + (size_t)b * NCOEF * RW);
+}
+
+__device__ __forceinline__ float readlane_r(float x, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+__device__ __forceinline__ double readlane_r(double x, int l)
+{
+    return readlane_d(x, l);
+}
+
+// x of the lane addr / 4 (ds_bpermute)
+__device__ __forceinline__ float bperm_r(float x, int addr)
+{
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
+}
+__device__ __forceinline__ double bperm_r(double x, int addr)
+{
+    const long long v = __double_as_longlong(x);
+    const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)v);
+    const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(addr, (int)(v >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Raises a kernel's dynamic-LDS limit to sh bytes (engine.hip): it only ever
+// rises, under one lock, so a batch on another host thread that set a larger
+// limit for the same kernel is never undercut between its call and its launch.
+int set_lds_limit(const void *kern, size_t sh);
+
+}  // namespace aw

@@ -1,0 +1,618 @@
+// traceback.hip -- stochastic traceback (stochastic_traceback,
+// sample_thread.cpp:522-569; sample_hmm_posterior_step :506-519; sample,
+// common.h:272-290).
+//
+// The sample of a column depends on the state sampled at the column to its
+// right, so one wave walking the columns pays the latency of a column's scan
+// and sampling for every one of them.  But the state hardly ever changes
+// inside a local-tree block (0.03-0.2 % of the columns), and across a switch
+// it follows the likeliest source state in 94-99.8 % of the cases.  So a
+// workgroup walks one tile, its waves working on consecutive runs of columns
+// (units, about a block each) at once: the entry state of every unit is
+// predicted by chasing the blocks' source tables from the true state, each
+// wave samples its unit from the predicted entry state, and the units up to
+// the first one whose outcome was not what the next one assumed are kept.
+// Every stored sample is the sample of its column given its right neighbour,
+// whatever was predicted, so the thread is that of a column-by-column walk.
+//
+// Inside a unit a wave tests columns for "the state stays" sixteen at a time:
+// the weights of the column's states under a fixed next state are summed in
+// FP32 below, at and in total, and the column stays when its pick lies inside
+// the state's share by more than 2^-13 of the total, sixty times the bound on
+// the FP32 sums' error.  Any other column is sampled with the FP64 cumulative
+// sums.
+//
+// Bound by the rows' latency: one CU streams them at about 33 GB/s, which is
+// 0.03 / 0.06 / 0.12 us per column at 4 / 8 FP32 and 8 FP64 states per lane,
+// against 0.6 / 0.9 / 1.0 us of a wave sampling column by column.  Measured
+// with it on MI355X: 10000 columns of 96 states, FP64, 5.1 -> 0.48 ms; 500k
+// columns of 700 states, FP32, 4096-column tiles, 76 -> 15 ms; 256 instances
+// (14.9M columns, FP32) 49.6 -> 8.6 ms after the forward.
+#include "traceback.h"
+
+#include "kernel_util.h"
+
+namespace aw {
+
+namespace {
+
+// waves of a tile's workgroup.  BIG: 32 states per lane, whose rows need the
+// registers of twice the waves
+template <bool BIG>
+constexpr int tb_waves()
+{
+    return BIG ? 8 : 16;
+}
+
+// columns tested per unit, at most 63: one lane each, and one for the switch
+// after them.  Blocks average 25-55 columns; 63 and 32 are 1-3 % slower (the
+// longest unit of a window sets its time; short ones pay more entries).
+constexpr int TB_SEG = 48;
+constexpr unsigned TB_NONE = 0xffff;   // no predicted source
+
+// LDS: per-unit results, then the units' source tables
+constexpr int TB_RES = 6;
+enum : int { RES_OUT = 0, RES_HYP, RES_FLAG, RES_NEXT, RES_BLK, RES_MATCH };
+enum : int { UNIT_LIVE = 1, UNIT_FINAL = 2 };
+
+__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+
+// inclusive prefix sum over the 64 lanes: Hillis-Steele inside each 16-lane
+// row, then the totals of the rows before
+__device__ __forceinline__ double incl_scan(double v)
+{
+    v += dpp_r<DPP_ROW_SHR1>(v);
+    v += dpp_r<DPP_ROW_SHR2>(v);
+    v += dpp_r<DPP_ROW_SHR4>(v);
+    v += dpp_r<DPP_ROW_SHR8>(v);
+    const double t0 = readlane_d(v, 15), t1 = readlane_d(v, 31), t2 = readlane_d(v, 47);
+    const int row = lane_id() >> 4;
+    double off = 0.0;
+    if (row >= 1) off = t0;
+    if (row >= 2) off += t1;
+    if (row >= 3) off += t2;
+    return v + off;
+}
+
+// First index k of the lane-run weights (lane l holds states l*R..l*R+R-1)
+// whose cumulative sum reaches u * total; S-1 if none does.  The products
+// are in the table's precision, the cumulative sums FP64.  Branch-free: the
+// owner lane counts the prefixes below the pick.
+template <class Real, int R>
+__device__ __forceinline__ int sample_state(const Real (&rv)[R], const Real (&tr)[R], int S, double u)
+{
+    const int lane = lane_id();
+    double pre[R];
+    double acc = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        acc += (double)(rv[r] * tr[r]);
+        pre[r] = acc;
+    }
+    const double inc = incl_scan(acc);
+    const double excl = dpp_r<DPP_WAVE_SHR1>(inc);
+    const double pick = u * readlane_d(inc, 63);
+    const unsigned long long m = __ballot(lane * R < S && excl + acc >= pick);
+    const int owner = m ? (int)__ffsll((long long)m) - 1 : (S - 1) / R;
+    const int nloc = min(R, S - lane * R);
+    const double thr = pick - excl;
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) cnt += (pre[r] < thr) ? 1 : 0;
+    const int rsel = m ? min(cnt, nloc - 1) : nloc - 1;
+    return __builtin_amdgcn_readlane(lane * R + rsel, owner);
+}
+
+template <class Real, int R>
+__device__ __forceinline__ void row_load(const AW_GLOBAL Real *alpha, int col, Real (&rv)[R])
+{
+    const AW_GLOBAL Real *row = alpha + (size_t)col * (64 * R);
+#pragma unroll
+    for (int r = 0; r < R; r++) rv[r] = row[r * 64 + lane_id()];
+}
+
+// state sampled from column col alone (the last column, or the speculative
+// start of a tile); every wave of the workgroup computes it
+template <class Real, int R>
+__device__ __forceinline__ int sample_alone(const DevInst &d, int col, int b, double u)
+{
+    Real rv[R], one[R];
+    row_load<Real, R>((const AW_GLOBAL Real *)d.alpha, col, rv);
+#pragma unroll
+    for (int r = 0; r < R; r++) one[r] = Real(1);   // padding slots hold 0
+    return sample_state<Real, R>(rv, one, cp(d.soff)[b + 1] - cp(d.soff)[b], u);
+}
+
+// The transition into state k within block b, as one register: lane a < 32
+// holds P(a -> time of k) from another branch, lane 32 + a from k's own.
+// (lk, rk) are k's lane and slot, node its branch.
+template <class Real>
+struct Target {
+    int k, lk, rk, node, time;
+    Real tab;
+};
+
+template <class Real, int R>
+__device__ __forceinline__ Target<Real> tb_target(const DevInst &d, int b, int k)
+{
+    const int lane = lane_id(), T1 = d.T - 1, TT = T1 * T1;
+    Target<Real> t;
+    t.k = k;
+    t.lk = k / R;
+    t.rk = k % R;
+    const int info = cp(d.linfo)[(size_t)b * (64 * R) + lane_pos(k, R)];
+    t.node = info_node(info);
+    t.time = info & INFO_TIME;
+    const int c = info_age(info), a = min(lane & 31, T1 - 1);
+    const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * TT;
+    const AW_GLOBAL double *tm2 = gp(d.tm2s) + (size_t)b * d.TC;
+    const int x = tc_base(c, T1) + (max(a, c) - c) * (T1 - c) + t.time - c;
+    const AW_GLOBAL double *src = lane < 32 ? tm + a * T1 + t.time : tm2 + x;
+    t.tab = (Real)*src;
+    return t;
+}
+
+// per-slot weights P(state -> k); padding slots carry time bin 31 and meet
+// zeros of the table: their index is clamped into it
+template <class Real, int R>
+__device__ __forceinline__ void tb_weights(const DevInst &d, const int (&ti)[R],
+                                           const Target<Real> &t, Real (&tr)[R])
+{
+    const int T1 = d.T - 1;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int a = min(ti[r] & INFO_TIME, T1 - 1);
+        tr[r] = bperm_r(t.tab, 4 * (a + (info_node(ti[r]) == t.node ? 32 : 0)));
+    }
+}
+
+// x of lanes [x.lo | y.lo] and [x.hi | y.hi], added: the lower half of the
+// wave keeps x, the upper half y
+__device__ __forceinline__ float fold32(float x, float y)
+{
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+// the same over the odd and even 16-lane rows
+__device__ __forceinline__ float fold16(float x, float y)
+{
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+// the same inside a row: lanes without bit keep x, the others y; CTRL pairs
+// lanes that differ in that bit
+template <int CTRL>
+__device__ __forceinline__ float fold_row(float x, float y, bool bit)
+{
+    return (bit ? y : x) + dpp_r<CTRL>(bit ? x : y);
+}
+constexpr int DPP_ROW_ROR8 = 0x128, DPP_ROW_HALF_MIRROR = 0x141, DPP_QUAD_SWAP2 = 0x4E;
+
+// Sums of 32 values over the 64 lanes at once, lane l receiving the sum of
+// value l >> 1: each fold halves the values, 70 instructions instead of the
+// 32 * 12 of separate butterflies.  v[i] holds values i and i + 16 already
+// folded by fold32.
+__device__ __forceinline__ float sum32(float (&v)[16])
+{
+    const int lane = lane_id();
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = fold16(v[i], v[i + 8]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = fold_row<DPP_ROW_ROR8>(v[i], v[i + 4], lane & 8);
+#pragma unroll
+    for (int i = 0; i < 2; i++) v[i] = fold_row<DPP_ROW_HALF_MIRROR>(v[i], v[i + 2], lane & 4);
+    v[0] = fold_row<DPP_QUAD_SWAP2>(v[0], v[1], lane & 2);
+    return v[0] + dpp_r<DPP_QUAD_SWAP1>(v[0]);
+}
+
+// One unit: the state of column ce is k; sample the n columns ce-1 .. ce-n
+// of block b, and with sw the column ce-n-1 of block b-1.  uw: lane j holds
+// the uniform of column ce-1-j.  pv receives the sampled states, lane j that
+// of column ce-1-j; returns the last one.
+template <class Real, int R>
+__device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, bool sw, int k,
+                                       double uw, int &pv)
+{
+    constexpr int RW = 64 * R;
+    // columns whose rows are in flight at once, within about 64 registers
+    constexpr int PER = R * (int)(sizeof(Real) / 4);
+    constexpr int CB = PER >= 16 ? 2 : PER >= 8 ? 4 : 8;
+    const int lane = lane_id();
+    const AW_GLOBAL Real *alpha = (const AW_GLOBAL Real *)d.alpha;
+    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
+    const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
+    const float uf = (float)uw;
+    pv = k;
+    int pos = 0;
+    while (pos < n) {
+        // weights into k, in FP32 for the tests
+        const Target<Real> t = tb_target<Real, R>(d, b, k);
+        float tf[R], tk[R];
+        {
+            int ti[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) ti[r] = info[r * 64 + lane];
+            Real tr[R];
+            tb_weights<Real, R>(d, ti, t, tr);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                tf[r] = (float)tr[r];
+                tk[r] = readlane_r(tf[r], t.lk);   // the states of k's lane
+            }
+        }
+        bool moved = false;
+        for (; pos < n && !moved; ) {
+            // lane's column of this chunk, and the entries of k's lane there:
+            // the states before k in its lane, and k itself
+            const int j = pos + (lane >> 2);
+            const AW_GLOBAL Real *grow = alpha + (size_t)(ce - 1 - min(j, n - 1)) * RW + t.lk;
+            Real gv[R];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (r <= t.rk) gv[r] = grow[r * 64];
+            // columns c and c + 8 together, so that their first fold follows
+            // at once; value 2c is column c's total, 2c + 1 its sum over the
+            // lanes before k's
+            float v[16];
+#pragma unroll
+            for (int c0 = 0; c0 < 8; c0 += CB / 2) {
+                if (pos + c0 >= n) {
+#pragma unroll
+                    for (int c = 0; c < CB; c++) v[2 * c0 + c] = 0.f;
+                    continue;
+                }
+                Real rv[CB][R];
+#pragma unroll
+                for (int c = 0; c < CB; c++)
+                    row_load<Real, R>(alpha, ce - 1 - min(pos + c0 + c / 2 + (c & 1) * 8, n - 1), rv[c]);
+#pragma unroll
+                for (int c = 0; c < CB; c += 2) {
+                    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        s0 += (float)rv[c][r] * tf[r];
+                        s1 += (float)rv[c + 1][r] * tf[r];
+                    }
+                    v[2 * (c0 + c / 2)] = fold32(s0, s1);
+                    v[2 * (c0 + c / 2) + 1] =
+                        fold32(lane < t.lk ? s0 : 0.f, lane < t.lk ? s1 : 0.f);
+                }
+            }
+            const float own = sum32(v), oth = dpp_r<DPP_QUAD_SWAP2>(own);
+            const float tot = (lane & 2) ? oth : own;
+            float below = (lane & 2) ? own : oth, at = 0.f;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (r < t.rk) below += (float)gv[r] * tk[r];
+                else if (r == t.rk) at = (float)gv[r] * tk[r];
+            }
+            const float pick = bperm_r(uf, 4 * min(j, 63)) * tot, guard = tot * 0x1p-13f;
+            const bool stay = pick > below + guard && pick < below + at - guard;
+            unsigned long long odd = __ballot(j < n && !stay);
+            while (odd) {
+                const int x = pos + (((int)__ffsll((long long)odd) - 1) >> 2);
+                Real rv[R], tr[R];
+                int ti[R];
+                row_load<Real, R>(alpha, ce - 1 - x, rv);
+#pragma unroll
+                for (int r = 0; r < R; r++) ti[r] = info[r * 64 + lane];
+                tb_weights<Real, R>(d, ti, t, tr);
+                const int kn = sample_state<Real, R>(rv, tr, S, readlane_d(uw, x));
+                if (kn != k) {
+                    k = kn;
+                    pv = lane >= x ? k : pv;
+                    pos = x + 1;
+                    moved = true;
+                    break;
+                }
+                odd &= ~(0xfull << (4 * (x - pos)));
+            }
+            if (!moved) pos += 16;
+        }
+    }
+    if (sw) {
+        // the switch into block b (TransMatrixSwitch::get, trans.h:201-209)
+        const int rs = cp(d.srcs)[2 * b], cs = cp(d.srcs)[2 * b + 1];
+        const AW_GLOBAL Real *cn = planes<Real>(d, b, RW);
+        const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)b * RW;
+        const int pk = lane_pos(k, R);
+        const Real rrk = cn[CRR * RW + pk], crk = cn[CCR * RW + pk];
+        Real rv[R], tr[R];
+        row_load<Real, R>(alpha, ce - n - 1, rv);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int s = lane * R + r;
+            const int dt = detn[r * 64 + lane];
+            const Real dp = cn[CDP * RW + r * 64 + lane];
+            tr[r] = (s == cs) ? crk : (s == rs) ? rrk : (dt == k ? dp : Real(0));
+        }
+        k = sample_state<Real, R>(rv, tr, cp(d.soff)[b] - cp(d.soff)[b - 1], readlane_d(uw, n));
+        pv = lane >= n ? k : pv;
+    }
+    return k;
+}
+
+// Sample columns hi, hi-1, .., lo given the state k at column hi+1 (block
+// blk), storing the samples in dst (nothing when dst is null).  With cmp the walk stops at the first column whose sample is the
+// one already stored in dst (the chains have met: the rest is that path) and
+// returns it; else it returns -1, k being the state of column lo.  The
+// uniform of column col is u[L-1-col].  Called by the whole workgroup with
+// the same arguments.
+template <class Real, int R, int NW>
+__device__ __forceinline__ int tb_walk(const DevInst &d, int *lds, int hi, int lo, int &k, int blk,
+                                       AW_GLOBAL int *dst, bool cmp)
+{
+    constexpr int RW = 64 * R;
+    const int lane = lane_id(), L = d.L;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int *res = lds;
+    unsigned *pred = (unsigned *)(lds + TB_RES * NW);   // NW tables of RW 16-bit states
+    const AW_GLOBAL double *ug = gp(d.u);
+    const AW_GLOBAL int *bstart = gp(d.bstart);
+    int cur = hi + 1, kc = k, bc = blk;
+    // lane i holds the first column of block bw - i
+    int bw = bc, bsv = bstart[max(bw - lane, 0)];
+    while (cur > lo) {
+        if (bw - bc > 63 - NW) {
+            bw = bc;
+            bsv = bstart[max(bw - lane, 0)];
+        }
+        // this wave's unit: the wave-th run of columns to the left of cur,
+        // each within one block and at most TB_SEG long
+        int ce = cur, b = bc, ct = 0, nce = 0, nb = 0;
+        bool sw = false, live = false;
+        unsigned swm = 0;   // units before this one that end in a switch
+        for (int i = 0;; i++) {
+            const int bs = __builtin_amdgcn_readlane(bsv, bw - b);
+            ct = max(max(bs, lo), ce - TB_SEG);
+            sw = ct == bs && ct > lo;
+            nce = sw ? ct - 1 : ct;
+            nb = sw ? b - 1 : b;
+            if (i == wave) {
+                live = true;
+                break;
+            }
+            if (nce <= lo) break;
+            if (sw) swm |= 1u << i;
+            ce = nce;
+            b = nb;
+        }
+        const int n = ce - ct;
+        double uw = 0.0;
+        int old = -1;
+        if (live) {
+            const int c = max(ce - 1 - lane, 0);
+            uw = ug[L - 1 - c];
+            if (cmp) old = dst[max(c, lo)];
+            if (sw && wave < NW - 1) {
+                const AW_GLOBAL unsigned *src =
+                    (const AW_GLOBAL unsigned *)gp(d.pred) + (size_t)b * (RW / 2);
+                for (int x = lane; x < RW / 2; x += 64) pred[wave * (RW / 2) + x] = src[x];
+            }
+        }
+        __syncthreads();
+        // the predicted entry state
+        unsigned h = (unsigned)kc;
+        for (int i = 0; i < wave && live; i++) {
+            if (!(swm >> i & 1)) continue;
+            h = __builtin_amdgcn_readfirstlane(
+                (int)((const unsigned short *)pred)[i * RW + h]);
+            if (h == TB_NONE) live = false;
+        }
+        int pv = -1, out = -1, match = -1;
+        const int nl = sw ? n : n - 1;   // last lane holding a sample
+        if (live) {
+            out = tb_unit<Real, R>(d, b, ce, n, sw, (int)h, uw, pv);
+            if (cmp) {
+                const unsigned long long m = __ballot(lane <= nl && old == pv);
+                if (m) match = ce - (int)__ffsll((long long)m);
+            }
+        }
+        if (lane == 0) {
+            res[RES_OUT * NW + wave] = out;
+            res[RES_HYP * NW + wave] = (int)h;
+            res[RES_FLAG * NW + wave] = (live ? UNIT_LIVE : 0) | (nce <= lo ? UNIT_FINAL : 0);
+            res[RES_NEXT * NW + wave] = nce;
+            res[RES_BLK * NW + wave] = nb;
+            res[RES_MATCH * NW + wave] = match;
+        }
+        __syncthreads();
+        // the units up to the first whose outcome the next did not assume
+        const int i0 = min(lane, NW - 1), i1 = min(lane + 1, NW - 1);
+        const int o0 = res[RES_OUT * NW + i0], h1 = res[RES_HYP * NW + i1];
+        const int f0 = res[RES_FLAG * NW + i0], f1 = res[RES_FLAG * NW + i1];
+        const int m0 = res[RES_MATCH * NW + i0];
+        const bool ok = lane < NW - 1 && !(f0 & UNIT_FINAL) && (f1 & UNIT_LIVE) && o0 == h1;
+        const int last = (int)__ffsll((long long)~__ballot(ok)) - 1;
+        int stop = -1;
+        if (cmp) {
+            const unsigned long long m = __ballot(lane <= last && m0 >= 0);
+            if (m) stop = __builtin_amdgcn_readlane(m0, (int)__ffsll((long long)m) - 1);
+        }
+        if (wave <= last && dst) {
+            const int c = ce - 1 - lane;
+            if (lane <= nl && c > stop) dst[c] = pv;
+        }
+        cur = __builtin_amdgcn_readfirstlane(res[RES_NEXT * NW + last]);
+        kc = __builtin_amdgcn_readfirstlane(res[RES_OUT * NW + last]);
+        bc = __builtin_amdgcn_readfirstlane(res[RES_BLK * NW + last]);
+        if (stop >= 0) return stop;
+    }
+    k = kc;
+    return -1;
+}
+
+template <class Real, int R, int NW>
+__device__ __forceinline__ void tb_spec(const DevInst d, const Chunk &ch, int *start, int *end, int *lds)
+{
+    const int L = d.L;
+    AW_GLOBAL int *path = gp(d.path);
+    // the chain's first state: from the last column (or the state it is
+    // conditioned on), or from column cw alone
+    int b = ch.last ? d.B - 1 : find_owner(cp(d.bstart), d.B, ch.cw);
+    int k = d.last_state;
+    if (!ch.last || k < 0) k = sample_alone<Real, R>(d, ch.cw, b, cp(d.u)[L - 1 - ch.cw]);
+    int k1 = -1;
+    if (ch.last && threadIdx.x == 0) path[L - 1] = k;
+    // the warm-up (no columns in the last tile), then the tile
+#pragma unroll 1
+    for (int ph = ch.last ? 1 : 0; ph < 2; ph++) {
+        const int top = ph ? (ch.last ? L - 1 : ch.c1) : ch.cw;
+        if (ph && !ch.last) {
+            k1 = k;
+            b = find_owner(cp(d.bstart), d.B, ch.c1);
+        }
+        tb_walk<Real, R, NW>(d, lds, top - 1, ph ? ch.c0 : ch.c1, k, b, ph ? path : nullptr, false);
+    }
+    if (threadIdx.x == 0) {
+        *start = k1;
+        *end = k;
+    }
+}
+
+template <class Real, int R, int NW>
+__device__ __forceinline__ void tb_rerun(const DevInst d, const Chunk &ch, int k, int *res, int *lds)
+{
+    AW_GLOBAL int *path = gp(d.path);
+    const int b = find_owner(cp(d.bstart), d.B, ch.c1);
+    const int col = tb_walk<Real, R, NW>(d, lds, ch.c1 - 1, ch.c0, k, b, path, true);
+    if (threadIdx.x == 0) {
+        res[0] = col;
+        res[1] = col >= 0 ? path[ch.c0] : k;
+    }
+}
+
+// calls f<R>() for the instance's states per lane
+#define TB_FOR_R(R_, CALL)                          \
+    switch (R_) {                                   \
+    case 1: { constexpr int R = 1; CALL; break; }   \
+    case 2: { constexpr int R = 2; CALL; break; }   \
+    case 4: { constexpr int R = 4; CALL; break; }   \
+    case 6: { constexpr int R = 6; CALL; break; }   \
+    case 8: { constexpr int R = 8; CALL; break; }   \
+    case 12: { constexpr int R = 12; CALL; break; } \
+    default: { constexpr int R = 16; CALL; break; } \
+    }
+
+template <class Real, bool BIG>
+__global__ __launch_bounds__(64 * tb_waves<BIG>()) void k_tb_spec(const DevInst *__restrict__ D,
+                                                                  const Chunk *__restrict__ chunks,
+                                                                  const int *__restrict__ list,
+                                                                  int *__restrict__ start,
+                                                                  int *__restrict__ end)
+{
+    extern __shared__ int tb_dyn[];
+    constexpr int NW = tb_waves<BIG>();
+    const int j = list[blockIdx.x];
+    const Chunk ch = chunks[j];
+    const DevInst &d = D[ch.inst];
+    if ((d.R > 16) != BIG) return;   // the other symbol's tile
+    if constexpr (BIG) tb_spec<Real, 32, NW>(d, ch, start + j, end + j, tb_dyn);
+    else TB_FOR_R(d.R, (tb_spec<Real, R, NW>(d, ch, start + j, end + j, tb_dyn)))
+}
+
+template <class Real, bool BIG>
+__global__ __launch_bounds__(64 * tb_waves<BIG>()) void k_tb_rerun(const DevInst *__restrict__ D,
+                                                                   const Chunk *__restrict__ chunks,
+                                                                   const int *__restrict__ idx,
+                                                                   const int *__restrict__ k1,
+                                                                   int *__restrict__ res)
+{
+    extern __shared__ int tb_dyn[];
+    constexpr int NW = tb_waves<BIG>();
+    const Chunk ch = chunks[idx[blockIdx.x]];
+    const DevInst &d = D[ch.inst];
+    const int k = k1[blockIdx.x];
+    int *rs = res + 2 * blockIdx.x;
+    if ((d.R > 16) != BIG) return;   // the other symbol's tile
+    if constexpr (BIG) tb_rerun<Real, 32, NW>(d, ch, k, rs, tb_dyn);
+    else TB_FOR_R(d.R, (tb_rerun<Real, R, NW>(d, ch, k, rs, tb_dyn)))
+}
+
+// Predicted sources: for every state k of block b the state j of block b-1
+// with the largest switch probability P(j -> k) (ties: the larger index),
+// TB_NONE where no state leads to k.  One workgroup per block; the
+// candidates (deterministic targets, then the two dense rows) meet in LDS.
+__global__ __launch_bounds__(256) void k_tb_pred(const DevInst *__restrict__ D,
+                                                 const int *__restrict__ blkoff, int ninst)
+{
+    extern __shared__ unsigned long long best[];
+    const int inst = find_owner(blkoff, ninst, (int)blockIdx.x);
+    const DevInst &d = D[inst];
+    const int b = blockIdx.x - blkoff[inst];
+    if (b == 0) return;
+    const int R = d.R, RW = 64 * R;
+    const int S1 = cp(d.soff)[b] - cp(d.soff)[b - 1], S2 = cp(d.soff)[b + 1] - cp(d.soff)[b];
+    const int rs = cp(d.srcs)[2 * b], cs = cp(d.srcs)[2 * b + 1];
+    auto weight = [&](int plane, int p) -> float {
+        const size_t x = ((size_t)b * NCOEF + plane) * RW + p;
+        return d.fp32 ? gp(d.lcoef32)[x] : (float)gp(d.lcoef)[x];
+    };
+    auto key = [](float w, int j) {
+        return (unsigned long long)__float_as_uint(w) << 32 | (unsigned)(j + 1);
+    };
+    for (int x = threadIdx.x; x < RW; x += 256) best[x] = 0;
+    __syncthreads();
+    for (int p = threadIdx.x; p < RW; p += 256) {
+        const int j = (p & 63) * R + (p >> 6);
+        const int t = gp(d.ldet)[(size_t)b * RW + p];
+        if (j < S1 && t >= 0 && t < S2 && j != rs && j != cs) atomicMax(&best[t], key(weight(CDP, p), j));
+    }
+    __syncthreads();
+    auto out = gp(d.pred) + (size_t)b * RW;
+    for (int p = threadIdx.x; p < RW; p += 256) {
+        const int k = (p & 63) * R + (p >> 6);
+        unsigned long long m = best[k];
+        if (rs >= 0) {
+            const float w = weight(CRR, p);
+            if (w > 0.f) m = max(m, key(w, rs));
+        }
+        if (cs >= 0) {
+            const float w = weight(CCR, p);
+            if (w > 0.f) m = max(m, key(w, cs));
+        }
+        out[k] = m ? (unsigned short)((unsigned)m - 1) : (unsigned short)TB_NONE;
+    }
+}
+
+template <class Kern, class... Args>
+int launch(Kern kern, int grid, int block, size_t sh, hipStream_t st, Args... args)
+{
+    if (set_lds_limit((const void *)kern, sh)) return 1;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), sh, st, args...);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
+}  // namespace
+
+size_t tb_lds_bytes(int R)
+{
+    const int NW = R > 16 ? tb_waves<true>() : tb_waves<false>();
+    return (size_t)NW * (TB_RES * sizeof(int) + 64 * R * sizeof(short));
+}
+
+int launch_tb_pred(const DevInst *D, const int *blkoff, int ninst, int nblk, int Rmax, hipStream_t s)
+{
+    return launch(k_tb_pred, nblk, 256, sizeof(unsigned long long) * 64 * Rmax, s, D, blkoff, ninst);
+}
+
+int launch_tb_spec(bool fp32, bool big, const DevInst *D, const Chunk *chunks, const int *list,
+                   int n, size_t sh, int *start, int *end, hipStream_t s)
+{
+    const int wg = 64 * (big ? tb_waves<true>() : tb_waves<false>());
+    auto kern = fp32 ? (big ? k_tb_spec<float, true> : k_tb_spec<float, false>)
+                     : (big ? k_tb_spec<double, true> : k_tb_spec<double, false>);
+    return launch(kern, n, wg, sh, s, D, chunks, list, start, end);
+}
+
+int launch_tb_rerun(bool fp32, bool big, const DevInst *D, const Chunk *chunks, const int *idx,
+                    const int *k1, int n, size_t sh, int *res, hipStream_t s)
+{
+    const int wg = 64 * (big ? tb_waves<true>() : tb_waves<false>());
+    auto kern = fp32 ? (big ? k_tb_rerun<float, true> : k_tb_rerun<float, false>)
+                     : (big ? k_tb_rerun<double, true> : k_tb_rerun<double, false>);
+    return launch(kern, n, wg, sh, s, D, chunks, idx, k1, res);
+}
+
+}  // namespace aw
