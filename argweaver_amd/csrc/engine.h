@@ -88,6 +88,10 @@ enum : int {
     NCOEF
 };
 
+// mark in ldet: the target has several sources (set by k_tb_pred, which also
+// sets the targets of the two dense rows' sources to -1)
+enum : int { DET_SHARED = 1 << 30 };
+
 // transposed position of state s in a lane-run row
 __host__ __device__ inline int lane_pos(int s, int R) { return (s % R) * 64 + s / R; }
 

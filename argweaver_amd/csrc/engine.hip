@@ -12,17 +12,16 @@
 //                  lane-run layout (engine.h)
 //   k_var_emit_b   one wave per variant column: Felsenstein partials and the
 //                  emission row over the block's states
-//   k_fw_all       one wave per instance over all its columns, every
-//                  instance of a batch in one launch (a switch on R picks
-//                  the instantiation).  Lane l owns states l*R .. l*R+R-1
-//                  (node-major).  The same-branch part of the transition is
-//                  a per-branch prefix and suffix sum (in-lane scan plus a
-//                  DPP wave-shift carry chain across the few lanes a branch
-//                  spans); the other-branch part goes through the per-time
-//                  sums (FP64 LDS atomics into 16 lane-group copies, a
-//                  lane-pair reduction, readlane broadcast) and the (a,b)
-//                  table, the result reaching each state by ds_bpermute; a
-//                  column costs O(S + T^2) and rows are written coalesced.
+//   k_fw_all       two waves per tile (an instance, or a part of a long one
+//                  in FP32) over all its columns, every tile of a batch in
+//                  one launch (forward_kernels.h).  Lane l owns states l*R ..
+//                  l*R+R-1 (node-major).  The same-branch part of the
+//                  transition is a per-branch prefix and suffix sum (in-lane
+//                  scan plus a DPP wave-shift carry chain across the few
+//                  lanes a branch spans), run by one wave; the other-branch
+//                  part goes through the per-time sums (FP64 LDS atomics) and
+//                  the (a,b) table, run by the other; a column costs
+//                  O(S + T^2) and rows are written coalesced.
 //   k_lnl_b        per-instance sum of log normalisers (FP64)
 //   traceback      one workgroup per column tile (traceback.hip).  A tile
 //                  before the last runs a speculative chain (a state sampled

@@ -18,19 +18,17 @@ int launch_fw_check(const DevInst *dD, const FwTile *tiles, const int *idx, int 
     return 0;
 }
 
-// LDS bytes of the forward kernel for R states per lane
 size_t fw_lds_bytes(bool fp32, int R)
 {
-    auto one = [&](auto f32, auto f64) { return fp32 ? 4 * (size_t)f32 : 8 * (size_t)f64; };
     switch (R) {
-    case 1: return one(fw_lds_reals<float, 1>(), fw_lds_reals<double, 1>());
-    case 2: return one(fw_lds_reals<float, 2>(), fw_lds_reals<double, 2>());
-    case 4: return one(fw_lds_reals<float, 4>(), fw_lds_reals<double, 4>());
-    case 6: return one(fw_lds_reals<float, 6>(), fw_lds_reals<double, 6>());
-    case 8: return one(fw_lds_reals<float, 8>(), fw_lds_reals<double, 8>());
-    case 12: return one(fw_lds_reals<float, 12>(), fw_lds_reals<double, 12>());
-    case 16: return one(fw_lds_reals<float, 16>(), fw_lds_reals<double, 16>());
-    default: return one(fw_lds_reals<float, 32>(), fw_lds_reals<double, 32>());
+    case 1: return fp32 ? sizeof(FwShared<float, 1>) : sizeof(FwShared<double, 1>);
+    case 2: return fp32 ? sizeof(FwShared<float, 2>) : sizeof(FwShared<double, 2>);
+    case 4: return fp32 ? sizeof(FwShared<float, 4>) : sizeof(FwShared<double, 4>);
+    case 6: return fp32 ? sizeof(FwShared<float, 6>) : sizeof(FwShared<double, 6>);
+    case 8: return fp32 ? sizeof(FwShared<float, 8>) : sizeof(FwShared<double, 8>);
+    case 12: return fp32 ? sizeof(FwShared<float, 12>) : sizeof(FwShared<double, 12>);
+    case 16: return fp32 ? sizeof(FwShared<float, 16>) : sizeof(FwShared<double, 16>);
+    default: return fp32 ? sizeof(FwShared<float, 32>) : sizeof(FwShared<double, 32>);
     }
 }
 

@@ -2,6 +2,8 @@
 // forward_f32.hip and forward_f64.hip.
 #pragma once
 
+#include <type_traits>
+
 #include "forward.h"
 #include "kernel_util.h"
 
@@ -15,97 +17,245 @@ namespace aw {
 // NT1 is a compile-time bound on the T-1 time bins (19 for the usual 20
 // time points), so the per-time loops are fully unrolled without padding.
 //
-// Per block, each lane keeps in registers the factor planes of its R
-// states, two 0/1 factors per state (not the first / not the last state of
-// its branch: they cut the prefix and suffix sums), and whether the lane
-// holds a branch start / end (the carry stops there).  Per state it also
-// keeps its time, which gives both the lane holding the other-branch term
-// of its time and where its value goes in the per-time partial sums;
-// padding states use time bin 31, whose term is 0, so they come out 0 with
-// no mask.  The 0/1 factors are floats in both precisions: FP64 runs apply
-// them as selects, which keeps their registers at one per state.
-template <class Real, int R, int NT1>
+// A tile's workgroup has two waves, and a column passes between them twice:
+//
+//   lanes wave   lane l holds the R states l*R .. l*R+R-1 of the lane-run
+//                layout: the scan along the branches, the emission, the new
+//                column, which it hands over in LDS
+//   sums wave    the per-time sums of that column, their product with the
+//                (a,b) table, the normaliser, which it hands back; then it
+//                stores the row
+//
+// The lanes wave runs its scan while the sums wave works.  The kernel is bound
+// by the latency of that chain: hand over, atomics, their sums, the product,
+// hand back, about 900 cycles at 8 FP32 states per lane.  One wave doing both
+// is bound by its instruction issue (a dependent instruction every 8 cycles, an
+// independent one every 5); four waves sharing the slots out lost more to
+// atomics from several waves meeting in LDS than they gained.
+//
+// us per column at R = 1 / 2 / 4 / 6 / 8 / 12 / 16 states per lane, one
+// instance on MI355X, switches included: FP32 0.44 0.41 0.39 0.45 0.52 0.59
+// 0.83 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
+// 0.99 1.24 1.82); FP64 0.52 0.46 0.43 0.47 0.53 0.84 1.62 (1.15 0.95 1.05
+// 1.12 1.30 1.67 2.74).
+constexpr int FW_THREADS = 128;
+
+// Per block, each lane of the lanes wave keeps in registers the factor planes
+// of its R states, two 0/1 factors per state (not the first / not the last
+// state of its branch: they cut the prefix and suffix sums) with their running
+// products from the lane's start / end (whether the carry reaches the state),
+// and whether the lane holds a branch start / end (the carry stops there), and
+// the state's time; padding states use time bin 31, whose term is 0, so they
+// come out 0 with no mask.  The 0/1 factors have the table's type, so that
+// applying one is one instruction; in FP64 with more than 12 states per lane
+// they are floats applied as selects, for their registers.
+template <class Real, int R>
 struct FwLane {
     Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R];
-    float nf[R], nl[R];
-    int boff[R];     // 4 * time: ds_bpermute address of the lane holding TF[time]
+    using Fac = std::conditional_t<(sizeof(Real) * R <= 96), Real, float>;
+    Fac nf[R], nl[R], ff[R], fl[R];
+    const AW_LDS Real *tf[R];   // the handed-back term of the state's time
     Real m1, m2;
-    Real tmc[NT1];   // lane b < T-1: column b of the (a,b) table (FP32)
+    int K;           // carry steps: lanes a branch of the block spans
 };
 
-// x times a 0/1 factor m (a select in FP64: the same value)
-template <class Real>
-__device__ __forceinline__ Real keep(Real x, float m)
+// What the lanes wave loads of a block: its planes, and the switch into it
+template <class Real, int R>
+struct FwRaw {
+    Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R], rr[R], cr[R], dp[R];
+    int info[R], dt[R];
+};
+
+// x times a 0/1 factor m, and acc + x * m: a product where the factor has the
+// table's type, a select (the same value) where it is a float beside doubles
+template <class Real, class F>
+__device__ __forceinline__ Real keep(Real x, F m)
 {
-    if constexpr (sizeof(Real) == 4) return x * m;
-    else return (m != 0.f) ? x : Real(0);
+    if constexpr (sizeof(Real) == sizeof(F)) return x * m;
+    else return (m != F(0)) ? x : Real(0);
+}
+template <class Real, class F>
+__device__ __forceinline__ Real add_kept(Real acc, Real x, F m)
+{
+    if constexpr (sizeof(Real) == sizeof(F)) return fma(x, m, acc);
+    else return acc + ((m != F(0)) ? x : Real(0));
 }
 
-// The (a,b) table lives in registers (lane b holds column b) for FP32 and
-// in LDS for FP64, where registers are short.
-template <class Real>
-constexpr bool tm_in_lds()
-{
-    return sizeof(Real) == 8;
-}
-
-// Per-time sums are accumulated in GCOPY copies of the 32 time bins, one
-// copy per group of 64 / GCOPY consecutive lanes, so that the LDS atomics of
-// one instruction seldom meet at one address (colliding atomics are
-// serialised).  Bin a, copy c sits at GP[a * GCOPY + c].  The sums are FP64
-// in both precisions: ds_add_f64 is much faster than ds_add_f32 here.
+// Per-time sums are accumulated in GCOPY copies of the 32 time bins, copy
+// lane % 16 at GP[a * GCOPY + copy].  LDS takes sixteen consecutive lanes of
+// an atomic at a time, 3 cycles and 3 more for every further lane at one
+// address, 2 for every further lane in one bank: with a copy a lane and
+// sixteen copies to a bin neither happens (12.6 cycles an atomic; 44 where
+// four lanes share a copy and their states a time).  The sums are FP64 in
+// both precisions: ds_add_f32 takes 192 cycles.
 constexpr int GCOPY = 16;
 
-template <class Real, int R, int NT1>
-__device__ __forceinline__ void fw_load_block(const DevInst &d, int b, FwLane<Real, R, NT1> &fl,
-                                              Real *TMS)
+// The time bin a lane reduces and multiplies: the wave's 16-lane rows 0 and 1
+// take the bins a with a % 4 < 2, rows 2 and 3 the others, position j of a
+// row the j-th of them.  Rows of a pair each read half of the copies.  A row
+// then holds all the sums its lanes need for their half of the product with
+// the (a,b) table (lane b and lane 32 + b: column b), and takes them by a row
+// broadcast inside the multiply-add instead of a readlane per bin.
+__device__ __forceinline__ int bin_of(int row, int j) { return 4 * (j >> 1) + (j & 1) + 2 * (row >> 1); }
+
+// acc0 / acc1 += g[j] * tm[j] over the even / odd positions j of the lane's
+// row.  The compiler does not fuse these broadcasts into the multiply-adds;
+// the waits cover the register hazards it cannot see inside.
+#define FW_BC(op, acc, src, j) op " " acc ", %2, " src " row_newbcast:" #j " row_mask:0xf bank_mask:0xf\n"
+#define FW_BC10(op)                                                                         \
+    "s_nop 1\n" FW_BC(op, "%0", "%3", 0) FW_BC(op, "%1", "%4", 1) FW_BC(op, "%0", "%5", 2)   \
+    FW_BC(op, "%1", "%6", 3) FW_BC(op, "%0", "%7", 4) FW_BC(op, "%1", "%8", 5)              \
+    FW_BC(op, "%0", "%9", 6) FW_BC(op, "%1", "%10", 7) FW_BC(op, "%0", "%11", 8)            \
+    FW_BC(op, "%1", "%12", 9)
+#define FW_BC16(op)                                                                         \
+    FW_BC10(op) FW_BC(op, "%0", "%13", 10) FW_BC(op, "%1", "%14", 11)                       \
+    FW_BC(op, "%0", "%15", 12) FW_BC(op, "%1", "%16", 13) FW_BC(op, "%0", "%17", 14)        \
+    FW_BC(op, "%1", "%18", 15)
+#define FW_T10(t) "v"(t[0]), "v"(t[1]), "v"(t[2]), "v"(t[3]), "v"(t[4]), "v"(t[5]), "v"(t[6]), "v"(t[7]), "v"(t[8]), "v"(t[9])
+#define FW_T16(t) FW_T10(t), "v"(t[10]), "v"(t[11]), "v"(t[12]), "v"(t[13]), "v"(t[14]), "v"(t[15])
+__device__ __forceinline__ void bin_product(float g, const float (&t)[10], float &a0, float &a1)
+{
+    asm(FW_BC10("v_fmac_f32_dpp") "s_nop 1" : "+v"(a0), "+v"(a1) : "v"(g), FW_T10(t));
+}
+__device__ __forceinline__ void bin_product(float g, const float (&t)[16], float &a0, float &a1)
+{
+    asm(FW_BC16("v_fmac_f32_dpp") "s_nop 1" : "+v"(a0), "+v"(a1) : "v"(g), FW_T16(t));
+}
+__device__ __forceinline__ void bin_product(double g, const double (&t)[10], double &a0, double &a1)
+{
+    asm(FW_BC10("v_fmac_f64_dpp") "s_nop 1" : "+v"(a0), "+v"(a1) : "v"(g), FW_T10(t));
+}
+__device__ __forceinline__ void bin_product(double g, const double (&t)[16], double &a0, double &a1)
+{
+    asm(FW_BC16("v_fmac_f64_dpp") "s_nop 1" : "+v"(a0), "+v"(a1) : "v"(g), FW_T16(t));
+}
+
+// carry chains of at most this many steps run in full; longer ones (few states
+// per lane) stop at the block's longest branch
+constexpr int FW_KFIX = 8;
+
+// N steps of the carry of the same-branch sums across lanes: y1 = p1 + m1 *
+// (y1 of the lane before), y2 = p2 + m2 * (y2 of the lane after).  In FP32 the
+// shift is part of the multiply-add; two instructions of the other chain lie
+// between a register's write and its shifted read.
+template <int N>
+__device__ __forceinline__ void carry_steps(float p1, float p2, float m1, float m2, float &y1, float &y2)
+{
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        float z1, z2;
+        asm("v_mov_b32 %0, %2\n"
+            "v_mov_b32 %1, %3\n"
+            "v_fmac_f32_dpp %0, %4, %6 wave_shr:1 row_mask:0xf bank_mask:0xf\n"
+            "v_fmac_f32_dpp %1, %5, %7 wave_shl:1 row_mask:0xf bank_mask:0xf"
+            : "=&v"(z1), "=&v"(z2)
+            : "v"(p1), "v"(p2), "v"(y1), "v"(y2), "v"(m1), "v"(m2));
+        y1 = z1;
+        y2 = z2;
+    }
+}
+template <int N>
+__device__ __forceinline__ void carry_steps(double p1, double p2, double m1, double m2, double &y1, double &y2)
+{
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        y1 = fma(m1, dpp_r<DPP_WAVE_SHR1>(y1), p1);
+        y2 = fma(m2, dpp_r<DPP_WAVE_SHL1>(y2), p2);
+    }
+}
+
+// x of the lane and of its partner in the other 16-lane row of the pair, or
+// in the other half of the wave, added (the same sum in both)
+__device__ __forceinline__ double add_rows(double x)
+{
+    const long long v = __double_as_longlong(x);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+    return __longlong_as_double((long long)((unsigned long long)hi[0] << 32 | lo[0])) +
+           __longlong_as_double((long long)((unsigned long long)hi[1] << 32 | lo[1]));
+}
+__device__ __forceinline__ float add_halves(float x)
+{
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+__device__ __forceinline__ double add_halves(double x)
+{
+    const long long v = __double_as_longlong(x);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+    return __longlong_as_double((long long)((unsigned long long)hi[0] << 32 | lo[0])) +
+           __longlong_as_double((long long)((unsigned long long)hi[1] << 32 | lo[1]));
+}
+
+// the barrier of a tile's workgroup, ordering its LDS accesses
+__device__ __forceinline__ void fw_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Loaded values go straight into their registers: selecting or copying a
+// value whose load is still in flight makes the compiler wait for it at once.
+template <class Real, int R>
+__device__ __forceinline__ void fw_load_raw(const DevInst &d, int b, FwRaw<Real, R> &x)
 {
     constexpr int RW = 64 * R;
-    const int lane = threadIdx.x, T1 = d.T - 1;
     // uniform bases, per-lane index: loads use the scalar-base address form
     const AW_GLOBAL Real *coef = planes<Real>(d, b, RW);
     const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    int ti[R];
+    const AW_GLOBAL int *det = gp(d.ldet) + (size_t)b * RW;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const int x = r * 64 + lane;
-        fl.cf[r] = coef[CF * RW + x];
-        fl.cd[r] = coef[CD * RW + x];
-        fl.cg[r] = coef[CG * RW + x];
-        fl.ck[r] = coef[CK * RW + x];
-        fl.cj[r] = coef[CJ * RW + x];
-        fl.ce[r] = coef[CE * RW + x];
-        ti[r] = info[x];
+        const int i = r * 64 + (threadIdx.x & 63);
+        x.info[r] = info[i];
+        x.dt[r] = det[i];
+        x.cf[r] = coef[CF * RW + i];
+        x.cd[r] = coef[CD * RW + i];
+        x.cg[r] = coef[CG * RW + i];
+        x.ck[r] = coef[CK * RW + i];
+        x.cj[r] = coef[CJ * RW + i];
+        x.ce[r] = coef[CE * RW + i];
+        x.rr[r] = coef[CRR * RW + i];
+        x.cr[r] = coef[CCR * RW + i];
+        x.dp[r] = coef[CDP * RW + i];
     }
+}
+
+template <class Real, int R, int NT1>
+__device__ __forceinline__ void fw_unpack(const FwRaw<Real, R> &x, const Real *tv, FwLane<Real, R> &fl)
+{
     bool first = false, last = false;
+    using Fac = typename FwLane<Real, R>::Fac;
+    Fac f1 = 1, f2 = 1;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const int t = ti[r] & INFO_TIME;
-        fl.nf[r] = (ti[r] & INFO_FIRST) ? 0.f : 1.f;
-        fl.nl[r] = (ti[r] & INFO_LAST) ? 0.f : 1.f;
-        fl.boff[r] = t * 4;
-        first |= (ti[r] & INFO_FIRST) != 0;
-        last |= (ti[r] & INFO_LAST) != 0;
+        fl.cf[r] = x.cf[r];
+        fl.cd[r] = x.cd[r];
+        fl.cg[r] = x.cg[r];
+        fl.ck[r] = x.ck[r];
+        fl.cj[r] = x.cj[r];
+        fl.ce[r] = x.ce[r];
+        fl.nf[r] = (x.info[r] & INFO_FIRST) ? Fac(0) : Fac(1);
+        fl.nl[r] = (x.info[r] & INFO_LAST) ? Fac(0) : Fac(1);
+        fl.ff[r] = f1 *= fl.nf[r];
+        fl.tf[r] = (const AW_LDS Real *)tv + (x.info[r] & INFO_TIME);
+        first |= (x.info[r] & INFO_FIRST) != 0;
+        last |= (x.info[r] & INFO_LAST) != 0;
     }
+#pragma unroll
+    for (int r = R - 1; r >= 0; r--) fl.fl[r] = f2 *= fl.nl[r];
     fl.m1 = first ? Real(0) : Real(1);
     fl.m2 = last ? Real(0) : Real(1);
-    // Loaded values go straight into their registers: selecting or copying
-    // a value whose load is still in flight makes the compiler wait for it
-    // at once.  Indices are clamped instead; entries a >= T-1 meet a zero
-    // per-time sum and lanes >= T-1 compute terms nobody uses.
-    const AW_GLOBAL double *tmb = gp(d.tm) + (size_t)b * T1 * T1;
-    const int lc = min(lane, T1 - 1);
-    if (tm_in_lds<Real>()) {
-        // TMS[a * 32 + b] = P(a -> b); lanes 32..63 duplicate lanes 0..31
-        double t[NT1];
-#pragma unroll
-        for (int a = 0; a < NT1; a++) t[a] = tmb[min(a, T1 - 1) * T1 + lc];
-#pragma unroll
-        for (int a = 0; a < NT1; a++)
-            if (lane < 32) TMS[a * 32 + lane] = (Real)t[a];
-    } else {
-#pragma unroll
-        for (int a = 0; a < NT1; a++) fl.tmc[a] = (Real)tmb[min(a, T1 - 1) * T1 + lc];
+    // the carry crosses lanes without a branch start (end): more steps than
+    // the longest run of them, plus one, change nothing
+    fl.K = 1;
+    if ((NT1 - 1 + R - 1) / R > FW_KFIX) {
+        for (unsigned long long m = __ballot(!first); m; m &= m << 1) fl.K++;
+        int k2 = 1;
+        for (unsigned long long m = __ballot(!last); m; m &= m << 1) k2++;
+        fl.K = max(fl.K, k2);
     }
 }
 
@@ -117,7 +267,7 @@ __device__ __forceinline__ void vrow_load(const DevInst &d, int v, double (&ev)[
     constexpr int RW = 64 * R;
     const AW_GLOBAL double *row = gp(d.vemit) + (size_t)max(min(v, d.nvar - 1), 0) * RW;
 #pragma unroll
-    for (int r = 0; r < R; r++) ev[r] = row[r * 64 + threadIdx.x];
+    for (int r = 0; r < R; r++) ev[r] = row[r * 64 + (threadIdx.x & 63)];
 }
 
 // 1 / x: FP32 tables use the hardware reciprocal (within 1 ulp; the
@@ -145,15 +295,25 @@ constexpr int fw_vch()
     return (32 / R) < 2 ? 2 : (32 / R) > fw_vst<Real, R>() ? fw_vst<Real, R>() : (32 / R);
 }
 
-// LDS of the forward kernel, in Reals: partial sums, the previous column in
-// state order, the switch targets (plus one dummy slot per lane), staged
-// variant rows, the (a,b) table
+// The column handed over: lane l's R values in one run, runs an odd number of
+// 16-byte pieces apart (the pieces sixteen lanes access are in distinct banks)
 template <class Real, int R>
-constexpr int fw_lds_reals()
+constexpr int xc_stride()
 {
-    return 32 * GCOPY * (int)(sizeof(double) / sizeof(Real)) + 64 * R + (64 * R + 64) +
-           fw_vst<Real, R>() * 64 * R + 31 * 32;
+    return ((R * (int)sizeof(Real) + 15) / 16 | 1) * 16 / (int)sizeof(Real);
 }
+
+// LDS of the forward kernel: partial sums, the column handed over, the terms
+// handed back, the switch targets (plus one dummy slot per lane), staged
+// variant rows
+template <class Real, int R>
+struct FwShared {
+    alignas(16) double gp[32 * GCOPY];
+    alignas(16) Real xc[64 * xc_stride<Real, R>()];
+    alignas(16) Real tv[64];       // the other-branch term of each time bin; [32] the scale, [33] rejoined
+    alignas(16) Real nw[64 * R + 64];
+    alignas(16) Real vs[fw_vst<Real, R>() * 64 * R];
+};
 
 // wave-wide maximum
 __device__ __forceinline__ double wave_max(double x)
@@ -165,48 +325,186 @@ __device__ __forceinline__ double wave_max(double x)
 // columns between the checks of a re-run tile against its stored columns
 constexpr int FW_RECHECK = 128;
 
-template <class Real, int R, int NT1>
-__device__ __forceinline__ void fw_instance(const DevInst d, Real *sm, const FwTile tile,
-                                            AW_GLOBAL Real *bnd, AW_GLOBAL double *bnorm,
-                                            double tol, AW_GLOBAL int *early)
+// The two waves of a tile walk its columns together, two barriers a column:
+// after the first the column is in sh.xc, after the second its terms are in
+// sh.tv.
+//
+// REDO: a re-run tile (mode 2).  It stops once a column it computes agrees
+// with the column stored by its speculative run (relative tolerance tol): the
+// filter is contractive, so the stored columns after it, the normalisers and
+// the boundary column stay within tolerance.  early receives the column after
+// that one, or 0.
+struct FwSpan {
+    int c0, cs, c1, mode, bout, bin;
+    int clast;   // the last column computed: c1 - 1, or c1 into the boundary slot
+};
+
+// The ends and switch sources of 64 blocks from b0 on, one block per lane,
+// read with readlane: scalar loads at a switch would be waited for with the
+// next LDS access.
+struct FwBlocks {
+    int b0, last, rs, rc;
+    __device__ __forceinline__ FwBlocks(const DevInst &d, int b) { load(d, b); }
+    __device__ __forceinline__ void load(const DevInst &d, int b)
+    {
+        b0 = b;
+        const int x = min(b + (int)(threadIdx.x & 63), d.B - 1);
+        last = gp(d.bstart)[x] + gp(d.blen)[x];
+        rs = gp(d.srcs)[2 * x];
+        rc = gp(d.srcs)[2 * x + 1];
+    }
+    // block b follows the one before in the window, or opens the next window
+    __device__ __forceinline__ void next(const DevInst &d, int b)
+    {
+        if (b >= b0 + 64) load(d, b);
+    }
+    __device__ __forceinline__ int end(int b) const { return __builtin_amdgcn_readlane(last, b - b0); }
+    __device__ __forceinline__ int recomb(int b) const { return __builtin_amdgcn_readlane(rs, b - b0); }
+    __device__ __forceinline__ int recoal(int b) const { return __builtin_amdgcn_readlane(rc, b - b0); }
+};
+
+template <class Real, int R, int NT1, bool REDO>
+__device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh, const FwSpan &sp,
+                                        AW_GLOBAL Real *bnd, AW_GLOBAL double *bnorm, double tol,
+                                        AW_GLOBAL int *early)
 {
-    constexpr int RW = 64 * R;
-    constexpr int VST = fw_vst<Real, R>();
-    constexpr int VCH = fw_vch<Real, R>();
-    const int lane = threadIdx.x;
-    const int T1 = d.T - 1, L = d.L;
-    // carry steps: a branch has at most T-1 states, so it reaches back at
-    // most ceil((T-2)/R) lanes from the lane holding its last state
-    const int K = (T1 - 1 + R - 1) / R;
-    double *GP = (double *)sm;       // 32 x GCOPY: per-time partial sums
-    // byte offset of this lane's copy within a time bin's GCOPY copies
-    const int gslot = (lane / (64 / GCOPY)) * (int)sizeof(double);
-    // the half of bin lane>>1 that this lane reduces, and its read rotation
-    double *gq = GP + (lane >> 1) * GCOPY + (lane & 1) * (GCOPY / 2);
-    const int grot = (lane >> 1) & (GCOPY / 2 - 1);
-    Real *XS = (Real *)(GP + 32 * GCOPY);   // RW: previous column in state order (switch)
-    Real *NW = XS + RW;              // RW + 64: switch targets, then a dummy slot per lane
-    Real *VS = NW + RW + 64;         // VST rows: staged variant-column emissions
-    Real *TMS = VS + VST * RW;       // 31 x 32: the (a,b) table (FP64)
+    constexpr int RW = 64 * R, NJ = (NT1 + 2) / 4 * 2, XC = xc_stride<Real, R>();
+    const int lane = threadIdx.x & 63, T1 = d.T - 1, L = d.L;
     AW_GLOBAL Real *alpha = (AW_GLOBAL Real *)d.alpha;
     auto norms = gp(d.norms);
-
-    const int c0 = tile.c0, cs = tile.cs;
-    // the last column computed: c1 - 1, or c1 into the boundary slot
-    const int clast = tile.bout >= 0 ? tile.c1 : tile.c1 - 1;
-    FwLane<Real, R, NT1> fl;
-    int b = find_owner(cp(d.bstart), d.B, c0);
-    int bend = cp(d.bstart)[b] + cp(d.blen)[b];
-    fw_load_block<Real, R, NT1>(d, b, fl, TMS);
+    // this lane's half of the copies of the bin it reduces (the other half is
+    // the lane's of the other row), in four pieces from the (lane / 4)-th on:
+    // the pieces that a row reads in one step lie in distinct banks
+    double2 *gq = (double2 *)(sh.gp + bin_of(lane >> 4, lane & 15) * GCOPY +
+                              (((lane >> 4) ^ (lane >> 1)) & 1) * (GCOPY / 2));
+    const int rot = lane >> 2;
+    // Of a block: the addresses of the states' bins and copies in the sums,
+    // and the lane's part of the (a,b) table.  Indices are clamped: entries
+    // a >= T-1 meet a zero sum, and lanes >= T-1 compute terms nobody uses,
+    // but for lanes 31 and 63, whose entries of 1 give the normaliser.  The
+    // next block's are loaded a block ahead.
+    AW_LDS double *gadd[R];
+    Real tmc[NJ];
+    int ni[R];
+    double nt[NJ];
+    auto load = [&](int b) {
+        const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
+        const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * T1 * T1 + min(lane & 31, T1 - 1);
 #pragma unroll
-    for (int k = 0; k < 32 * GCOPY / 64; k++) GP[k * 64 + lane] = 0.0;
+        for (int r = 0; r < R; r++) ni[r] = info[r * 64 + lane];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) nt[j] = tm[min(bin_of(lane >> 4, j), T1 - 1) * T1];
+    };
+    auto unpack = [&] {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            gadd[r] = (AW_LDS double *)sh.gp + (ni[r] & INFO_TIME) * GCOPY + (lane & (GCOPY - 1));
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; j++) tmc[j] = (lane & 31) == 31 ? Real(1) : (Real)nt[j];
+    };
+    int b = find_owner(cp(d.bstart), d.B, sp.c0);
+    FwBlocks bl(d, b);
+    int bend = bl.end(b);
+    load(b);
+    for (int k = lane; k < 32 * GCOPY; k += 64) sh.gp[k] = 0.0;
+    unpack();
+    load(min(b + 1, d.B - 1));
+    Real nw = Real(0);   // lane i: the normaliser of the column with col % 64 == i
+    bool rejoined = false;
+    int col = sp.c0;
+    // the normalisers of the columns up to col of col's window of 64
+    auto flush = [&] {
+        const int c = (col & ~63) + lane;
+        if (c >= sp.cs && c <= min(col, sp.c1 - 1)) norms[c] = (double)nw;
+    };
+    for (;; col++) {
+        fw_barrier();
+        Real x[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) x[r] = sh.xc[lane * XC + r];
+#pragma unroll
+        for (int r = 0; r < R; r++) (void)__builtin_amdgcn_ds_atomic_fadd_f64(gadd[r], (double)x[r]);
+        // the LDS operations of one wave run in order: the sums are complete
+        // when they are read, and cleared before the next column's
+        double2 q[GCOPY / 4];
+#pragma unroll
+        for (int k = 0; k < GCOPY / 4; k++) q[k] = gq[(k + rot) & 3];
+        const Real g = (Real)add_rows(((q[0].x + q[0].y) + (q[1].x + q[1].y)) +
+                                      ((q[2].x + q[2].y) + (q[3].x + q[3].y)));
+        Real a0 = Real(0), a1 = Real(0);
+        bin_product(g, tmc, a0, a1);
+        const Real t = add_halves(a0 + a1);
+        const Real norm = readlane_r(t, 31);
+        // column 0 is stored unnormalised (scale 1); a restarted tile's first
+        // column is the boundary column as stored by the tile before
+        const bool asis = col == sp.c0 && (col == 0 || (REDO && sp.mode == 2));
+        const Real nsc = asis ? Real(1) : recip(norm);
+        // the terms of the time bins, 0 for the padding's, and the scale
+        Real tv = (lane < T1) ? t * nsc : Real(0);
+        tv = lane == 32 ? nsc : tv;
+        if (REDO) {
+            if (col > sp.c0 && col < sp.c1 && (col - sp.c0) % FW_RECHECK == 0) {
+                const AW_GLOBAL Real *row = alpha + (size_t)col * RW;
+                double dmax = 0.0, amax = 0.0;
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const double nv = (double)(x[r] * nsc), ov = (double)row[r * 64 + lane];
+                    dmax = fmax(dmax, fabs(nv - ov));
+                    amax = fmax(amax, fabs(nv));
+                }
+                rejoined = wave_max(dmax) <= tol * wave_max(amax);
+            }
+            tv = (lane == 33 && rejoined) ? Real(1) : tv;
+        }
+        sh.tv[lane] = tv;
+        fw_barrier();
+#pragma unroll
+        for (int k = 0; k < GCOPY / 4; k++) gq[(k + rot) & 3] = double2{0.0, 0.0};
+        if (col >= sp.cs) {
+            AW_GLOBAL Real *row = col < sp.c1 ? alpha + (size_t)col * RW
+                                              : bnd + (size_t)sp.bout * BND_STRIDE;
+#pragma unroll
+            for (int r = 0; r < R; r++) row[r * 64 + lane] = x[r] * nsc;
+        }
+        nw = (lane == (col & 63)) ? norm : nw;
+        if ((col & 63) == 63 || col == sp.clast || (REDO && rejoined)) flush();
+        if (col == sp.clast || (REDO && rejoined)) break;
+        if (col + 1 == bend) {
+            bl.next(d, ++b);
+            bend = bl.end(b);
+            unpack();
+            load(min(b + 1, d.B - 1));
+        }
+    }
+    if (sp.bout >= 0 && !rejoined && lane == (col & 63)) bnorm[sp.bout] = (double)nw;
+    // the first column's own normaliser
+    if (sp.c0 >= sp.cs && sp.c0 < sp.c1 && lane == 0) {
+        if (sp.c0 == 0 && L > 1) norms[0] = 1.0;
+        if (REDO && sp.mode == 2) norms[sp.c0] = bnorm[sp.bin];
+    }
+    if (REDO && early && lane == 0) *early = rejoined ? col + 1 : 0;
+}
+
+template <class Real, int R, int NT1, bool REDO>
+__device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh, const FwSpan &sp,
+                                         const AW_GLOBAL Real *bnd)
+{
+    constexpr int RW = 64 * R, XC = xc_stride<Real, R>();
+    constexpr int VST = fw_vst<Real, R>(), VCH = fw_vch<Real, R>();
+    const int lane = threadIdx.x & 63, L = d.L;
+    int b = find_owner(cp(d.bstart), d.B, sp.c0);
+    FwBlocks bl(d, b);
+    int bend = bl.end(b);
+    FwLane<Real, R> fl;
+    FwRaw<Real, R> raw;
+    fw_load_raw<Real, R>(d, b, raw);
+    fw_unpack<Real, R, NT1>(raw, sh.tv, fl);
+    for (int k = lane; k < RW; k += 64) sh.nw[k] = Real(0);
     // Column classes of a window of 64 columns, one per lane, read with
-    // readlane; the next window's are loaded a window ahead.  vmcnt counts
-    // the table stores too, so any wait on a load inside the column loop
-    // would also wait for the stores of the column before: the windows are
-    // an outer loop, and the one wait per window is taken there.
+    // readlane; the next window's are loaded a window ahead.
     const AW_GLOBAL int *clsg = gp(d.cls);
-    int wb = c0 & ~63;
+    int wb = sp.c0 & ~63;
     int clsv = clsg[min(wb + lane, L - 1)];
     int clsn = clsg[min(wb + 64 + lane, L - 1)];
     // Variant rows (row index = the column's class) are consumed in order
@@ -214,239 +512,161 @@ __device__ __forceinline__ void fw_instance(const DevInst d, Real *sm, const FwT
     // and the columns read their row from LDS.
     int vbase = 0, vend = 0;
 
-    Real x[R], tfs[R], v[R];
-    Real sc = Real(1);   // the previous column is x * sc
-
-    // A re-run tile (mode 2) stops once a column it computes agrees with
-    // the column stored by its speculative run (relative tolerance tol):
-    // the filter is contractive, so the stored columns after it, the
-    // normalisers and the boundary column stay within tolerance.
-    bool rejoined = false;
-
-    // per-time sums, normaliser, stored row, other-branch term of the next
-    // column
-    auto finish = [&](int col, bool first) {
-#pragma unroll
-        for (int r = 0; r < R; r++)
-            lds_add((double *)((char *)GP + fl.boff[r] * (2 * GCOPY) + gslot), (double)v[r]);
-        // lane l takes the copies of bin l>>1 in its half (l&1), leaving 0
-        // (one exchange each; the LDS operations of one wave run in order).
-        // Step k reads copy (k + l/2) mod 8 of the half: the lanes of one
-        // step then spread over the banks (copy k of every bin would sit in
-        // two banks), which also fixes each lane's summation order
-        double q[GCOPY / 2];
-#pragma unroll
-        for (int k = 0; k < GCOPY / 2; k++)
-            q[k] = __longlong_as_double((long long)__hip_atomic_exchange(
-                (unsigned long long *)(gq + ((k + grot) & (GCOPY / 2 - 1))), 0ull,
-                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-#pragma unroll
-        for (int w = 1; w < GCOPY / 2; w *= 2)
-#pragma unroll
-            for (int k = 0; k < GCOPY / 2; k += 2 * w) q[k] += q[k + w];
-        const Real g = (Real)(q[0] + dpp_r<DPP_QUAD_SWAP1>(q[0]));   // lanes 2a, 2a+1: G[a]
-        // four interleaved partial sums keep the dependency chains short
-        Real nq[4] = {Real(0), Real(0), Real(0), Real(0)};
-        Real tq[4] = {Real(0), Real(0), Real(0), Real(0)};
-#pragma unroll
-        for (int a = 0; a < NT1; a++) {
-            const Real ga = readlane_r(g, 2 * a);
-            nq[a & 3] += ga;
-            tq[a & 3] += ga * (tm_in_lds<Real>() ? TMS[a * 32 + (lane & 31)] : fl.tmc[a]);
-        }
-        const Real norm = (nq[0] + nq[1]) + (nq[2] + nq[3]);
-        const Real t = (tq[0] + tq[1]) + (tq[2] + tq[3]);
-        // column 0 is stored unnormalised (scale 1); a restarted tile's first
-        // column is the boundary column as stored by the tile before
-        const Real nsc = (col == 0 || (first && tile.mode == 2)) ? Real(1) : recip(norm);
-        if (col >= cs && col < tile.c1) {
-            AW_GLOBAL Real *row = alpha + (size_t)col * RW;
-            if (tile.mode == 2 && !first && (col - tile.c0) % FW_RECHECK == 0) {
-                double dmax = 0.0, amax = 0.0;
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const double nv = (double)(v[r] * nsc), ov = (double)row[r * 64 + lane];
-                    dmax = fmax(dmax, fabs(nv - ov));
-                    amax = fmax(amax, fabs(nv));
-                }
-                dmax = wave_max(dmax);
-                amax = wave_max(amax);
-                rejoined = dmax <= tol * amax;
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) row[r * 64 + lane] = v[r] * nsc;
-            if (lane == 0) {
-                double nv = (col == 0) ? ((L == 1) ? (double)norm : 1.0) : (double)norm;
-                if (first && tile.mode == 2) nv = bnorm[tile.bin];
-                norms[col] = nv;
-            }
-        } else if (col == tile.c1) {
-            AW_GLOBAL Real *row = bnd + (size_t)tile.bout * BND_STRIDE;
-#pragma unroll
-            for (int r = 0; r < R; r++) row[r * 64 + lane] = v[r] * nsc;
-            if (lane == 0) bnorm[tile.bout] = (double)norm;
-        }
-        // TF[b] lives in lane b; lanes >= T-1 (padding bin 31) hold 0
-        const Real tv = (lane < T1) ? t * nsc : Real(0);
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            tfs[r] = bperm_r(tv, fl.boff[r]);
-            x[r] = v[r];
-        }
-        sc = nsc;
-    };
-
     // first column.  mode 0: the unnormalised prior, not multiplied by the
     // emission (calc_state_priors, trans.cpp:785-831); padding positions
     // hold 0.  mode 1: 1 on every state.  mode 2: the boundary column.
-    if (tile.mode == 0) {
+    Real v[R];
+    if (sp.mode == 0) {
         const AW_GLOBAL double *pr = gp(d.lprior);
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = (Real)pr[r * 64 + lane];
-    } else if (tile.mode == 1) {
+    } else if (sp.mode == 1) {
         const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = (lane * R + r < S) ? Real(1) : Real(0);
     } else {
-        const AW_GLOBAL Real *src = bnd + (size_t)tile.bin * BND_STRIDE;
+        const AW_GLOBAL Real *src = bnd + (size_t)sp.bin * BND_STRIDE;
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = src[r * 64 + lane];
     }
-    finish(c0, true);
 
-    // an empty asm reading the register makes the compiler complete its
-    // load here rather than at a use inside the column loop
-    asm volatile("" : "+v"(clsv));
-    int col = c0 + 1;
-    while (col <= clast && !rejoined) {
-        if (col >= wb + 64) {
+    for (int col = sp.c0;; col++) {
+#pragma unroll
+        for (int r = 0; r < R; r++) sh.xc[lane * XC + r] = v[r];
+        fw_barrier();
+        // What follows until the second barrier runs beside the sums wave: the
+        // empty asms keep the compiler from moving it before the first barrier
+        // or behind the second.
+#pragma unroll
+        for (int r = 0; r < R; r++) asm volatile("" : "+v"(v[r]));
+        // the next column's class (past the last column: a repeat, unused),
+        // emission, and same-branch terms or switch
+        const int next = col + 1;
+        if (next >= wb + 64) {
             wb += 64;
             clsv = clsn;
-            asm volatile("" : "+v"(clsv));
             clsn = clsg[min(wb + 64 + lane, L - 1)];
         }
-        const int wend = min(wb + 63, clast);
-    for (; col <= wend; col++) {
-        const int cls = __builtin_amdgcn_readlane(clsv, col & 63);
-        const bool var = cls >= 0;
-        Real ev[R];
-        if (var) {
+        const int cls = __builtin_amdgcn_readlane(clsv, next & 63);
+        const bool sw = next == bend && next < L;
+        Real e[R], same[R];
+        Real prs = Real(0), pcs = Real(0);
+        if (sw) {
+            // switch column: deterministic transitions scattered into nw
+            // (the recombination and recoalescence sources excluded); the two
+            // dense rows follow below
+            bl.next(d, ++b);
+            bend = bl.end(b);
+            const int rs = bl.recomb(b), rc = bl.recoal(b);
+            // (loading these a block ahead gains nothing measurable)
+            fw_load_raw<Real, R>(d, b, raw);
+            if (rs != -1) prs = sh.xc[(rs / R) * XC + rs % R];
+            if (rc != -1) pcs = sh.xc[(rc / R) * XC + rc % R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const Real x = v[r] * raw.dp[r];
+                // atomics (192 cycles over a full wave in FP32) only where
+                // several sources meet
+                const bool shared = raw.dt[r] >= DET_SHARED;
+                sh.nw[raw.dt[r] < 0 || shared ? RW + lane : raw.dt[r]] = x;
+                if (shared) lds_add(&sh.nw[raw.dt[r] & ~DET_SHARED], x);
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                same[r] = sh.nw[lane * R + r];
+                sh.nw[lane * R + r] = Real(0);   // for the next switch
+            }
+            fw_unpack<Real, R, NT1>(raw, sh.tv, fl);
+        } else {
+            // same-branch prefix sums (younger states) with the carry from the
+            // lanes before, suffix sums (older states) with the carry from the
+            // lanes after
+            Real P[R], Q[R];
+            Real p = Real(0), q = Real(0);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int t = R - 1 - r;
+                P[r] = keep(p, fl.nf[r]);
+                Q[t] = keep(q, fl.nl[t]);
+                p = fma(fl.cf[r], v[r], P[r]);
+                q = fma(fl.cd[t], v[t], Q[t]);
+            }
+            Real y1 = p, y2 = q;
+            constexpr int KMAX = (NT1 - 1 + R - 1) / R, KB = KMAX <= FW_KFIX ? KMAX - 1 : 4;
+            if constexpr (KB > 0)
+                for (int k = 1; k < (KMAX <= FW_KFIX ? 2 : fl.K); k += KB)
+                    carry_steps<KB>(p, q, fl.m1, fl.m2, y1, y2);
+            // the wait covers the chains' last registers, which the compiler
+            // does not know to be fresh
+            asm("s_nop 1" : "+v"(y1), "+v"(y2));
+            y1 = dpp_r<DPP_WAVE_SHR1>(y1);
+            y2 = dpp_r<DPP_WAVE_SHL1>(y2);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const Real pr = add_kept(P[r], y1, fl.ff[r]), qr = add_kept(Q[r], y2, fl.fl[r]);
+                // the last slot of a lane adds its two products in the other
+                // order in FP32
+                const Real two = (sizeof(Real) == 8 || r < R - 1) ? fma(fl.cg[r], pr, fl.ck[r] * qr)
+                                                                  : fma(fl.ck[r], qr, fl.cg[r] * pr);
+                same[r] = fma(fl.cj[r], v[r], two);
+            }
+        }
+        if (cls >= 0) {
             if (cls >= vend) {
                 vbase = cls;
                 vend = min(cls + VST, d.nvar);
 #pragma unroll
                 for (int k0 = 0; k0 < VST; k0 += VCH) {
                     // VST need not be a multiple of VCH
-                    double buf[VCH][R];
+                    double rows[VCH][R];
 #pragma unroll
                     for (int k = 0; k < VCH; k++)
-                        if (k0 + k < VST) vrow_load<R>(d, vbase + k0 + k, buf[k]);
+                        if (k0 + k < VST) vrow_load<R>(d, vbase + k0 + k, rows[k]);
 #pragma unroll
                     for (int k = 0; k < VCH; k++)
 #pragma unroll
                         for (int r = 0; r < R; r++)
-                            if (k0 + k < VST) VS[(k0 + k) * RW + r * 64 + lane] = (Real)buf[k][r];
+                            if (k0 + k < VST) sh.vs[(k0 + k) * RW + r * 64 + lane] = (Real)rows[k][r];
                 }
             }
 #pragma unroll
-            for (int r = 0; r < R; r++) ev[r] = VS[(cls - vbase) * RW + r * 64 + lane];
-        }
-
-        if (col == bend) {
-            // switch column: deterministic transitions scattered into NW
-            // (the recombination and recoalescence sources excluded), then
-            // the two dense rows.  Every load of the column is issued before
-            // the first use, branch-free, so the column waits once.
-            const int nb = b + 1;
-            const int so0 = cp(d.soff)[b], so1 = cp(d.soff)[nb];
-            const int S1 = so1 - so0, S2 = cp(d.soff)[nb + 1] - so1;
-            const int rs = cp(d.srcs)[2 * nb], cs = cp(d.srcs)[2 * nb + 1];
-            const AW_GLOBAL Real *swn = planes<Real>(d, nb, RW);
-            const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)nb * RW;
-            int dt[R];
-            Real dpv[R], rr[R], cr[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int x = r * 64 + lane;
-                dt[r] = detn[x];
-                dpv[r] = swn[CDP * RW + x];
-                rr[r] = swn[CRR * RW + x];
-                cr[r] = swn[CCR * RW + x];
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                XS[lane * R + r] = x[r];   // padding slots (s >= S1) are never read
-                NW[r * 64 + lane] = Real(0);
-            }
-            b = nb;
-            bend += cp(d.blen)[nb];
-            fw_load_block<Real, R, NT1>(d, b, fl, TMS);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int s = lane * R + r;
-                const bool ok = s < S1 && dt[r] >= 0 && s != rs && s != cs;
-                lds_add(&NW[ok ? dt[r] : RW + lane], ok ? x[r] * dpv[r] : Real(0));
-            }
-            const Real prs = (rs != -1) ? XS[max(rs, 0)] * sc : Real(0);
-            const Real pcs = (cs != -1) ? XS[max(cs, 0)] * sc : Real(0);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int s = lane * R + r;
-                const Real e = var ? ev[r] : (cls == -1) ? fl.ce[r] : Real(1);
-                Real acc = (s < S2) ? NW[s] * sc : Real(0);
-                if (rs != -1 && rr[r] > Real(0)) acc += prs * rr[r];
-                if (cs != -1 && cr[r] > Real(0)) acc += pcs * cr[r];
-                v[r] = (s < S2) ? acc * e : Real(0);
-            }
+            for (int r = 0; r < R; r++) e[r] = sh.vs[(cls - vbase) * RW + r * 64 + lane];
         } else {
-            // same-branch prefix sums (younger states) with the carry from
-            // the lanes before, suffix sums (older states) with the carry
-            // from the lanes after
-            Real P[R], Q[R];
-            Real p = Real(0);
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                P[r] = keep(p, fl.nf[r]);
-                p = fl.cf[r] * x[r] + P[r];
-            }
-            Real q = Real(0);
-#pragma unroll
-            for (int r = R - 1; r >= 0; r--) {
-                Q[r] = keep(q, fl.nl[r]);
-                q = fl.cd[r] * x[r] + Q[r];
-            }
-            Real c1 = Real(0), c2 = Real(0);
-            for (int k = 0; k < K; k++) {
-                c1 = dpp_r<DPP_WAVE_SHR1>(fl.m1 * c1 + p);
-                c2 = dpp_r<DPP_WAVE_SHL1>(fl.m2 * c2 + q);
-            }
-            // the carry reaches the slots before the lane's first branch
-            // start (prefix) / after its last branch end (suffix)
-            Real f1 = Real(1);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                f1 = keep(f1, fl.nf[r]);
-                P[r] += c1 * f1;
-            }
-            Real f2 = Real(1);
-#pragma unroll
-            for (int r = R - 1; r >= 0; r--) {
-                f2 = keep(f2, fl.nl[r]);
-                Q[r] += c2 * f2;
-            }
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const Real e = var ? ev[r] : (cls == -1) ? fl.ce[r] : Real(1);
-                const Real same = (fl.cg[r] * P[r] + fl.ck[r] * Q[r]) + fl.cj[r] * x[r];
-                v[r] = e * (tfs[r] + sc * same);
-            }
+            for (int r = 0; r < R; r++) e[r] = cls == -1 ? fl.ce[r] : Real(1);
         }
-        finish(col, false);
-        if (rejoined) break;
+#pragma unroll
+        for (int r = 0; r < R; r++) asm volatile("" : "+v"(same[r]), "+v"(e[r]));
+        fw_barrier();
+        if (col == sp.clast || (REDO && (col - sp.c0) % FW_RECHECK == 0 && sh.tv[33] != Real(0))) return;
+        const Real sc = sh.tv[32];
+        if (sw) {
+            // the recombination and recoalescence rows; padding slots hold 0 in
+            // every row
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                v[r] = fma(pcs * sc, raw.cr[r], fma(prs * sc, raw.rr[r], same[r] * sc)) * e[r];
+        } else {
+            Real tf[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) tf[r] = *fl.tf[r];
+#pragma unroll
+            for (int r = 0; r < R; r++) v[r] = e[r] * fma(sc, same[r], tf[r]);
+        }
     }
-    }
-    // the column after the one that rejoined (never 0), else 0
-    if (early && lane == 0) *early = rejoined ? col + 1 : 0;
+}
+
+template <class Real, int R, int NT1, bool REDO>
+__device__ __forceinline__ void fw_instance(const DevInst d, void *lds, const FwTile &t,
+                                            AW_GLOBAL Real *bnd, AW_GLOBAL double *bnorm,
+                                            double tol, AW_GLOBAL int *early)
+{
+    FwShared<Real, R> &sh = *(FwShared<Real, R> *)lds;
+    auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    FwSpan sp{uni(t.c0), uni(t.cs), uni(t.c1), uni(t.mode), uni(t.bout), uni(t.bin), 0};
+    sp.clast = sp.bout >= 0 ? sp.c1 : sp.c1 - 1;
+    if (uni((int)threadIdx.x >> 6)) fw_sums<Real, R, NT1, REDO>(d, sh, sp, bnd, bnorm, tol, early);
+    else fw_lanes<Real, R, NT1, REDO>(d, sh, sp, bnd);
 }
 
 // One launch covers every instance of a batch, whatever its states-per-lane
@@ -458,30 +678,28 @@ __device__ __forceinline__ void fw_instance(const DevInst d, Real *sm, const FwT
 // their own, launched over the same tiles, so that their register demand
 // (spilled to AGPRs and scratch) does not weigh on the others.
 template <class Real, int NT1, bool REDO, bool BIG>
-__global__ __launch_bounds__(64) void k_fw_all(const DevInst *__restrict__ D,
-                                               const FwTile *__restrict__ tiles,
-                                               Real *__restrict__ bnd, double *__restrict__ bnorm,
-                                               double tol, int *__restrict__ early)
+__global__ __launch_bounds__(FW_THREADS)
+void k_fw_all(const DevInst *__restrict__ D, const FwTile *__restrict__ tiles,
+              Real *__restrict__ bnd, double *__restrict__ bnorm, double tol, int *__restrict__ early)
 {
     extern __shared__ __align__(16) double fw_dyn[];
     const FwTile t = tiles[blockIdx.x];
     const DevInst &d = D[t.inst];
-    Real *sm = (Real *)fw_dyn;
     AW_GLOBAL Real *bg = (AW_GLOBAL Real *)bnd;
     AW_GLOBAL double *ng = (AW_GLOBAL double *)bnorm;
     AW_GLOBAL int *eg = early ? (AW_GLOBAL int *)(early + blockIdx.x) : nullptr;
     if ((d.R > 16) != BIG) return;   // the other symbol's tile
     if constexpr (BIG) {
-        fw_instance<Real, 32, NT1>(d, sm, t, bg, ng, tol, eg);
+        fw_instance<Real, 32, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg);
     } else {
         switch (d.R) {
-        case 1: fw_instance<Real, 1, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 2: fw_instance<Real, 2, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 4: fw_instance<Real, 4, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 6: fw_instance<Real, 6, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 8: fw_instance<Real, 8, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        case 12: fw_instance<Real, 12, NT1>(d, sm, t, bg, ng, tol, eg); break;
-        default: fw_instance<Real, 16, NT1>(d, sm, t, bg, ng, tol, eg); break;
+        case 1: fw_instance<Real, 1, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        case 2: fw_instance<Real, 2, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        case 4: fw_instance<Real, 4, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        case 6: fw_instance<Real, 6, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        case 8: fw_instance<Real, 8, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        case 12: fw_instance<Real, 12, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
+        default: fw_instance<Real, 16, NT1, REDO>(d, fw_dyn, t, bg, ng, tol, eg); break;
         }
     }
 }
@@ -527,7 +745,8 @@ int launch_fw(const DevInst *dD, const FwTile *tiles, int cnt, void *bnd, double
     if constexpr (sizeof(Real) == 4)
         if (early) kern = (T1max <= 19) ? k_fw_all<Real, 19, true, BIG> : k_fw_all<Real, MAXT - 1, true, BIG>;
     if (set_lds_limit((const void *)kern, sh)) return 1;
-    hipLaunchKernelGGL(kern, dim3(cnt), dim3(64), sh, st, dD, tiles, (Real *)bnd, bnorm, tol, early);
+    hipLaunchKernelGGL(kern, dim3(cnt), dim3(FW_THREADS), sh, st, dD, tiles,
+                       (Real *)bnd, bnorm, tol, early);
     HIP_OK(hipGetLastError());
     return 0;
 }

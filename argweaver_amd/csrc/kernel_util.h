@@ -31,6 +31,8 @@ __device__ inline AW_GLOBAL X *gp(X *p)
     return (AW_GLOBAL X *)p;
 }
 
+#define AW_LDS __attribute__((address_space(3)))
+
 // Read-only data indexed by wave-uniform values (block bounds, uniforms)
 // goes through the constant address space so it is fetched with scalar loads.
 #define AW_CONST __attribute__((address_space(4)))
@@ -70,7 +72,7 @@ constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114,
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int x)
 {
-    return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false);
+    return __builtin_amdgcn_mov_dpp(x, CTRL, 0xf, 0xf, true);
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_r(float x)

@@ -322,7 +322,7 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int s = lane * R + r;
-            const int dt = detn[r * 64 + lane];
+            const int dt = detn[r * 64 + lane] & ~DET_SHARED;   // -1 stays no state
             const Real dp = cn[CDP * RW + r * 64 + lane];
             tr[r] = (s == cs) ? crk : (s == rs) ? rrk : (dt == k ? dp : Real(0));
         }
@@ -529,19 +529,22 @@ __global__ __launch_bounds__(64 * tb_waves<BIG>()) void k_tb_rerun(const DevInst
     else TB_FOR_R(d.R, (tb_rerun<Real, R, NW>(d, ch, k, rs, tb_dyn)))
 }
 
-// Predicted sources: for every state k of block b the state j of block b-1
-// with the largest switch probability P(j -> k) (ties: the larger index),
-// TB_NONE where no state leads to k.  One workgroup per block; the
-// candidates (deterministic targets, then the two dense rows) meet in LDS.
+// Tables of the switch into a block b.  Predicted sources: for every state k
+// of block b the state j of block b-1 with the largest switch probability
+// P(j -> k) (ties: the larger index), TB_NONE where no state leads to k.
+// Deterministic targets in ldet: marked where they have several sources, and -1
+// for the states that the dense rows take.  One workgroup per block; the candidates (deterministic targets,
+// then the two dense rows) meet in LDS.
 __global__ __launch_bounds__(256) void k_tb_pred(const DevInst *__restrict__ D,
                                                  const int *__restrict__ blkoff, int ninst)
 {
-    extern __shared__ unsigned long long best[];
+    extern __shared__ unsigned long long best[];   // RW keys, then RW counts
     const int inst = find_owner(blkoff, ninst, (int)blockIdx.x);
     const DevInst &d = D[inst];
     const int b = blockIdx.x - blkoff[inst];
     if (b == 0) return;
     const int R = d.R, RW = 64 * R;
+    int *count = (int *)(best + RW);
     const int S1 = cp(d.soff)[b] - cp(d.soff)[b - 1], S2 = cp(d.soff)[b + 1] - cp(d.soff)[b];
     const int rs = cp(d.srcs)[2 * b], cs = cp(d.srcs)[2 * b + 1];
     auto weight = [&](int plane, int p) -> float {
@@ -551,14 +554,29 @@ __global__ __launch_bounds__(256) void k_tb_pred(const DevInst *__restrict__ D,
     auto key = [](float w, int j) {
         return (unsigned long long)__float_as_uint(w) << 32 | (unsigned)(j + 1);
     };
-    for (int x = threadIdx.x; x < RW; x += 256) best[x] = 0;
-    __syncthreads();
-    for (int p = threadIdx.x; p < RW; p += 256) {
-        const int j = (p & 63) * R + (p >> 6);
-        const int t = gp(d.ldet)[(size_t)b * RW + p];
-        if (j < S1 && t >= 0 && t < S2 && j != rs && j != cs) atomicMax(&best[t], key(weight(CDP, p), j));
+    auto det = gp(d.ldet) + (size_t)b * RW;
+    for (int x = threadIdx.x; x < RW; x += 256) {
+        best[x] = 0;
+        count[x] = 0;
     }
     __syncthreads();
+    auto source = [&](int p, int t) {   // a deterministic transition into t
+        const int j = (p & 63) * R + (p >> 6);
+        return j < S1 && t >= 0 && t < S2 && j != rs && j != cs;
+    };
+    for (int p = threadIdx.x; p < RW; p += 256) {
+        const int t = det[p];
+        if (source(p, t)) {
+            atomicMax(&best[t], key(weight(CDP, p), (p & 63) * R + (p >> 6)));
+            atomicAdd(&count[t], 1);
+        }
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < RW; p += 256) {
+        const int t = det[p];
+        if (!source(p, t)) det[p] = -1;
+        else if (count[t] > 1) det[p] = t | DET_SHARED;
+    }
     auto out = gp(d.pred) + (size_t)b * RW;
     for (int p = threadIdx.x; p < RW; p += 256) {
         const int k = (p & 63) * R + (p >> 6);
@@ -594,7 +612,8 @@ size_t tb_lds_bytes(int R)
 
 int launch_tb_pred(const DevInst *D, const int *blkoff, int ninst, int nblk, int Rmax, hipStream_t s)
 {
-    return launch(k_tb_pred, nblk, 256, sizeof(unsigned long long) * 64 * Rmax, s, D, blkoff, ninst);
+    return launch(k_tb_pred, nblk, 256, (sizeof(unsigned long long) + sizeof(int)) * 64 * Rmax, s, D,
+                  blkoff, ninst);
 }
 
 int launch_tb_spec(bool fp32, bool big, const DevInst *D, const Chunk *chunks, const int *list,
