@@ -133,8 +133,8 @@ struct HostInstance {
     int last_state = -1;
 };
 
-// Schedule of a batch run.  The forward runs one wave per instance over
-// all of its columns, or, in FP32, one wave per forward tile (checked
+// Schedule of a batch run.  The forward runs one workgroup per instance over
+// all of its columns, or, in FP32, one per forward tile (checked
 // speculative starts); the traceback runs one workgroup per column tile.
 struct BatchOptions {
     Precision prec = Precision::FP64;

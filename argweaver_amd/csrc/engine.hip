@@ -1680,7 +1680,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     if (launch_tb_pred(m.dD, m.d_blkoff, n, blkoff[n], rmax, s)) return 1;
     (void)hipEventRecord(c.ev[3], s);
 
-    // forward: one wave per tile, all tiles in one launch, the longest
+    // forward: one workgroup per tile, all tiles in one launch, the longest
     // instances first
     std::vector<int> order(n);
     std::iota(order.begin(), order.end(), 0);

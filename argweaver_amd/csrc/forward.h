@@ -7,7 +7,7 @@
 
 namespace aw {
 
-// A forward tile: columns [c0, c1) of an instance computed by one wave.
+// A forward tile: columns [c0, c1) of an instance computed by one workgroup.
 // mode 0 starts from the prior at column 0.  mode 1 starts at c0 from a
 // uniform vector and stores nothing before cs (a warm-up: the filter
 // forgets its start).  mode 2 starts at c0 from the column held in boundary

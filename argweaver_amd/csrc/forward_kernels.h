@@ -10,7 +10,7 @@
 namespace aw {
 
 //===========================================================================
-// forward recursion, one wave per instance (arghmm_forward_alg,
+// forward recursion, two waves per tile (arghmm_forward_alg,
 // sample_thread.cpp:394-460; arghmm_forward_block :186-296;
 // arghmm_forward_switch :345-389)
 
@@ -34,10 +34,12 @@ namespace aw {
 // atomics from several waves meeting in LDS than they gained.
 //
 // us per column at R = 1 / 2 / 4 / 6 / 8 / 12 / 16 states per lane, one
-// instance on MI355X, switches included: FP32 0.44 0.41 0.39 0.45 0.52 0.59
-// 0.83 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
-// 0.99 1.24 1.82); FP64 0.52 0.46 0.43 0.47 0.53 0.84 1.62 (1.15 0.95 1.05
-// 1.12 1.30 1.67 2.74).
+// instance on MI355X, switches included: FP32 0.30 0.32 0.36 0.40 0.46 0.55
+// 0.78 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
+// 0.99 1.24 1.82); FP64 0.36 0.36 0.38 0.43 0.48 0.64 2.1 (1.15 0.95 1.05
+// 1.12 1.30 1.67 2.74).  Both waves run the columns between two events (block
+// ends, variant columns, windows of 64) in a loop of their own: with the tests
+// for events in every column it was 0.44 0.41 0.39 0.45 0.52 0.59 0.83.
 constexpr int FW_THREADS = 128;
 
 // Per block, each lane of the lanes wave keeps in registers the factor planes
@@ -47,23 +49,16 @@ constexpr int FW_THREADS = 128;
 // and whether the lane holds a branch start / end (the carry stops there), and
 // the state's time; padding states use time bin 31, whose term is 0, so they
 // come out 0 with no mask.  The 0/1 factors have the table's type, so that
-// applying one is one instruction; in FP64 with more than 12 states per lane
+// applying one is one instruction; in FP64 with more than 8 states per lane
 // they are floats applied as selects, for their registers.
 template <class Real, int R>
 struct FwLane {
     Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R];
-    using Fac = std::conditional_t<(sizeof(Real) * R <= 96), Real, float>;
+    using Fac = std::conditional_t<(sizeof(Real) * R <= 64), Real, float>;
     Fac nf[R], nl[R], ff[R], fl[R];
     const AW_LDS Real *tf[R];   // the handed-back term of the state's time
     Real m1, m2;
     int K;           // carry steps: lanes a branch of the block spans
-};
-
-// What the lanes wave loads of a block: its planes, and the switch into it
-template <class Real, int R>
-struct FwRaw {
-    Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R], rr[R], cr[R], dp[R];
-    int info[R], dt[R];
 };
 
 // x times a 0/1 factor m, and acc + x * m: a product where the factor has the
@@ -196,53 +191,48 @@ __device__ __forceinline__ void fw_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Loaded values go straight into their registers: selecting or copying a
-// value whose load is still in flight makes the compiler wait for it at once.
+// plane `which` of block b, one value per slot.  Loaded values go straight into
+// their registers: selecting or copying a value whose load is still in flight
+// makes the compiler wait for it at once.
 template <class Real, int R>
-__device__ __forceinline__ void fw_load_raw(const DevInst &d, int b, FwRaw<Real, R> &x)
+__device__ __forceinline__ void fw_plane(const DevInst &d, int b, int which, Real (&x)[R])
 {
-    constexpr int RW = 64 * R;
-    // uniform bases, per-lane index: loads use the scalar-base address form
-    const AW_GLOBAL Real *coef = planes<Real>(d, b, RW);
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
-    const AW_GLOBAL int *det = gp(d.ldet) + (size_t)b * RW;
+    // uniform base, per-lane index: loads use the scalar-base address form
+    const AW_GLOBAL Real *p = planes<Real>(d, b, 64 * R) + which * (64 * R);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int i = r * 64 + (threadIdx.x & 63);
-        x.info[r] = info[i];
-        x.dt[r] = det[i];
-        x.cf[r] = coef[CF * RW + i];
-        x.cd[r] = coef[CD * RW + i];
-        x.cg[r] = coef[CG * RW + i];
-        x.ck[r] = coef[CK * RW + i];
-        x.cj[r] = coef[CJ * RW + i];
-        x.ce[r] = coef[CE * RW + i];
-        x.rr[r] = coef[CRR * RW + i];
-        x.cr[r] = coef[CCR * RW + i];
-        x.dp[r] = coef[CDP * RW + i];
-    }
+    for (int r = 0; r < R; r++) x[r] = p[r * 64 + (threadIdx.x & 63)];
+}
+template <int R>
+__device__ __forceinline__ void fw_row(const int *rows, int b, int (&x)[R])
+{
+    const AW_GLOBAL int *p = gp(rows) + (size_t)b * (64 * R);
+#pragma unroll
+    for (int r = 0; r < R; r++) x[r] = p[r * 64 + (threadIdx.x & 63)];
 }
 
+// Block b in the lanes wave; tv: the handed-back terms
 template <class Real, int R, int NT1>
-__device__ __forceinline__ void fw_unpack(const FwRaw<Real, R> &x, const Real *tv, FwLane<Real, R> &fl)
+__device__ __forceinline__ void fw_block(const DevInst &d, int b, const Real *tv, FwLane<Real, R> &fl)
 {
+    int info[R];
+    fw_row<R>(d.linfo, b, info);
+    fw_plane<Real, R>(d, b, CF, fl.cf);
+    fw_plane<Real, R>(d, b, CD, fl.cd);
+    fw_plane<Real, R>(d, b, CG, fl.cg);
+    fw_plane<Real, R>(d, b, CK, fl.ck);
+    fw_plane<Real, R>(d, b, CJ, fl.cj);
+    fw_plane<Real, R>(d, b, CE, fl.ce);
     bool first = false, last = false;
     using Fac = typename FwLane<Real, R>::Fac;
     Fac f1 = 1, f2 = 1;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        fl.cf[r] = x.cf[r];
-        fl.cd[r] = x.cd[r];
-        fl.cg[r] = x.cg[r];
-        fl.ck[r] = x.ck[r];
-        fl.cj[r] = x.cj[r];
-        fl.ce[r] = x.ce[r];
-        fl.nf[r] = (x.info[r] & INFO_FIRST) ? Fac(0) : Fac(1);
-        fl.nl[r] = (x.info[r] & INFO_LAST) ? Fac(0) : Fac(1);
+        fl.nf[r] = (info[r] & INFO_FIRST) ? Fac(0) : Fac(1);
+        fl.nl[r] = (info[r] & INFO_LAST) ? Fac(0) : Fac(1);
         fl.ff[r] = f1 *= fl.nf[r];
-        fl.tf[r] = (const AW_LDS Real *)tv + (x.info[r] & INFO_TIME);
-        first |= (x.info[r] & INFO_FIRST) != 0;
-        last |= (x.info[r] & INFO_LAST) != 0;
+        fl.tf[r] = (const AW_LDS Real *)tv + (info[r] & INFO_TIME);
+        first |= (info[r] & INFO_FIRST) != 0;
+        last |= (info[r] & INFO_LAST) != 0;
     }
 #pragma unroll
     for (int r = R - 1; r >= 0; r--) fl.fl[r] = f2 *= fl.nl[r];
@@ -413,64 +403,74 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
     Real nw = Real(0);   // lane i: the normaliser of the column with col % 64 == i
     bool rejoined = false;
     int col = sp.c0;
-    // the normalisers of the columns up to col of col's window of 64
-    auto flush = [&] {
-        const int c = (col & ~63) + lane;
-        if (c >= sp.cs && c <= min(col, sp.c1 - 1)) norms[c] = (double)nw;
-    };
-    for (;; col++) {
-        fw_barrier();
-        Real x[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) x[r] = sh.xc[lane * XC + r];
-#pragma unroll
-        for (int r = 0; r < R; r++) (void)__builtin_amdgcn_ds_atomic_fadd_f64(gadd[r], (double)x[r]);
-        // the LDS operations of one wave run in order: the sums are complete
-        // when they are read, and cleared before the next column's
-        double2 q[GCOPY / 4];
-#pragma unroll
-        for (int k = 0; k < GCOPY / 4; k++) q[k] = gq[(k + rot) & 3];
-        const Real g = (Real)add_rows(((q[0].x + q[0].y) + (q[1].x + q[1].y)) +
-                                      ((q[2].x + q[2].y) + (q[3].x + q[3].y)));
-        Real a0 = Real(0), a1 = Real(0);
-        bin_product(g, tmc, a0, a1);
-        const Real t = add_halves(a0 + a1);
-        const Real norm = readlane_r(t, 31);
+    // Columns run in stretches without an event: the first column by itself
+    // (its scale), then up to the block's end, the end of a window of 64
+    // (normalisers stored), the end of the warm-up, the tile's last column,
+    // and the boundary column by itself.
+    for (bool done = false; !done;) {
+        int ev = min(min(bend - 1, col | 63), sp.clast);
+        if (col < sp.c1) ev = min(ev, sp.c1 - 1);
+        const bool store = col >= sp.cs;
+        if (!store) ev = min(ev, sp.cs - 1);
         // column 0 is stored unnormalised (scale 1); a restarted tile's first
         // column is the boundary column as stored by the tile before
         const bool asis = col == sp.c0 && (col == 0 || (REDO && sp.mode == 2));
-        const Real nsc = asis ? Real(1) : recip(norm);
-        // the terms of the time bins, 0 for the padding's, and the scale
-        Real tv = (lane < T1) ? t * nsc : Real(0);
-        tv = lane == 32 ? nsc : tv;
-        if (REDO) {
-            if (col > sp.c0 && col < sp.c1 && (col - sp.c0) % FW_RECHECK == 0) {
-                const AW_GLOBAL Real *row = alpha + (size_t)col * RW;
-                double dmax = 0.0, amax = 0.0;
+        if (col == sp.c0) ev = col;
+        AW_GLOBAL Real *row = (col < sp.c1 ? alpha + (size_t)col * RW
+                                           : bnd + (size_t)sp.bout * BND_STRIDE) + lane;
+        for (;; col++, row += RW) {
+            fw_barrier();
+            Real x[R];
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const double nv = (double)(x[r] * nsc), ov = (double)row[r * 64 + lane];
-                    dmax = fmax(dmax, fabs(nv - ov));
-                    amax = fmax(amax, fabs(nv));
+            for (int r = 0; r < R; r++) x[r] = sh.xc[lane * XC + r];
+#pragma unroll
+            for (int r = 0; r < R; r++) (void)__builtin_amdgcn_ds_atomic_fadd_f64(gadd[r], (double)x[r]);
+            // the LDS operations of one wave run in order: the sums are
+            // complete when they are read, and cleared before the next column's
+            double2 q[GCOPY / 4];
+#pragma unroll
+            for (int k = 0; k < GCOPY / 4; k++) q[k] = gq[(k + rot) & 3];
+#pragma unroll
+            for (int k = 0; k < GCOPY / 4; k++) gq[(k + rot) & 3] = double2{0.0, 0.0};
+            const Real g = (Real)add_rows(((q[0].x + q[0].y) + (q[1].x + q[1].y)) +
+                                          ((q[2].x + q[2].y) + (q[3].x + q[3].y)));
+            Real a0 = Real(0), a1 = Real(0);
+            bin_product(g, tmc, a0, a1);
+            const Real t = add_halves(a0 + a1);
+            const Real norm = readlane_r(t, 31);
+            const Real nsc = asis ? Real(1) : recip(norm);
+            // the terms of the time bins, 0 for the padding's, and the scale
+            Real tv = (lane < T1) ? t * nsc : Real(0);
+            tv = lane == 32 ? nsc : tv;
+            if (REDO) {
+                if (col > sp.c0 && col < sp.c1 && (col - sp.c0) % FW_RECHECK == 0) {
+                    double dmax = 0.0, amax = 0.0;
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const double nv = (double)(x[r] * nsc), ov = (double)row[r * 64];
+                        dmax = fmax(dmax, fabs(nv - ov));
+                        amax = fmax(amax, fabs(nv));
+                    }
+                    rejoined = wave_max(dmax) <= tol * wave_max(amax);
                 }
-                rejoined = wave_max(dmax) <= tol * wave_max(amax);
+                tv = (lane == 33 && rejoined) ? Real(1) : tv;
             }
-            tv = (lane == 33 && rejoined) ? Real(1) : tv;
-        }
-        sh.tv[lane] = tv;
-        fw_barrier();
+            sh.tv[lane] = tv;
+            fw_barrier();
+            if (store) {
 #pragma unroll
-        for (int k = 0; k < GCOPY / 4; k++) gq[(k + rot) & 3] = double2{0.0, 0.0};
-        if (col >= sp.cs) {
-            AW_GLOBAL Real *row = col < sp.c1 ? alpha + (size_t)col * RW
-                                              : bnd + (size_t)sp.bout * BND_STRIDE;
-#pragma unroll
-            for (int r = 0; r < R; r++) row[r * 64 + lane] = x[r] * nsc;
+                for (int r = 0; r < R; r++) row[r * 64] = x[r] * nsc;
+            }
+            nw = (lane == (col & 63)) ? norm : nw;
+            if (col == ev || (REDO && rejoined)) break;
         }
-        nw = (lane == (col & 63)) ? norm : nw;
-        if ((col & 63) == 63 || col == sp.clast || (REDO && rejoined)) flush();
-        if (col == sp.clast || (REDO && rejoined)) break;
-        if (col + 1 == bend) {
+        done = col == sp.clast || (REDO && rejoined);
+        if ((col & 63) == 63 || done) {
+            const int c = (col & ~63) + lane;
+            if (c >= sp.cs && c <= min(col, sp.c1 - 1)) norms[c] = (double)nw;
+        }
+        if (done) break;
+        if (++col == bend) {
             bl.next(d, ++b);
             bend = bl.end(b);
             unpack();
@@ -492,14 +492,15 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
 {
     constexpr int RW = 64 * R, XC = xc_stride<Real, R>();
     constexpr int VST = fw_vst<Real, R>(), VCH = fw_vch<Real, R>();
+    // registers allow a loop of its own for plain columns, and a switch's loads
+    // all at once
+    constexpr bool TWICE = R * sizeof(Real) <= 96;
     const int lane = threadIdx.x & 63, L = d.L;
     int b = find_owner(cp(d.bstart), d.B, sp.c0);
     FwBlocks bl(d, b);
     int bend = bl.end(b);
     FwLane<Real, R> fl;
-    FwRaw<Real, R> raw;
-    fw_load_raw<Real, R>(d, b, raw);
-    fw_unpack<Real, R, NT1>(raw, sh.tv, fl);
+    fw_block<Real, R, NT1>(d, b, sh.tv, fl);
     for (int k = lane; k < RW; k += 64) sh.nw[k] = Real(0);
     // Column classes of a window of 64 columns, one per lane, read with
     // readlane; the next window's are loaded a window ahead.
@@ -530,15 +531,81 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
         for (int r = 0; r < R; r++) v[r] = src[r * 64 + lane];
     }
 
-    for (int col = sp.c0;; col++) {
+    // the column goes to the sums wave
+    auto publish = [&] {
 #pragma unroll
         for (int r = 0; r < R; r++) sh.xc[lane * XC + r] = v[r];
         fw_barrier();
-        // What follows until the second barrier runs beside the sums wave: the
+        // What follows until the second barrier runs beside the sums wave:
         // empty asms keep the compiler from moving it before the first barrier
         // or behind the second.
 #pragma unroll
         for (int r = 0; r < R; r++) asm volatile("" : "+v"(v[r]));
+    };
+    // same-branch prefix sums (younger states) with the carry from the lanes
+    // before, suffix sums (older states) with the carry from the lanes after
+    auto scan = [&](Real (&same)[R]) {
+        Real P[R], Q[R];
+        Real p = Real(0), q = Real(0);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int t = R - 1 - r;
+            P[r] = keep(p, fl.nf[r]);
+            Q[t] = keep(q, fl.nl[t]);
+            p = fma(fl.cf[r], v[r], P[r]);
+            q = fma(fl.cd[t], v[t], Q[t]);
+        }
+        Real y1 = p, y2 = q;
+        constexpr int KMAX = (NT1 - 1 + R - 1) / R, KB = KMAX <= FW_KFIX ? KMAX - 1 : 4;
+        if constexpr (KB > 0)
+            for (int k = 1; k < (KMAX <= FW_KFIX ? 2 : fl.K); k += KB)
+                carry_steps<KB>(p, q, fl.m1, fl.m2, y1, y2);
+        // the wait covers the chains' last registers, which the compiler does
+        // not know to be fresh
+        asm("s_nop 1" : "+v"(y1), "+v"(y2));
+        y1 = dpp_r<DPP_WAVE_SHR1>(y1);
+        y2 = dpp_r<DPP_WAVE_SHL1>(y2);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const Real pr = add_kept(P[r], y1, fl.ff[r]), qr = add_kept(Q[r], y2, fl.fl[r]);
+            // the last slot of a lane adds its two products in the other order
+            // in FP32
+            const Real two = (sizeof(Real) == 8 || r < R - 1) ? fma(fl.cg[r], pr, fl.ck[r] * qr)
+                                                              : fma(fl.ck[r], qr, fl.cg[r] * pr);
+            same[r] = fma(fl.cj[r], v[r], two);
+            if (TWICE) asm volatile("" : "+v"(same[r]));
+        }
+    };
+    // whether the walk ends at column col
+    auto ends = [&](int col) {
+        return col == sp.clast || (REDO && (col - sp.c0) % FW_RECHECK == 0 && sh.tv[33] != Real(0));
+    };
+    // invariant columns without a switch: the columns before `plain`
+    auto plain_to = [&](int next) {
+        const unsigned long long m = __ballot(clsv != -1) >> (next & 63);
+        const int n = m ? next + (int)__ffsll((long long)m) - 1 : wb + 64;
+        return min(min(n, bend), sp.clast + 1);
+    };
+
+    for (int col = sp.c0;;) {
+        // Every column goes from here to the next one, in this loop while that
+        // is a plain one (not where a second copy of the scan would spill).
+        int plain = 0;
+        if (TWICE && col + 1 < wb + 64) plain = plain_to(col + 1);
+        for (; col + 1 < plain; col++) {
+            publish();
+            Real same[R];
+            scan(same);
+            fw_barrier();
+            if (REDO && ends(col)) return;
+            const Real sc = sh.tv[32];
+            Real tf[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) tf[r] = *fl.tf[r];
+#pragma unroll
+            for (int r = 0; r < R; r++) v[r] = fl.ce[r] * fma(sc, same[r], tf[r]);
+        }
+        publish();
         // the next column's class (past the last column: a repeat, unused),
         // emission, and same-branch terms or switch
         const int next = col + 1;
@@ -549,7 +616,7 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
         }
         const int cls = __builtin_amdgcn_readlane(clsv, next & 63);
         const bool sw = next == bend && next < L;
-        Real e[R], same[R];
+        Real e[R], same[R], rr[R], cr[R];
         Real prs = Real(0), pcs = Real(0);
         if (sw) {
             // switch column: deterministic transitions scattered into nw
@@ -558,58 +625,35 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
             bl.next(d, ++b);
             bend = bl.end(b);
             const int rs = bl.recomb(b), rc = bl.recoal(b);
-            // (loading these a block ahead gains nothing measurable)
-            fw_load_raw<Real, R>(d, b, raw);
+            // (loading the block's data a block ahead gains nothing measurable)
+            int dt[R];
+            Real dp[R];
+            fw_row<R>(d.ldet, b, dt);
+            fw_plane<Real, R>(d, b, CDP, dp);
+            if (TWICE) {
+                fw_plane<Real, R>(d, b, CRR, rr);
+                fw_plane<Real, R>(d, b, CCR, cr);
+                fw_block<Real, R, NT1>(d, b, sh.tv, fl);
+            }
             if (rs != -1) prs = sh.xc[(rs / R) * XC + rs % R];
             if (rc != -1) pcs = sh.xc[(rc / R) * XC + rc % R];
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                const Real x = v[r] * raw.dp[r];
+                const Real x = v[r] * dp[r];
                 // atomics (192 cycles over a full wave in FP32) only where
                 // several sources meet
-                const bool shared = raw.dt[r] >= DET_SHARED;
-                sh.nw[raw.dt[r] < 0 || shared ? RW + lane : raw.dt[r]] = x;
-                if (shared) lds_add(&sh.nw[raw.dt[r] & ~DET_SHARED], x);
+                const bool shared = dt[r] >= DET_SHARED;
+                sh.nw[dt[r] < 0 || shared ? RW + lane : dt[r]] = x;
+                if (shared) lds_add(&sh.nw[dt[r] & ~DET_SHARED], x);
             }
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 same[r] = sh.nw[lane * R + r];
                 sh.nw[lane * R + r] = Real(0);   // for the next switch
             }
-            fw_unpack<Real, R, NT1>(raw, sh.tv, fl);
+            if (!TWICE) fw_block<Real, R, NT1>(d, b, sh.tv, fl);
         } else {
-            // same-branch prefix sums (younger states) with the carry from the
-            // lanes before, suffix sums (older states) with the carry from the
-            // lanes after
-            Real P[R], Q[R];
-            Real p = Real(0), q = Real(0);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const int t = R - 1 - r;
-                P[r] = keep(p, fl.nf[r]);
-                Q[t] = keep(q, fl.nl[t]);
-                p = fma(fl.cf[r], v[r], P[r]);
-                q = fma(fl.cd[t], v[t], Q[t]);
-            }
-            Real y1 = p, y2 = q;
-            constexpr int KMAX = (NT1 - 1 + R - 1) / R, KB = KMAX <= FW_KFIX ? KMAX - 1 : 4;
-            if constexpr (KB > 0)
-                for (int k = 1; k < (KMAX <= FW_KFIX ? 2 : fl.K); k += KB)
-                    carry_steps<KB>(p, q, fl.m1, fl.m2, y1, y2);
-            // the wait covers the chains' last registers, which the compiler
-            // does not know to be fresh
-            asm("s_nop 1" : "+v"(y1), "+v"(y2));
-            y1 = dpp_r<DPP_WAVE_SHR1>(y1);
-            y2 = dpp_r<DPP_WAVE_SHL1>(y2);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const Real pr = add_kept(P[r], y1, fl.ff[r]), qr = add_kept(Q[r], y2, fl.fl[r]);
-                // the last slot of a lane adds its two products in the other
-                // order in FP32
-                const Real two = (sizeof(Real) == 8 || r < R - 1) ? fma(fl.cg[r], pr, fl.ck[r] * qr)
-                                                                  : fma(fl.ck[r], qr, fl.cg[r] * pr);
-                same[r] = fma(fl.cj[r], v[r], two);
-            }
+            scan(same);
         }
         if (cls >= 0) {
             if (cls >= vend) {
@@ -638,14 +682,18 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
 #pragma unroll
         for (int r = 0; r < R; r++) asm volatile("" : "+v"(same[r]), "+v"(e[r]));
         fw_barrier();
-        if (col == sp.clast || (REDO && (col - sp.c0) % FW_RECHECK == 0 && sh.tv[33] != Real(0))) return;
+        if (ends(col)) return;
         const Real sc = sh.tv[32];
         if (sw) {
             // the recombination and recoalescence rows; padding slots hold 0 in
             // every row
+            if (!TWICE) {
+                fw_plane<Real, R>(d, b, CRR, rr);
+                fw_plane<Real, R>(d, b, CCR, cr);
+            }
 #pragma unroll
             for (int r = 0; r < R; r++)
-                v[r] = fma(pcs * sc, raw.cr[r], fma(prs * sc, raw.rr[r], same[r] * sc)) * e[r];
+                v[r] = fma(pcs * sc, cr[r], fma(prs * sc, rr[r], same[r] * sc)) * e[r];
         } else {
             Real tf[R];
 #pragma unroll
@@ -653,6 +701,7 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
 #pragma unroll
             for (int r = 0; r < R; r++) v[r] = e[r] * fma(sc, same[r], tf[r]);
         }
+        col++;
     }
 }
 

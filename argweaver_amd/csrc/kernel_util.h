@@ -42,12 +42,6 @@ __device__ inline AW_CONST const X *cp(const X *p)
     return (AW_CONST const X *)p;
 }
 
-// LDS operations of one wave are performed in order, so inside a
-// single-wave workgroup only the compiler's order matters; every LDS access
-// of a kernel goes through one dynamic shared array, so accesses that may
-// overlap are never reordered.  This marks the places that rely on it.
-__device__ inline void lds_order() {}
-
 // index i such that off[i] <= x < off[i+1]
 template <class PT, class X>
 __device__ inline int find_owner(PT off, int n, X x)
@@ -94,23 +88,6 @@ __device__ __forceinline__ double readlane_d(double x, int l)
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)v, l);
     const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// inclusive prefix sum over the 64 lanes: Hillis-Steele inside each 16-lane
-// row, then the totals of the rows before
-__device__ __forceinline__ double wave_incl_scan(double v)
-{
-    v += dpp_r<DPP_ROW_SHR1>(v);
-    v += dpp_r<DPP_ROW_SHR2>(v);
-    v += dpp_r<DPP_ROW_SHR4>(v);
-    v += dpp_r<DPP_ROW_SHR8>(v);
-    const double t0 = readlane_d(v, 15), t1 = readlane_d(v, 31), t2 = readlane_d(v, 47);
-    const int row = threadIdx.x >> 4;
-    double off = 0.0;
-    if (row >= 1) off = t0;
-    if (row >= 2) off += t1;
-    if (row >= 3) off += t2;
-    return v + off;
 }
 
 
