@@ -773,6 +773,25 @@ std::recursive_mutex &device_mutex()
 }
 #define DEVICE_LOCK std::lock_guard<std::recursive_mutex> device_lock_(device_mutex())
 
+//===========================================================================
+// table rows for the host: columns [c0, c0 + n) of a lane-run table, `pitch`
+// states each, in state order and FP64, one wave per column.  `out` is pinned
+// host memory, which the stores reach over the link in whole lines (a lane's
+// states lie apart in the row instead, whose second reader finds it in cache);
+// the host then copies rows of S states.  Copying the padded rows out and
+// picking the states on the host took 18 ms of a call's 23 (20011 columns, 19
+// haplotypes, FP32); this way the call takes 11.7 ms.
+template <class Real>
+__global__ __launch_bounds__(256) void k_rows_out(const void *alpha, int c0, int n, int R, int pitch,
+                                                  double *__restrict__ out)
+{
+    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (c >= n) return;
+    const Real *row = (const Real *)alpha + (size_t)(c0 + c) * (64 * R);
+    double *o = out + (size_t)c * pitch;
+    for (int s = threadIdx.x & 63; s < pitch; s += 64) o[s] = (double)row[lane_pos(s, R)];
+}
+
 // The batch's streams: main carries every stage; side carries only the
 // traceback of the instances whose forward is final (their chains and
 // re-runs, driven by a helper host thread) while the forward
@@ -887,6 +906,30 @@ int set_lds_limit(const void *kern, size_t sh)
     return 0;
 }
 
+// Pinned host memory in two halves that table rows pass through on their way
+// out, taken when the first table is copied out (a workspace batch: with its
+// streams).
+struct HostStage {
+    static constexpr size_t HALF = size_t(2) << 20;   // bytes; a row has at most 16 KB
+    char *p = nullptr;
+    hipEvent_t filled[2];
+    int ensure()
+    {
+        if (p) return 0;
+        for (auto &e : filled) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIP_OK(hipHostMalloc((void **)&p, 2 * HALF, hipHostMallocDefault));
+        return 0;
+    }
+    double *half(int k) const { return reinterpret_cast<double *>(p + k * HALF); }
+    void release()
+    {
+        if (!p) return;
+        for (auto &e : filled) (void)hipEventDestroy(e);
+        (void)hipHostFree(p);
+        p = nullptr;
+    }
+};
+
 struct Batch::Impl {
     std::vector<HostInstance> hosts;
     std::vector<std::vector<double>> us, priors;
@@ -902,6 +945,7 @@ struct Batch::Impl {
     Arena arena;   // base == nullptr: buffers come from hipMalloc
     std::vector<std::vector<float>> staged32;   // FP32 planes of host-prepared instances
     Streams st;
+    HostStage stage;
     DevInst *dD = nullptr;
     long long *d_coloff = nullptr;
     int *d_blkoff = nullptr, *d_voff = nullptr, *d_nvar = nullptr, *d_list = nullptr;
@@ -927,6 +971,7 @@ struct Batch::Impl {
     ~Impl()
     {
         st.destroy();
+        stage.release();
         in.release();
         work.release();
         tab.release();
@@ -961,7 +1006,8 @@ void Batch::use_workspace(void *base, size_t cap)
 int Batch::init_streams()
 {
     if (ctx_init()) return 1;
-    return impl_->st.create();
+    if (impl_->st.create()) return 1;
+    return impl_->arena.base ? impl_->stage.ensure() : 0;
 }
 
 void Batch::clear()
@@ -1803,65 +1849,51 @@ int Batch::copy_norms(int i, double *norms) const
 }
 
 // block-major view (block b holds blocklen_b rows of S_b states, the
-// reference's table layout) of the lane-run table
-int Batch::copy_alpha(int i, double *alpha) const
+// reference's table layout) of columns [c0, c1) of the lane-run table.  While
+// the kernel fills one half of the staging memory, the host copies the rows of
+// the other half out.
+int Batch::copy_alpha_range(int i, int c0, int c1, double *alpha) const
 {
     BATCH_LOCK;
-    const Impl &m = *impl_;
+    Impl &m = *impl_;
     const DevInst &d = m.h[i];
     const FlatTrees &ft = m.hosts[i].ft;
-    const int R = d.R, RW = 64 * R;
-    const size_t cells = (size_t)d.L * RW;
-    std::vector<double> tab(cells);
-    if (m.prec_done == Precision::FP64) {
-        HIP_OK(hipMemcpy(tab.data(), d.alpha, sizeof(double) * cells, hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float> t32(cells);
-        HIP_OK(hipMemcpy(t32.data(), d.alpha, sizeof(float) * cells, hipMemcpyDeviceToHost));
-        for (size_t x = 0; x < cells; x++) tab[x] = t32[x];
-    }
-    std::vector<int> pos;
-    long long o = 0;
-    for (int b = 0; b < ft.nblocks; b++) {
-        const int S = m.Sv[i][b];
-        pos.resize(S);
-        for (int k = 0; k < S; k++) pos[k] = lane_pos(k, R);
-        for (int cc = 0; cc < ft.len[b]; cc++) {
-            const double *row = &tab[(size_t)(ft.start[b] + cc) * RW];
-            for (int k = 0; k < S; k++) alpha[o++] = row[pos[k]];
+    const std::vector<int> &Sv = m.Sv[i];
+    if (c0 < 0 || c1 > d.L || c0 >= c1) return 1;
+    const bool fp32 = m.prec_done == Precision::FP32;
+    // no table before a run, or only part of one after a run that failed
+    const size_t bytes = (size_t)d.L * 64 * d.R * (fp32 ? sizeof(float) : sizeof(double));
+    if (!d.alpha || (char *)d.alpha + bytes > m.tab.p + m.tab.cap) return 1;
+    if (m.stage.ensure()) return 1;
+    const int pitch = *std::max_element(Sv.begin(), Sv.end());
+    const int rows = (int)(HostStage::HALF / sizeof(double) / pitch);
+    const auto fill = [&](int c, int half) {
+        const int n = std::min(rows, c1 - c);
+        hipLaunchKernelGGL(fp32 ? k_rows_out<float> : k_rows_out<double>, dim3((n + 3) / 4),
+                           dim3(256), 0, m.st.main, d.alpha, c, n, d.R, pitch, m.stage.half(half));
+        HIP_OK(hipGetLastError());
+        HIP_OK(hipEventRecord(m.stage.filled[half], m.st.main));
+        return 0;
+    };
+    int b = 0;
+    if (fill(c0, 0)) return 1;
+    for (int c = c0, half = 0; c < c1; c += rows, half ^= 1) {
+        if (c + rows < c1 && fill(c + rows, half ^ 1)) return 1;
+        HIP_OK(hipEventSynchronize(m.stage.filled[half]));
+        const double *row = m.stage.half(half);
+        for (int x = c; x < std::min(c + rows, c1); x++, row += pitch) {
+            while (ft.start[b] + ft.len[b] <= x) b++;
+            memcpy(alpha, row, sizeof(double) * Sv[b]);
+            alpha += Sv[b];
         }
     }
     return 0;
 }
 
-int Batch::copy_alpha_range(int i, int c0, int c1, double *alpha) const
+int Batch::copy_alpha(int i, double *alpha) const
 {
     BATCH_LOCK;
-    const Impl &m = *impl_;
-    const DevInst &d = m.h[i];
-    const FlatTrees &ft = m.hosts[i].ft;
-    if (c0 < 0 || c1 > d.L || c0 >= c1) return 1;
-    const int R = d.R, RW = 64 * R;
-    const size_t cells = (size_t)(c1 - c0) * RW;
-    std::vector<double> tab(cells);
-    if (m.prec_done == Precision::FP64) {
-        HIP_OK(hipMemcpy(tab.data(), (const double *)d.alpha + (size_t)c0 * RW,
-                         sizeof(double) * cells, hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float> t32(cells);
-        HIP_OK(hipMemcpy(t32.data(), (const float *)d.alpha + (size_t)c0 * RW,
-                         sizeof(float) * cells, hipMemcpyDeviceToHost));
-        for (size_t x = 0; x < cells; x++) tab[x] = t32[x];
-    }
-    long long o = 0;
-    int b = 0;
-    for (int c = c0; c < c1; c++) {
-        while (ft.start[b] + ft.len[b] <= c) b++;
-        const int S = m.Sv[i][b];
-        const double *row = &tab[(size_t)(c - c0) * RW];
-        for (int k = 0; k < S; k++) alpha[o++] = row[lane_pos(k, R)];
-    }
-    return 0;
+    return copy_alpha_range(i, 0, impl_->h[i].L, alpha);
 }
 
 long long instance_states(const FlatTrees &ft, int T, std::vector<int> *Sv)

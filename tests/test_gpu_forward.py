@@ -42,3 +42,30 @@ def test_forward_tables(aw, k, L, T, c):
             got = got / got.sum(axis=1, keepdims=True)
             assert np.abs(got - ref / ref.sum(axis=1, keepdims=True)).max() <= 2e-4
     aw.delete_local_trees(tr)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_table_copied_in_pieces(aw, prec):
+    """Tables of several staging halves, and ranges of them from odd columns
+    on: every entry is the whole table's, which agrees with the oracle."""
+    k, L = 30, 5000
+    print("table copy prec=%d k=%d L=%d" % (prec, k, L), flush=True)
+    tr, seqs, inst, model = instance(aw, k, L, 5, ntimes=20, c=20)
+    nst = np.asarray(inst.nstates())
+    fw, _ = inst.forward()
+    assert fw.size > 3 * (2 << 20) // 8
+    b = aw.Batch()
+    b.add(tr, seqs, *model, k - 1, np.random.RandomState(L).uniform(size=L))
+    b.upload()
+    b.run(prec, 0)
+    whole = b.alpha(0)
+    for got, ref in zip(_columns(inst, whole), _columns(inst, fw)):
+        got = got / got.sum(axis=1, keepdims=True)
+        assert np.abs(got - ref / ref.sum(axis=1, keepdims=True)).max() <= (2e-4 if prec else 1e-12)
+    per_col = np.concatenate([[n] * (int(y - x) // int(n)) for n, x, y in
+                              zip(nst, inst.block_offsets(), inst.block_offsets()[1:])])
+    off = np.concatenate([[0], np.cumsum(per_col)])
+    for c0, c1 in ((0, 1), (L - 1, L), (1, L), (777, 2778), (1234, 1235)):
+        part = b.alpha_range(0, c0, c1, per_col)
+        assert np.array_equal(part, whole[off[c0]:off[c1]])
+    aw.delete_local_trees(tr)
