@@ -22,9 +22,10 @@ namespace aw {
 // per traceback tile); lane l owns the R consecutive states l*R .. l*R+R-1
 // of the node-major state order, so the states of one branch sit in one
 // lane or in neighbouring lanes.  Every per-state array is stored
-// transposed, position(s) = (s % R) * 64 + s / R, in rows of RW = 64*R
-// entries: slot r of all 64 lanes is one contiguous 64-entry segment, so
-// the loads and stores of a slot are coalesced.  R is fixed per instance
+// transposed (lane_pos) in rows of RW = 64*R entries: the slots of a lane are
+// taken in pieces of V = 4, 2 or 1, and a piece of all 64 lanes is one
+// contiguous segment of 64*V entries, so that loads and stores are coalesced
+// and a lane moves up to 16 bytes with each.  R is fixed per instance
 // (the smallest supported value with 64*R >= max states per block), so
 // forward-table rows have a constant stride and column col starts at
 // col * RW.
@@ -92,8 +93,19 @@ enum : int {
 // sets the targets of the two dense rows' sources to -1)
 enum : int { DET_SHARED = 1 << 30 };
 
-// transposed position of state s in a lane-run row
-__host__ __device__ inline int lane_pos(int s, int R) { return (s % R) * 64 + s / R; }
+// slots of a lane that lie side by side in a lane-run row
+__host__ __device__ constexpr int slot_vec(int R) { return R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1; }
+// position of slot r of a lane, of state s; the state at position p
+__host__ __device__ constexpr int slot_pos(int r, int lane, int R)
+{
+    return (r / slot_vec(R) * 64 + lane) * slot_vec(R) + r % slot_vec(R);
+}
+__host__ __device__ inline int lane_pos(int s, int R) { return slot_pos(s % R, s / R, R); }
+__host__ __device__ inline int pos_state(int p, int R)
+{
+    const int V = slot_vec(R), q = p / V;
+    return (q & 63) * R + (q >> 6) * V + p % V;
+}
 
 // offset of the (c, a, b) entry of the per-block same-branch table:
 // sum_{x<c} (T1-x)^2, in closed form

@@ -447,7 +447,7 @@ __global__ __launch_bounds__(256, 5) void k_prep_b(const DevInst *__restrict__ D
     // ct_b = exp(lnG4[b] + lnB[c-1]) (lnG4 = lnE2), so the branch-local
     // sum is a prefix sum (a < b) and a suffix sum (a > b) along the branch.
     for (int p = tid; p < RW; p += NT) {
-        const int s = (p & 63) * R + (p >> 6);
+        const int s = pos_state(p, R);
         double cf = 0, cd = 0, cg = 0, ck = 0, cj = 0, ce = 0, pr = 0;
         int inf = INFO_FIRST | INFO_LAST | 31;   // padding: time bin 31, whose TF is 0
         if (s < S) {
@@ -695,7 +695,7 @@ __global__ __launch_bounds__(64) void k_var_emit_b(const DevInst *__restrict__ D
     const int so = cp(d.soff)[b], S = cp(d.soff)[b + 1] - so;
     auto row = gp(d.vemit) + (size_t)v * RW;
     for (int p = lane; p < RW; p += 64) {
-        const int k = (p & 63) * R + (p >> 6);
+        const int k = pos_state(p, R);
         double e = 0.0;
         if (k < S) {
             int n = gp(d.snode)[so + k];

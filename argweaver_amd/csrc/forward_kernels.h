@@ -34,9 +34,9 @@ namespace aw {
 // atomics from several waves meeting in LDS than they gained.
 //
 // us per column at R = 1 / 2 / 4 / 6 / 8 / 12 / 16 states per lane, one
-// instance on MI355X, switches included: FP32 0.30 0.32 0.36 0.40 0.46 0.55
-// 0.78 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
-// 0.99 1.24 1.82); FP64 0.36 0.36 0.38 0.43 0.48 0.64 2.1 (1.15 0.95 1.05
+// instance on MI355X, switches included: FP32 0.30 0.31 0.35 0.40 0.45 0.53
+// 0.74 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
+// 0.99 1.24 1.82); FP64 0.36 0.35 0.38 0.42 0.46 0.64 2.1 (1.15 0.95 1.05
 // 1.12 1.30 1.67 2.74).  Both waves run the columns between two events (block
 // ends, variant columns, windows of 64) in a loop of their own: with the tests
 // for events in every column it was 0.44 0.41 0.39 0.45 0.52 0.59 0.83.
@@ -197,17 +197,12 @@ __device__ __forceinline__ void fw_barrier()
 template <class Real, int R>
 __device__ __forceinline__ void fw_plane(const DevInst &d, int b, int which, Real (&x)[R])
 {
-    // uniform base, per-lane index: loads use the scalar-base address form
-    const AW_GLOBAL Real *p = planes<Real>(d, b, 64 * R) + which * (64 * R);
-#pragma unroll
-    for (int r = 0; r < R; r++) x[r] = p[r * 64 + (threadIdx.x & 63)];
+    slots_load<R>(planes<Real>(d, b, 64 * R) + which * (64 * R), threadIdx.x & 63, x);
 }
 template <int R>
 __device__ __forceinline__ void fw_row(const int *rows, int b, int (&x)[R])
 {
-    const AW_GLOBAL int *p = gp(rows) + (size_t)b * (64 * R);
-#pragma unroll
-    for (int r = 0; r < R; r++) x[r] = p[r * 64 + (threadIdx.x & 63)];
+    slots_load<R>((const AW_GLOBAL int *)gp(rows) + (size_t)b * (64 * R), threadIdx.x & 63, x);
 }
 
 // Block b in the lanes wave; tv: the handed-back terms
@@ -256,8 +251,7 @@ __device__ __forceinline__ void vrow_load(const DevInst &d, int v, double (&ev)[
 {
     constexpr int RW = 64 * R;
     const AW_GLOBAL double *row = gp(d.vemit) + (size_t)max(min(v, d.nvar - 1), 0) * RW;
-#pragma unroll
-    for (int r = 0; r < R; r++) ev[r] = row[r * 64 + (threadIdx.x & 63)];
+    slots_load<R>(row, threadIdx.x & 63, ev);
 }
 
 // 1 / x: FP32 tables use the hardware reciprocal (within 1 ulp; the
@@ -327,6 +321,11 @@ constexpr int FW_RECHECK = 128;
 struct FwSpan {
     int c0, cs, c1, mode, bout, bin;
     int clast;   // the last column computed: c1 - 1, or c1 into the boundary slot
+    // the first column from col on that is checked against the stored one
+    __device__ __forceinline__ int recheck(int col) const
+    {
+        return c0 + (col - c0 + FW_RECHECK - 1) / FW_RECHECK * FW_RECHECK;
+    }
 };
 
 // The ends and switch sources of 64 blocks from b0 on, one block per lane,
@@ -377,15 +376,29 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
     Real tmc[NJ];
     int ni[R];
     double nt[NJ];
+    // The lanes wave loads all of a block at its switch and waits for it; a
+    // word of each 128-byte line of it, read here a block ahead, has the lines
+    // in cache by then (2 % of a column in FP32, nothing in FP64).
+    constexpr bool WARM = sizeof(Real) == 4;
+    constexpr int PB = NCOEF * RW * (int)sizeof(Real), NP = WARM ? (PB + 8191) / 8192 : 0;
+    unsigned warm[NP + 1];
     auto load = [&](int b) {
+        const AW_GLOBAL char *pl = (const AW_GLOBAL char *)planes<Real>(d, b, RW);
+        const AW_GLOBAL char *dt = (const AW_GLOBAL char *)(gp(d.ldet) + (size_t)b * RW);
+#pragma unroll
+        for (int x = 0; x < NP; x++)
+            warm[x] = *(const AW_GLOBAL unsigned *)(pl + min((x * 64 + lane) * 128, PB - 4));
+        if (WARM) warm[NP] = *(const AW_GLOBAL unsigned *)(dt + min(lane * 128, RW * 4 - 4));
         const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
         const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * T1 * T1 + min(lane & 31, T1 - 1);
-#pragma unroll
-        for (int r = 0; r < R; r++) ni[r] = info[r * 64 + lane];
+        slots_load<R>(info, lane, ni);
 #pragma unroll
         for (int j = 0; j < NJ; j++) nt[j] = tm[min(bin_of(lane >> 4, j), T1 - 1) * T1];
     };
     auto unpack = [&] {
+#pragma unroll
+        for (int x = 0; x <= NP; x++)
+            if (WARM) asm volatile("" ::"v"(warm[x]));
 #pragma unroll
         for (int r = 0; r < R; r++) {
             gadd[r] = (AW_LDS double *)sh.gp + (ni[r] & INFO_TIME) * GCOPY + (lane & (GCOPY - 1));
@@ -405,8 +418,8 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
     int col = sp.c0;
     // Columns run in stretches without an event: the first column by itself
     // (its scale), then up to the block's end, the end of a window of 64
-    // (normalisers stored), the end of the warm-up, the tile's last column,
-    // and the boundary column by itself.
+    // (normalisers stored), the end of the warm-up, a check against the stored
+    // columns, the tile's last column, and the boundary column by itself.
     for (bool done = false; !done;) {
         int ev = min(min(bend - 1, col | 63), sp.clast);
         if (col < sp.c1) ev = min(ev, sp.c1 - 1);
@@ -415,9 +428,11 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
         // column 0 is stored unnormalised (scale 1); a restarted tile's first
         // column is the boundary column as stored by the tile before
         const bool asis = col == sp.c0 && (col == 0 || (REDO && sp.mode == 2));
+        const int chk = REDO ? sp.recheck(col) : 0;
+        if (REDO) ev = min(ev, chk);
         if (col == sp.c0) ev = col;
-        AW_GLOBAL Real *row = (col < sp.c1 ? alpha + (size_t)col * RW
-                                           : bnd + (size_t)sp.bout * BND_STRIDE) + lane;
+        AW_GLOBAL Real *row = col < sp.c1 ? alpha + (size_t)col * RW
+                                           : bnd + (size_t)sp.bout * BND_STRIDE;
         for (;; col++, row += RW) {
             fw_barrier();
             Real x[R];
@@ -443,26 +458,29 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
             Real tv = (lane < T1) ? t * nsc : Real(0);
             tv = lane == 32 ? nsc : tv;
             if (REDO) {
-                if (col > sp.c0 && col < sp.c1 && (col - sp.c0) % FW_RECHECK == 0) {
+                if (col == chk && col > sp.c0 && col < sp.c1) {
                     double dmax = 0.0, amax = 0.0;
+                    Real old[R];
+                    slots_load<R>((const AW_GLOBAL Real *)row, lane, old);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
-                        const double nv = (double)(x[r] * nsc), ov = (double)row[r * 64];
+                        const double nv = (double)(x[r] * nsc), ov = (double)old[r];
                         dmax = fmax(dmax, fabs(nv - ov));
                         amax = fmax(amax, fabs(nv));
                     }
                     rejoined = wave_max(dmax) <= tol * wave_max(amax);
+                    tv = (lane == 33 && rejoined) ? Real(1) : tv;
                 }
-                tv = (lane == 33 && rejoined) ? Real(1) : tv;
             }
             sh.tv[lane] = tv;
             fw_barrier();
             if (store) {
 #pragma unroll
-                for (int r = 0; r < R; r++) row[r * 64] = x[r] * nsc;
+                for (int r = 0; r < R; r++) x[r] *= nsc;
+                slots_store<R>(row, lane, x);
             }
             nw = (lane == (col & 63)) ? norm : nw;
-            if (col == ev || (REDO && rejoined)) break;
+            if (col == ev) break;
         }
         done = col == sp.clast || (REDO && rejoined);
         if ((col & 63) == 63 || done) {
@@ -520,15 +538,14 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
     if (sp.mode == 0) {
         const AW_GLOBAL double *pr = gp(d.lprior);
 #pragma unroll
-        for (int r = 0; r < R; r++) v[r] = (Real)pr[r * 64 + lane];
+        for (int r = 0; r < R; r++) v[r] = (Real)pr[slot_pos(r, lane, R)];
     } else if (sp.mode == 1) {
         const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = (lane * R + r < S) ? Real(1) : Real(0);
     } else {
         const AW_GLOBAL Real *src = bnd + (size_t)sp.bin * BND_STRIDE;
-#pragma unroll
-        for (int r = 0; r < R; r++) v[r] = src[r * 64 + lane];
+        slots_load<R>(src, lane, v);
     }
 
     // the column goes to the sums wave
@@ -583,8 +600,9 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
     // invariant columns without a switch: the columns before `plain`
     auto plain_to = [&](int next) {
         const unsigned long long m = __ballot(clsv != -1) >> (next & 63);
-        const int n = m ? next + (int)__ffsll((long long)m) - 1 : wb + 64;
-        return min(min(n, bend), sp.clast + 1);
+        int n = m ? next + (int)__ffsll((long long)m) - 1 : wb + 64;
+        n = min(min(n, bend), sp.clast + 1);
+        return REDO ? min(n, sp.recheck(next - 1) + 1) : n;
     };
 
     for (int col = sp.c0;;) {
@@ -597,7 +615,6 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
             Real same[R];
             scan(same);
             fw_barrier();
-            if (REDO && ends(col)) return;
             const Real sc = sh.tv[32];
             Real tf[R];
 #pragma unroll
@@ -670,11 +687,11 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
                     for (int k = 0; k < VCH; k++)
 #pragma unroll
                         for (int r = 0; r < R; r++)
-                            if (k0 + k < VST) sh.vs[(k0 + k) * RW + r * 64 + lane] = (Real)rows[k][r];
+                            if (k0 + k < VST) sh.vs[(k0 + k) * RW + slot_pos(r, lane, R)] = (Real)rows[k][r];
                 }
             }
 #pragma unroll
-            for (int r = 0; r < R; r++) e[r] = sh.vs[(cls - vbase) * RW + r * 64 + lane];
+            for (int r = 0; r < R; r++) e[r] = sh.vs[(cls - vbase) * RW + slot_pos(r, lane, R)];
         } else {
 #pragma unroll
             for (int r = 0; r < R; r++) e[r] = cls == -1 ? fl.ce[r] : Real(1);
@@ -714,6 +731,9 @@ __device__ __forceinline__ void fw_instance(const DevInst d, void *lds, const Fw
     auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
     FwSpan sp{uni(t.c0), uni(t.cs), uni(t.c1), uni(t.mode), uni(t.bout), uni(t.bin), 0};
     sp.clast = sp.bout >= 0 ? sp.c1 : sp.c1 - 1;
+    // a re-run's columns are waited for while other instances' tracebacks fill
+    // the device
+    __builtin_amdgcn_s_setprio(3);
     if (uni((int)threadIdx.x >> 6)) fw_sums<Real, R, NT1, REDO>(d, sh, sp, bnd, bnorm, tol, early);
     else fw_lanes<Real, R, NT1, REDO>(d, sh, sp, bnd);
 }

@@ -90,6 +90,36 @@ __device__ __forceinline__ double readlane_d(double x, int l)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// the slots of a lane in a lane-run row (slot_pos), loaded and stored up to 16
+// bytes at a time
+template <class X, int R>
+struct SlotPiece {
+    static constexpr int N = slot_vec(R) * sizeof(X) <= 16 ? slot_vec(R) : 16 / sizeof(X);
+    typedef X type __attribute__((ext_vector_type(N)));
+};
+template <int R, class X>
+__device__ __forceinline__ void slots_load(const AW_GLOBAL X *row, int lane, X (&x)[R])
+{
+    using P = SlotPiece<X, R>;
+#pragma unroll
+    for (int r = 0; r < R; r += P::N) {
+        const auto v = *(const AW_GLOBAL typename P::type *)(row + slot_pos(r, lane, R));
+#pragma unroll
+        for (int k = 0; k < P::N; k++) x[r + k] = v[k];
+    }
+}
+template <int R, class X>
+__device__ __forceinline__ void slots_store(AW_GLOBAL X *row, int lane, const X (&x)[R])
+{
+    using P = SlotPiece<X, R>;
+#pragma unroll
+    for (int r = 0; r < R; r += P::N) {
+        typename P::type v;
+#pragma unroll
+        for (int k = 0; k < P::N; k++) v[k] = x[r + k];
+        *(AW_GLOBAL typename P::type *)(row + slot_pos(r, lane, R)) = v;
+    }
+}
 
 template <class Real>
 __device__ __forceinline__ const AW_GLOBAL Real *planes(const DevInst &d, int b, int RW)

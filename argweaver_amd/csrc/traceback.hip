@@ -106,9 +106,7 @@ __device__ __forceinline__ int sample_state(const Real (&rv)[R], const Real (&tr
 template <class Real, int R>
 __device__ __forceinline__ void row_load(const AW_GLOBAL Real *alpha, int col, Real (&rv)[R])
 {
-    const AW_GLOBAL Real *row = alpha + (size_t)col * (64 * R);
-#pragma unroll
-    for (int r = 0; r < R; r++) rv[r] = row[r * 64 + lane_id()];
+    slots_load<R>(alpha + (size_t)col * (64 * R), lane_id(), rv);
 }
 
 // state sampled from column col alone (the last column, or the speculative
@@ -230,8 +228,7 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
         float tf[R], tk[R];
         {
             int ti[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) ti[r] = info[r * 64 + lane];
+            slots_load<R>(info, lane, ti);
             Real tr[R];
             tb_weights<Real, R>(d, ti, t, tr);
 #pragma unroll
@@ -245,11 +242,11 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
             // lane's column of this chunk, and the entries of k's lane there:
             // the states before k in its lane, and k itself
             const int j = pos + (lane >> 2);
-            const AW_GLOBAL Real *grow = alpha + (size_t)(ce - 1 - min(j, n - 1)) * RW + t.lk;
+            const AW_GLOBAL Real *grow = alpha + (size_t)(ce - 1 - min(j, n - 1)) * RW;
             Real gv[R];
 #pragma unroll
             for (int r = 0; r < R; r++)
-                if (r <= t.rk) gv[r] = grow[r * 64];
+                if (r <= t.rk) gv[r] = grow[slot_pos(r, t.lk, R)];
             // columns c and c + 8 together, so that their first fold follows
             // at once; value 2c is column c's total, 2c + 1 its sum over the
             // lanes before k's
@@ -294,8 +291,7 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
                 Real rv[R], tr[R];
                 int ti[R];
                 row_load<Real, R>(alpha, ce - 1 - x, rv);
-#pragma unroll
-                for (int r = 0; r < R; r++) ti[r] = info[r * 64 + lane];
+                slots_load<R>(info, lane, ti);
                 tb_weights<Real, R>(d, ti, t, tr);
                 const int kn = sample_state<Real, R>(rv, tr, S, readlane_d(uw, x));
                 if (kn != k) {
@@ -317,14 +313,16 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
         const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)b * RW;
         const int pk = lane_pos(k, R);
         const Real rrk = cn[CRR * RW + pk], crk = cn[CCR * RW + pk];
-        Real rv[R], tr[R];
+        Real rv[R], tr[R], dp[R];
+        int dt[R];
         row_load<Real, R>(alpha, ce - n - 1, rv);
+        slots_load<R>(detn, lane, dt);
+        slots_load<R>(cn + CDP * RW, lane, dp);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int s = lane * R + r;
-            const int dt = detn[r * 64 + lane] & ~DET_SHARED;   // -1 stays no state
-            const Real dp = cn[CDP * RW + r * 64 + lane];
-            tr[r] = (s == cs) ? crk : (s == rs) ? rrk : (dt == k ? dp : Real(0));
+            // (-1 stays no state)
+            tr[r] = (s == cs) ? crk : (s == rs) ? rrk : ((dt[r] & ~DET_SHARED) == k ? dp[r] : Real(0));
         }
         k = sample_state<Real, R>(rv, tr, cp(d.soff)[b] - cp(d.soff)[b - 1], readlane_d(uw, n));
         pv = lane >= n ? k : pv;
@@ -561,13 +559,13 @@ __global__ __launch_bounds__(256) void k_tb_pred(const DevInst *__restrict__ D,
     }
     __syncthreads();
     auto source = [&](int p, int t) {   // a deterministic transition into t
-        const int j = (p & 63) * R + (p >> 6);
+        const int j = pos_state(p, R);
         return j < S1 && t >= 0 && t < S2 && j != rs && j != cs;
     };
     for (int p = threadIdx.x; p < RW; p += 256) {
         const int t = det[p];
         if (source(p, t)) {
-            atomicMax(&best[t], key(weight(CDP, p), (p & 63) * R + (p >> 6)));
+            atomicMax(&best[t], key(weight(CDP, p), pos_state(p, R)));
             atomicAdd(&count[t], 1);
         }
     }
@@ -579,7 +577,7 @@ __global__ __launch_bounds__(256) void k_tb_pred(const DevInst *__restrict__ D,
     }
     auto out = gp(d.pred) + (size_t)b * RW;
     for (int p = threadIdx.x; p < RW; p += 256) {
-        const int k = (p & 63) * R + (p >> 6);
+        const int k = pos_state(p, R);
         unsigned long long m = best[k];
         if (rs >= 0) {
             const float w = weight(CRR, p);
