@@ -391,6 +391,18 @@ struct EmitTime {
     double mut0, nomut0, inv, inv_root;
 };
 
+__host__ __device__ inline void emit_invariant(const TreeView &t, const Model &m, double mainlen,
+                                               int time, double &inv, double &inv_root)
+{
+    const double mintime = m.times[1] * .1;
+    const double coal_time = m.times[time];
+    const double len = mainlen + fmax(coal_time - 0.0, mintime);
+    inv = .25 * exp(-m.mu * fmax(len, mintime));
+    const double len_r = mainlen + fmax(coal_time - 0.0, mintime) +
+                         fmax(coal_time - m.times[t.age[t.root]], mintime);
+    inv_root = .25 * exp(-m.mu * fmax(len_r, mintime));
+}
+
 __host__ __device__ inline void emit_time_terms(const TreeView &t, const Model &m, double mainlen,
                                                 int time, EmitTime &et)
 {
@@ -399,11 +411,7 @@ __host__ __device__ inline void emit_time_terms(const TreeView &t, const Model &
     const double d0 = fmax(coal_time - 0.0, mintime);
     et.mut0 = prob_branch(d0, m.mu, true);
     et.nomut0 = prob_branch(d0, m.mu, false);
-    const double len = mainlen + fmax(coal_time - 0.0, mintime);
-    et.inv = .25 * exp(-m.mu * fmax(len, mintime));
-    const double len_r = mainlen + fmax(coal_time - 0.0, mintime) +
-                         fmax(coal_time - m.times[t.age[t.root]], mintime);
-    et.inv_root = .25 * exp(-m.mu * fmax(len_r, mintime));
+    emit_invariant(t, m, mainlen, time, et.inv, et.inv_root);
 }
 
 __host__ __device__ inline void emit_terms(const TreeView &t, const Model &m, const EmitTime &et,

@@ -30,7 +30,7 @@ namespace aw {
 // forward-table rows have a constant stride and column col starts at
 // col * RW.
 struct DevInst {
-    int T, N, B, L, nrows, Smax, TC, R, nvar;
+    int T, N, B, L, nrows, Smax, R, nvar;
     long long W;              // column-states sum_b blocklen_b * S_b
     const Model *model;
     // trees
@@ -41,11 +41,10 @@ struct DevInst {
     // column classes: -1 invariant, -2 masked, >=0 variant row index
     int *vflag, *cls, *vcol;  // [L]
     // prep outputs in state order (pruning and traceback lookups)
-    int *snode, *stime;       // [Stot]
-    double *eterm;            // [Stot*6]
     int *order, *roots;       // [B*N] node levels: height | depth << 16, [B] roots
-    double *nmut;             // [B*N*2]
-    double *tm, *tm2s;        // [B*(T-1)^2] P(a->b) other branch, [B*TC] same branch
+    double *pmut;             // [(T+1)*T*2] see mut_entry
+    double *tm;               // [B*(T-1)^2] P(a->b), other branch
+    double *tvec;             // [B*time_vecs(T-1)] what P(a->b) on the same branch adds
     int *srcs;                // [2B] recombination / recoalescence source of the switch into b
     // prep outputs in the lane-run layout, one row of RW per block
     int *linfo;               // [B*RW] time | flags | age(node) << 11 | node << 16
@@ -107,12 +106,22 @@ __host__ __device__ inline int pos_state(int p, int R)
     return (q & 63) * R + (q >> 6) * V + p % V;
 }
 
-// offset of the (c, a, b) entry of the per-block same-branch table:
-// sum_{x<c} (T1-x)^2, in closed form
-__host__ __device__ inline int tc_base(int c, int T1)
-{
-    return c * T1 * T1 - T1 * c * (c - 1) + (c - 1) * c * (2 * c - 1) / 6;
-}
+// The mutation and no-mutation probabilities of a branch by its two times: the
+// entry of a branch from time j up to time i, i >= j; row T: from 0 to time j.
+// Times are few, branches are many.
+__host__ __device__ inline int mut_entry(int i, int j, int T) { return 2 * (i * T + j); }
+
+// What a block keeps, besides tm, of the same-branch entries P(a -> b) (see
+// TransVec): D, E and norecombs by time, Y[b] = X[m-1][b] with m the youngest
+// age a thread can reach (0 where m is 0, as it is unless the thread starts
+// inside a subtree), m itself, and X[a][b] = exp(lnE2[b] + lnB[a]) for a < b,
+// the term that a branch's age c takes off:
+//   P_same(a -> b) = 2 P_other(a -> b) + D[a] E[b] (Y[b] - X[c-1][b])
+//                    + (a == b) norecombs[b]
+enum : int { TV_D = 0, TV_E, TV_NORECOMBS, TV_Y, TV_N };
+__host__ __device__ inline int tv_minage(int T1) { return TV_N * T1; }
+__host__ __device__ inline int tv_x(int T1) { return TV_N * T1 + 1; }
+__host__ __device__ inline int time_vecs(int T1) { return tv_x(T1) + T1 * T1; }
 
 enum class Precision { FP64 = 0, FP32 = 1 };
 

@@ -74,38 +74,65 @@ __global__ void k_classify_b(const DevInst *__restrict__ D, const long long *col
     gp(d.cls)[col] = inv ? (c0 == 'N' ? -2 : -1) : 0;
 }
 
-// variant-column numbering of one instance: each of 1024 threads owns a
-// contiguous run of columns
+// variant-column numbering of one instance: each of 16 waves owns a contiguous
+// run of columns and counts them 64 at a time, a load of 8 times that in flight
+// (runs of single threads, uncoalesced, took 0.77 ms for 500000 columns, this
+// 0.28).  Also the instance's table of branch mutation probabilities.
 __global__ __launch_bounds__(1024) void k_scan_b(const DevInst *__restrict__ D, int *nvar_out)
 {
-    __shared__ int part[1024];
+    __shared__ int part[16];
     const DevInst &d = D[blockIdx.x];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
     if (d.hostprep) {   // the whole workgroup leaves: the host knows the count
         if (tid == 0) nvar_out[blockIdx.x] = 0;
         return;
     }
-    const int per = (d.L + 1023) / 1024;
-    const int s0 = min(d.L, tid * per), e0 = min(d.L, s0 + per);
-    int loc = 0;
-    for (int i = s0; i < e0; i++) loc += gp(d.vflag)[i];
-    part[tid] = loc;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int v = (tid >= off) ? part[tid - off] : 0;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    int run = part[tid] - loc;
-    for (int i = s0; i < e0; i++) {
-        if (gp(d.vflag)[i]) {
-            gp(d.cls)[i] = run;
-            gp(d.vcol)[run] = i;
-            run++;
+    {
+        const Model &M = *d.model;
+        const int T = d.T;
+        const double mintime = M.times[1] * .1;
+        for (int x = tid; x < (T + 1) * T; x += 1024) {
+            const int i = x / T, j = x % T;
+            const double t = i < T ? M.times[i] - M.times[j] : M.times[j] - 0.0;
+            gp(d.pmut)[2 * x] = prob_branch(fmax(t, mintime), M.mu, true);
+            gp(d.pmut)[2 * x + 1] = prob_branch(fmax(t, mintime), M.mu, false);
         }
     }
-    if (tid == 1023) nvar_out[blockIdx.x] = part[1023];
+    const int per = (d.L + 16 * 64 - 1) / (16 * 64) * 64;
+    const int s0 = min(d.L, (tid >> 6) * per), e0 = min(d.L, s0 + per);
+    constexpr int U = 8;
+    const auto walk = [&](int run, bool store) {
+        for (int c0 = s0; c0 < e0; c0 += 64 * U) {
+            int f[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = c0 + 64 * u + lane;
+                f[u] = c < e0 ? gp(d.vflag)[c] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const unsigned long long m = __ballot(f[u] != 0);
+                if (store && f[u]) {
+                    const int c = c0 + 64 * u + lane;
+                    const int k = run + __popcll(m & ((1ull << lane) - 1));
+                    gp(d.cls)[c] = k;
+                    gp(d.vcol)[k] = c;
+                }
+                run += __popcll(m);
+            }
+        }
+        return run;
+    };
+    const int cnt = walk(0, false);
+    if (lane == 0) part[tid >> 6] = cnt;
+    __syncthreads();
+    int base = 0, total = 0;
+    for (int w = 0; w < 16; w++) {
+        if (w < (tid >> 6)) base += part[w];
+        total += part[w];
+    }
+    walk(base, true);
+    if (tid == 0) nvar_out[blockIdx.x] = total;
 }
 
 //===========================================================================
@@ -130,7 +157,7 @@ struct PrepShared {
     double red[3 * 4];
     // per-time factors of the state planes
     double eB[MAXT], eN[MAXT], eE2[MAXT], low[MAXT];
-    EmitTime et[MAXT];
+    double inv[MAXT], inv_root[MAXT];   // emission of an invariant column, off and on the root
 };
 
 // Lineage counts (count_lineages) with one thread per node and integer LDS
@@ -219,8 +246,12 @@ __device__ inline void block_sums3(double (&v)[3], double *red)
     for (int x = 0; x < 3; x++) v[x] = ((red[4 * x] + red[4 * x + 1]) + red[4 * x + 2]) + red[4 * x + 3];
 }
 
-// At most 95 VGPRs (five waves per SIMD, no spill): 16.5 -> 14.7 ms on the
-// 256-instance batch against the 119 the compiler picks unbounded (four).
+// Bound by its vector instructions (half of the cycles) and the barriers between
+// its short phases; what it writes is 25 KB a block.  A table of all same-branch
+// entries (20 KB) and emission terms per state (48 bytes) took it from 11.2 to
+// 16.4 ms on the 256-instance batch (407000 blocks): the traceback forms the
+// entries from X (engine.h), the emission terms depend on times only.
+// At most 95 VGPRs: five waves per SIMD, without a spill.
 __global__ __launch_bounds__(256, 5) void k_prep_b(const DevInst *__restrict__ D,
                                                 const int *__restrict__ blkoff, int ninst)
 {
@@ -414,26 +445,8 @@ __global__ __launch_bounds__(256, 5) void k_prep_b(const DevInst *__restrict__ D
         sh.eN[a] = exp(tv.lnNegG1[a]);
         sh.eE2[a] = exp(tv.lnE2[a]);
         sh.low[a] = a > 0 ? exp(tv.lnE2[a] + tv.lnB[a - 1]) : 0.0;
-        emit_time_terms(t, M, sh.mainlen, a, sh.et[a]);
+        emit_invariant(t, M, sh.mainlen, a, sh.inv[a], sh.inv_root[a]);
     }
-    for (int n = tid; n < N; n += NT) {
-        for (int a = sh.ag[n]; a <= sh.ni.hi[n]; a++) {
-            int k = sh.ni.first[n] + a - sh.ag[n];
-            gp(d.snode)[so + k] = n;
-            gp(d.stime)[so + k] = a;
-        }
-        // branch mutation probabilities for pruning (prob_tree_mutation)
-        double mut = 0.0, nomut = 0.0;
-        if (n != sh.root) {
-            const double mintime = M.times[1] * .1;
-            double tt = fmax(M.times[sh.ag[sh.par[n]]] - M.times[sh.ag[n]], mintime);
-            mut = prob_branch(tt, M.mu, true);
-            nomut = prob_branch(tt, M.mu, false);
-        }
-        gp(d.nmut)[2 * ((size_t)b * N + n)] = mut;
-        gp(d.nmut)[2 * ((size_t)b * N + n) + 1] = nomut;
-    }
-
     __syncthreads();   // per-time factors complete
 
     // Per-state planes.  For a target state (n, b) with c = age(n), the
@@ -468,13 +481,7 @@ __global__ __launch_bounds__(256, 5) void k_prep_b(const DevInst *__restrict__ D
             const double term1 = tv.D[a] * tv.E[a];
             cj = (term1 * ((2 * (low + tv.G3[a])) - ct) + tv.norecombs[a]) -
                  term1 * (low + tv.G3[a]);
-            EmitTerms e;
-            emit_terms(t, M, sh.et[a], n, a, e);
-            ce = e.inv;
-            for (int x = 0; x < 3; x++) {
-                gp(d.eterm)[6 * (size_t)(so + s) + x] = e.mut[x];
-                gp(d.eterm)[6 * (size_t)(so + s) + 3 + x] = e.nomut[x];
-            }
+            ce = n == sh.root ? sh.inv_root[a] : sh.inv[a];
             if (b == 0) pr = prior_time(a, sh.L, M);
             inf = a | (a == c ? INFO_FIRST : 0) | (a == h ? INFO_LAST : 0) | INFO_VALID |
                   (c << 11) | (n << 16);
@@ -493,20 +500,21 @@ __global__ __launch_bounds__(256, 5) void k_prep_b(const DevInst *__restrict__ D
         if (b == 0) gp(d.lprior)[p] = pr;
     }
 
-    const int TT = T1 * T1;
-    for (int x = tid; x < TT; x += NT) {
-        int a = x / T1, bb = x % T1;
-        gp(d.tm)[(size_t)b * TT + x] = tv.get_time(a, bb, 0, false);
+    // P(a -> b) on another branch (get_time), and the terms the traceback forms
+    // the same-branch entries from (a table of all of those, 20 KB a block, was
+    // a quarter of this kernel's time)
+    auto vec = gp(d.tvec) + (size_t)b * time_vecs(T1);
+    for (int x = tid; x < T1 * T1; x += NT) {
+        const int a = x / T1, bb = x % T1;
+        gp(d.tm)[(size_t)b * T1 * T1 + x] = tv.get_time(a, bb, 0, false);
+        if (a < bb) vec[tv_x(T1) + x] = exp(tv.lnE2[bb] + tv.lnB[a]);
     }
-    for (int x = tid; x < d.TC; x += NT) {
-        int c = 0, base = 0;
-        while (base + (T1 - c) * (T1 - c) <= x) {
-            base += (T1 - c) * (T1 - c);
-            c++;
-        }
-        int r = x - base, w = T1 - c;
-        int a = c + r / w, bb = c + r % w;
-        gp(d.tm2s)[(size_t)b * d.TC + x] = tv.get_time(a, bb, c, true);
+    for (int a = tid; a < T1; a += NT) {
+        vec[TV_D * T1 + a] = tv.D[a];
+        vec[TV_E * T1 + a] = tv.E[a];
+        vec[TV_NORECOMBS * T1 + a] = tv.norecombs[a];
+        vec[TV_Y * T1 + a] = 0.0;
+        if (a == 0) vec[tv_minage(T1)] = 0.0;
     }
 
     if (b == 0) return;
@@ -680,43 +688,55 @@ __global__ __launch_bounds__(64) void k_var_emit_b(const DevInst *__restrict__ D
         ch1[i] = gp(d.c1)[x];
         ag[i] = gp(d.age)[x];
         lvl[i] = gp(d.order)[x];
-        muts[i] = gp(d.nmut)[2 * x];
-        nomuts[i] = gp(d.nmut)[2 * x + 1];
         if (i < nleaves) bases[i] = gp(d.seq)[(size_t)i * d.L + col];
     }
     __syncthreads();
-    const int root = gp(d.roots)[b];
+    const int root = gp(d.roots)[b], T = d.T;
+    // branch mutation probabilities for the pruning (prob_tree_mutation)
+    const auto pm = gp(d.pmut);
+    for (int i = lane; i < N; i += 64) {
+        const auto e = pm + (i != root ? mut_entry(min(ag[par[i]], T - 1), ag[i], T) : 0);
+        muts[i] = i != root ? e[0] : 0.0;
+        nomuts[i] = i != root ? e[1] : 0.0;
+    }
+    __syncthreads();
     {
         TreeView t{N, root, par, ch0, ch1, ag};
         pruning_wave(t, lvl, bases, muts, nomuts, inner, outer);
         if (lane == 0) leaf_partial(gp(d.seq)[(size_t)nleaves * d.L + col], in2);
     }
     __syncthreads();
-    const int so = cp(d.soff)[b], S = cp(d.soff)[b + 1] - so;
+    const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
     auto row = gp(d.vemit) + (size_t)v * RW;
+    const auto info = gp(d.linfo) + (size_t)b * RW;
     for (int p = lane; p < RW; p += 64) {
         const int k = pos_state(p, R);
         double e = 0.0;
         if (k < S) {
-            int n = gp(d.snode)[so + k];
-            const double *et = d.eterm + 6 * (size_t)(so + k);
-            e = emit_variant(in2, inner + 4 * n, outer + 4 * n, n == root, et, et + 3);
+            // the new leaf's branch, and the two parts of the node's branch
+            const int x = info[p], n = info_node(x), a = x & INFO_TIME;
+            const int top = n != root ? min(ag[par[n]], T - 1) : a;
+            const auto e0 = pm + mut_entry(T, a, T), e1 = pm + mut_entry(a, ag[n], T),
+                       e2 = pm + mut_entry(top, a, T);
+            const double mut[3] = {e0[0], e1[0], e2[0]}, nomut[3] = {e0[1], e1[1], e2[1]};
+            e = emit_variant(in2, inner + 4 * n, outer + 4 * n, n == root, mut, nomut);
         }
         row[p] = e;
     }
 }
 
-// log-likelihood: sum of log column normalisers
-__global__ __launch_bounds__(256) void k_lnl_b(const DevInst *__restrict__ D,
+// log-likelihood: sum of log column normalisers (16 waves: 0.42 ms for 500000
+// columns; 4 waves took 1.1)
+__global__ __launch_bounds__(1024) void k_lnl_b(const DevInst *__restrict__ D,
                                                const int *__restrict__ list)
 {
-    __shared__ double part[256];
+    __shared__ double part[1024];
     const DevInst &d = D[list[blockIdx.x]];
     double s = 0.0;
-    for (int c = threadIdx.x; c < d.L; c += 256) s += log(gp(d.norms)[c]);
+    for (int c = threadIdx.x; c < d.L; c += 1024) s += log(gp(d.norms)[c]);
     part[threadIdx.x] = s;
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
+    for (int off = 512; off > 0; off >>= 1) {
         if (threadIdx.x < off) part[threadIdx.x] += part[threadIdx.x + off];
         __syncthreads();
     }
@@ -1118,7 +1138,7 @@ int Batch::upload()
                 d.hostprep = hi.prep ? 1 : 0;
                 d.last_state = hi.last_state;
                 d.T = T; d.N = N; d.B = B; d.L = L; d.nrows = (int)hi.rows.size();
-                d.Smax = Smax; d.TC = tc_base(T - 1, T - 1); d.W = m.W[i]; d.R = R;
+                d.Smax = Smax; d.W = m.W[i]; d.R = R;
             }
             d.model = p.take<Model>(1);
             d.parent = p.take<int>((size_t)B * N);
@@ -1589,18 +1609,14 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         for (int i = 0; i < n; i++) {
             DevInst &d = m.h[i];
             const int B = d.B, N = d.N, L = d.L, T1 = d.T - 1, RW = 64 * d.R;
-            const int Stot = m.soff[i][B];
             d.vflag = p.take<int>(L);
             d.cls = p.take<int>(L);
             d.vcol = p.take<int>(L);
-            d.snode = p.take<int>(Stot);
-            d.stime = p.take<int>(Stot);
-            d.eterm = p.take<double>((size_t)Stot * 6);
             d.order = p.take<int>((size_t)B * N);
             d.roots = p.take<int>(B);
-            d.nmut = p.take<double>((size_t)B * N * 2);
+            d.pmut = p.take<double>(mut_entry(d.T + 1, 0, d.T));
             d.tm = p.take<double>((size_t)B * T1 * T1);
-            d.tm2s = p.take<double>((size_t)B * d.TC);
+            d.tvec = p.take<double>((size_t)B * time_vecs(T1));
             d.srcs = p.take<int>(2 * (size_t)B);
             d.linfo = p.take<int>((size_t)B * RW);
             // coefficient planes in the run's precision only
@@ -1702,7 +1718,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
                               hipMemcpyHostToDevice, s));
         HIP_OK(hipMemcpyAsync(d.tm, hp->tm.data(), sizeof(double) * (size_t)B * T1 * T1,
                               hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.tm2s, hp->tm2s.data(), sizeof(double) * (size_t)B * d.TC,
+        HIP_OK(hipMemcpyAsync(d.tvec, hp->tvec.data(), sizeof(double) * hp->tvec.size(),
                               hipMemcpyHostToDevice, s));
         HIP_OK(hipMemcpyAsync(d.srcs, hp->srcs.data(), sizeof(int) * 2 * (size_t)B,
                               hipMemcpyHostToDevice, s));
@@ -1783,7 +1799,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     } joiner{helper};
     if (forward_stage(m, fp32, opt, order, shf, t1max, rs, early_tb)) return 1;
     (void)hipEventRecord(c.ev[4], s);
-    hipLaunchKernelGGL(k_lnl_b, dim3(n), dim3(256), 0, s, m.dD, m.d_list);
+    hipLaunchKernelGGL(k_lnl_b, dim3(n), dim3(1024), 0, s, m.dD, m.d_list);
     HIP_OK(hipGetLastError());
     // traceback tiles: the chains of every tile, then their resolution
     if (opt.traceback) {

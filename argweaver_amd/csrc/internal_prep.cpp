@@ -594,12 +594,11 @@ int prepare_internal(const ArgTrees &tr, const Model &m, char **seqs, int minage
         return 1;
     }
     const int R = hp.R, RW = 64 * R;
-    const int TC = tc_base(T1, T1);
     hp.planes.assign((size_t)B * NCOEF * RW, 0.0);
     hp.info.assign((size_t)B * RW, INFO_FIRST | INFO_LAST | 31);
     hp.det.assign((size_t)B * RW, -1);
     hp.tm.assign((size_t)B * T1 * T1, 0.0);
-    hp.tm2s.assign((size_t)B * TC, 0.0);
+    hp.tvec.assign((size_t)B * time_vecs(T1), 0.0);
     hp.srcs.assign(2 * (size_t)B, -1);
     hp.prior.assign(RW, 0.0);
     hp.cls.assign(L, -1);
@@ -621,7 +620,7 @@ int prepare_internal(const ArgTrees &tr, const Model &m, char **seqs, int minage
         double *pl = &hp.planes[(size_t)b * NCOEF * RW];
         int *info = &hp.info[(size_t)b * RW];
         double *tmb = &hp.tm[(size_t)b * T1 * T1];
-        double *tm2 = &hp.tm2s[(size_t)b * TC];
+        double *vec = &hp.tvec[(size_t)b * time_vecs(T1)];
         Lineages Lc{};
         TransVec tv{};
         if (S == 0) {
@@ -630,7 +629,7 @@ int prepare_internal(const ArgTrees &tr, const Model &m, char **seqs, int minage
             pl[CJ * RW + p] = 1.0;
             pl[CE * RW + p] = 1.0;
             info[p] = 0 | INFO_FIRST | INFO_LAST | INFO_VALID;
-            for (int x = 0; x < TC; x++) tm2[x] = 1.0;
+            vec[TV_NORECOMBS * T1] = 1.0;
             if (b == 0) hp.prior[p] = 1.0;
         } else {
             lineages_internal(t, T, Lc);
@@ -638,9 +637,15 @@ int prepare_internal(const ArgTrees &tr, const Model &m, char **seqs, int minage
             const int mina = std::max(minage, t.nodes[sub_root(t)].age);
             for (int a = 0; a < T1; a++)
                 for (int bb = 0; bb < T1; bb++) tmb[a * T1 + bb] = get_time_min(tv, a, bb, 0, mina, false);
-            for (int c = 0, x = 0; c < T1; c++)
-                for (int a = c; a < T1; a++)
-                    for (int bb = c; bb < T1; bb++, x++) tm2[x] = get_time_min(tv, a, bb, c, mina, true);
+            for (int a = 0; a < T1; a++) {
+                vec[TV_D * T1 + a] = tv.D[a];
+                vec[TV_E * T1 + a] = tv.E[a];
+                vec[TV_NORECOMBS * T1 + a] = tv.norecombs[a];
+                vec[TV_Y * T1 + a] = mina > 0 ? exp(tv.lnE2[a] + tv.lnB[mina - 1]) : 0.0;
+                for (int bb = a + 1; bb < T1; bb++)
+                    vec[tv_x(T1) + a * T1 + bb] = exp(tv.lnE2[bb] + tv.lnB[a]);
+            }
+            vec[tv_minage(T1)] = mina;
             EmitInternal em(t, m, s);
             for (int k = 0; k < S; k++) {
                 const int n = s.node[k], a = s.time[k], c = t.nodes[n].age;

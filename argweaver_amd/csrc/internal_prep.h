@@ -16,7 +16,7 @@ struct HostPrep {
     std::vector<int> Sreal;      // [B] states of the reference (0 for a complete tree)
     std::vector<double> planes;  // [B * NCOEF * 64R] coefficient planes (see Coef)
     std::vector<int> info, det;  // [B * 64R] state info, switch targets of block b-1's states
-    std::vector<double> tm, tm2s;   // [B * (T-1)^2], [B * TC]
+    std::vector<double> tm, tvec;   // [B * (T-1)^2], [B * time_vecs(T-1)]
     std::vector<int> srcs;       // [2B] recombination / recoalescence source of each switch
     std::vector<double> prior;   // [64R] first-column prior
     std::vector<int> cls;        // [L] -1 invariant, -2 masked (or no states), >= 0 variant row

@@ -44,11 +44,7 @@ size_t Server::footprint(const HostInstance &hi, Precision prec)
     std::vector<int> Sv;
     instance_states(ft, T, &Sv);
     int Smax = 1;
-    long long Stot = 0;
-    for (int S : Sv) {
-        Smax = std::max(Smax, S);
-        Stot += S;
-    }
+    for (int S : Sv) Smax = std::max(Smax, S);
     // states per lane as the kernels round it (1, 2, 4, 6, 8, 12, 16)
     size_t R = 16;
     for (int r : {1, 2, 4, 6, 8, 12, 16})
@@ -69,13 +65,11 @@ size_t Server::footprint(const HostInstance &hi, Precision prec)
         }
     }
     const size_t rsz = prec == Precision::FP32 ? 4 : 8;
-    const size_t TC = (size_t)tc_base(T1, T1);
     size_t b = (size_t)L * RW * rsz;                          // forward table
     b += (size_t)B * RW * (NCOEF * rsz + 4 + 4 + 2);          // planes, info, targets, sources
     b += (size_t)std::max<long long>(nvar, 1) * RW * 8;        // variant rows
-    b += (size_t)B * ((size_t)T1 * T1 + TC) * 8;               // transition tables
-    b += (size_t)Stot * (4 + 4 + 48);                          // state tables, emission terms
-    b += (size_t)B * N * (5 * 4 + 16 + 4) + (size_t)B * 12;    // trees, pruning
+    b += (size_t)B * ((size_t)T1 * T1 + time_vecs(T1)) * 8;    // transition tables
+    b += (size_t)B * N * (5 * 4 + 4) + (size_t)B * 12;         // trees, pruning
     b += (size_t)L * (3 * 4 + 8 + 4 + 8 + hi.rows.size());     // columns, uniforms, sequences
     return b + (size_t)16 * 4096;
 }
