@@ -60,6 +60,9 @@ struct DevInst {
     // outputs
     void *alpha;              // [L*RW] forward table, double or float
     double *norms;            // [L] column normalisers
+    // [L/32+1] bit c: column c is not the recursion of the column stored before
+    // it (an FP32 tile's start; where a re-run tile rejoined its stored columns)
+    unsigned *cut;
     int *path;                // [L]
     double *lnl;              // [1]
 };

@@ -83,6 +83,7 @@ __global__ __launch_bounds__(1024) void k_scan_b(const DevInst *__restrict__ D, 
     __shared__ int part[16];
     const DevInst &d = D[blockIdx.x];
     const int tid = threadIdx.x, lane = tid & 63;
+    for (int x = tid; x < d.L / 32 + 1; x += 1024) gp(d.cut)[x] = 0;
     if (d.hostprep) {   // the whole workgroup leaves: the host knows the count
         if (tid == 0) nvar_out[blockIdx.x] = 0;
         return;
@@ -1627,6 +1628,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
             d.pred = p.take<unsigned short>((size_t)B * RW);
             d.lprior = p.take<double>(RW);
             d.norms = p.take<double>(L);
+            d.cut = p.take<unsigned>(L / 32 + 1);
             d.path = p.take<int>(L);
             d.lnl = p.take<double>(1);
         }
@@ -1989,7 +1991,9 @@ static int run_one(Batch &bt, const HostInstance &hi, const double *u, int *path
     opt.traceback = (u != nullptr);
     // long instances trace back in tiles (the thread is the same as with one
     // tile: fix-up passes re-sample until the chains coalesce)
-    opt.tile_cols = (tile_cols == 0 && hi.ft.seqlen >= 16384) ? 4096 : tile_cols;
+    // (500000 columns in tiles of 4096 / 8192 / 16384 / none: 3.3 / 3.1 / 3.2 / 22
+    // ms; 100000 in FP64: 1.4 / 1.2 / 0.9 / 2.4; 20000: 0.33 / 0.33 / - / 0.38)
+    opt.tile_cols = (tile_cols == 0 && hi.ft.seqlen >= 16384) ? 8192 : tile_cols;
     // FP32 forwards of long instances run as tiles (FP64 keeps the
     // sequential forward: its contract is the reference's table)
     if (prec == Precision::FP32) {

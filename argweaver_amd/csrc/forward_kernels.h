@@ -501,6 +501,12 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
         if (sp.c0 == 0 && L > 1) norms[0] = 1.0;
         if (REDO && sp.mode == 2) norms[sp.c0] = bnorm[sp.bin];
     }
+    // the columns that do not follow from the one stored before them
+    auto mark = [&](int c) { atomicOr(&d.cut[c >> 5], 1u << (c & 31)); };
+    if (sizeof(Real) == 4 && lane == 0) {
+        if (sp.cs > 0) mark(sp.cs);
+        if (rejoined && col + 1 < sp.c1) mark(col + 1);
+    }
     if (REDO && early && lane == 0) *early = rejoined ? col + 1 : 0;
 }
 

@@ -70,7 +70,7 @@ size_t Server::footprint(const HostInstance &hi, Precision prec)
     b += (size_t)std::max<long long>(nvar, 1) * RW * 8;        // variant rows
     b += (size_t)B * ((size_t)T1 * T1 + time_vecs(T1)) * 8;    // transition tables
     b += (size_t)B * N * (5 * 4 + 4) + (size_t)B * 12;         // trees, pruning
-    b += (size_t)L * (3 * 4 + 8 + 4 + 8 + hi.rows.size());     // columns, uniforms, sequences
+    b += (size_t)L * (3 * 4 + 8 + 4 + 8 + hi.rows.size()) + L / 8;   // columns, uniforms, sequences
     return b + (size_t)16 * 4096;
 }
 

@@ -15,19 +15,24 @@
 // Every stored sample is the sample of its column given its right neighbour,
 // whatever was predicted, so the thread is that of a column-by-column walk.
 //
-// Inside a unit a wave tests columns for "the state stays" sixteen at a time:
-// the weights of the column's states under a fixed next state are summed in
-// FP32 below, at and in total, and the column stays when its pick lies inside
-// the state's share by more than 2^-13 of the total, sixty times the bound on
-// the FP32 sums' error.  Any other column is sampled with the FP64 cumulative
-// sums.
+// Inside a unit a wave decides its columns at once, a lane each, without
+// reading their rows.  The total that a column's pick is a fraction of is what
+// the forward recursion computed the next column's entry from: entry * normaliser
+// / emission.  The state j assumed for the column has the share entry *
+// weight of it; the sums below j are unknown, but lie between 0 and the rest, so
+// a uniform that is off both ends by more than that (and 2^-13, sixty times
+// the bound on the FP32 recursion's rounding) picks j wherever j stands.
+// Only the other columns, about twice the share that is not j's, are sampled from
+// their rows, with the FP64 cumulative sums; so are those whose next column
+// was not computed from the stored one (DevInst::cut).  The columns at switches go
+// the same way, j being the likeliest source.
 //
-// Bound by the rows' latency: one CU streams them at about 33 GB/s, which is
-// 0.03 / 0.06 / 0.12 us per column at 4 / 8 FP32 and 8 FP64 states per lane,
-// against 0.6 / 0.9 / 1.0 us of a wave sampling column by column.  Measured
-// with it on MI355X: 10000 columns of 96 states, FP64, 5.1 -> 0.48 ms; 500k
-// columns of 700 states, FP32, 4096-column tiles, 76 -> 15 ms; 256 instances
-// (14.9M columns, FP32) 49.6 -> 8.6 ms after the forward.
+// Reading every row, a CU's bandwidth bound the walk (33 GB/s: 0.03 / 0.06 / 0.12
+// us per column at 4 / 8 FP32 and 8 FP64 states per lane); now the latency of
+// about six dependent loads per round of units does.  On MI355X: 10000 columns of
+// 96 states, FP64, 5.1 ms column by column, 0.39 by rows, 0.24; 500k columns of
+// 700 states, FP32, in tiles, 76, 16.6, 4.4; 256 instances (14.9M columns, FP32)
+// after the forward 49.6, 8.3, 3.1.
 #include "traceback.h"
 
 #include "kernel_util.h"
@@ -44,10 +49,9 @@ constexpr int tb_waves()
     return BIG ? 8 : 16;
 }
 
-// columns tested per unit, at most 63: one lane each, and one for the switch
-// after them.  Blocks average 25-55 columns; 63 and 32 are 1-3 % slower (the
-// longest unit of a window sets its time; short ones pay more entries).
-constexpr int TB_SEG = 48;
+// columns per unit, at most 63: one lane each, and one for the switch after
+// them.  Blocks average 10-55 columns; 48 and 32 are 2-10 % slower.
+constexpr int TB_SEG = 63;
 constexpr unsigned TB_NONE = 0xffff;   // no predicted source
 
 // LDS: per-unit results, then the units' source tables
@@ -172,43 +176,24 @@ __device__ __forceinline__ void tb_weights(const DevInst &d, const int (&ti)[R],
     }
 }
 
-// x of lanes [x.lo | y.lo] and [x.hi | y.hi], added: the lower half of the
-// wave keeps x, the upper half y
-__device__ __forceinline__ float fold32(float x, float y)
+// Table entries below this may have lost bits to underflow: such columns are
+// sampled from their rows.
+template <class Real>
+constexpr double tb_small()
 {
-    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+    return sizeof(Real) == 4 ? 1e-30 : 1e-280;
 }
-// the same over the odd and even 16-lane rows
-__device__ __forceinline__ float fold16(float x, float y)
-{
-    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
-}
-// the same inside a row: lanes without bit keep x, the others y; CTRL pairs
-// lanes that differ in that bit
-template <int CTRL>
-__device__ __forceinline__ float fold_row(float x, float y, bool bit)
-{
-    return (bit ? y : x) + dpp_r<CTRL>(bit ? x : y);
-}
-constexpr int DPP_ROW_ROR8 = 0x128, DPP_ROW_HALF_MIRROR = 0x141, DPP_QUAD_SWAP2 = 0x4E;
 
-// Sums of 32 values over the 64 lanes at once, lane l receiving the sum of
-// value l >> 1: each fold halves the values, 70 instructions instead of the
-// 32 * 12 of separate butterflies.  v[i] holds values i and i + 16 already
-// folded by fold32.
-__device__ __forceinline__ float sum32(float (&v)[16])
+// Whether the state j of column c, with entry a0 and transition weight w into
+// state k of column c+1, is certainly the sample for the uniform u.  v1: the
+// entry of k in column c+1 before normalisation, which by the recursion is
+// e * (sum over the states of column c of entry * weight), e being k's emission
+// there.  Cumulative sums below j lie between 0 and the total less j's share.
+template <class Real>
+__device__ __forceinline__ bool tb_certain(double a0, double w, double v1, double e, double u)
 {
-    const int lane = lane_id();
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = fold16(v[i], v[i + 8]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = fold_row<DPP_ROW_ROR8>(v[i], v[i + 4], lane & 8);
-#pragma unroll
-    for (int i = 0; i < 2; i++) v[i] = fold_row<DPP_ROW_HALF_MIRROR>(v[i], v[i + 2], lane & 4);
-    v[0] = fold_row<DPP_QUAD_SWAP2>(v[0], v[1], lane & 2);
-    return v[0] + dpp_r<DPP_QUAD_SWAP1>(v[0]);
+    const double at = a0 * w * e, guard = v1 * 0x1p-13;
+    return v1 >= tb_small<Real>() && u * v1 > (v1 - at) + guard && u * v1 < at - guard;
 }
 
 // One unit: the state of column ce is k; sample the n columns ce-1 .. ce-n
@@ -220,126 +205,91 @@ __device__ __forceinline__ int tb_unit(const DevInst &d, int b, int ce, int n, b
                                        double uw, int &pv)
 {
     constexpr int RW = 64 * R;
-    // columns whose rows are in flight at once, within about 64 registers
-    constexpr int PER = R * (int)(sizeof(Real) / 4);
-    constexpr int CB = PER >= 16 ? 2 : PER >= 8 ? 4 : 8;
     const int lane = lane_id();
     const AW_GLOBAL Real *alpha = (const AW_GLOBAL Real *)d.alpha;
-    const AW_GLOBAL int *info = gp(d.linfo) + (size_t)b * RW;
+    const AW_GLOBAL Real *pl = planes<Real>(d, b, RW);
     const int S = cp(d.soff)[b + 1] - cp(d.soff)[b];
-    const float uf = (float)uw;
+    // lane j: the transition from column ce-1-j to the next, the switch last
+    const int c = max(ce - 1 - min(lane, n), 0);
+    const double norm = gp(d.norms)[c + 1];
+    const int cls = gp(d.cls)[c + 1];
+    // FP32: a column that is not the recursion of the one stored before it
+    bool cut = false;
+    if (sizeof(Real) == 4) cut = gp(d.cut)[(c + 1) >> 5] >> ((c + 1) & 31) & 1;
+    // emission of state position p in column c + 1
+    auto emission = [&](int p) -> double {
+        double e = 1.0;
+        if (cls == -1) e = pl[CE * RW + p];
+        if (cls >= 0) e = gp(d.vemit)[(size_t)cls * RW + p];
+        return e;
+    };
     pv = k;
     int pos = 0;
     while (pos < n) {
-        // weights into k, in FP32 for the tests
         const Target<Real> t = tb_target<Real, R>(d, b, k);
-        float tf[R], tk[R];
-        {
+        const int pk = lane_pos(k, R);
+        const double a0 = alpha[(size_t)c * RW + pk], a1 = alpha[(size_t)(c + 1) * RW + pk];
+        const bool stay = !cut && tb_certain<Real>(a0, readlane_r(t.tab, 32 + t.time), a1 * norm,
+                                                   emission(pk), uw);
+        unsigned long long odd = __ballot(lane >= pos && lane < n && !stay);
+        pos = n;
+        while (odd) {
+            const int x = (int)__ffsll((long long)odd) - 1;
+            Real rv[R], tr[R];
             int ti[R];
-            slots_load<R>(info, lane, ti);
-            Real tr[R];
+            row_load<Real, R>(alpha, ce - 1 - x, rv);
+            slots_load<R>((const AW_GLOBAL int *)gp(d.linfo) + (size_t)b * RW, lane, ti);
             tb_weights<Real, R>(d, ti, t, tr);
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                tf[r] = (float)tr[r];
-                tk[r] = readlane_r(tf[r], t.lk);   // the states of k's lane
+            const int kn = sample_state<Real, R>(rv, tr, S, readlane_d(uw, x));
+            if (kn != k) {
+                k = kn;
+                pv = lane >= x ? k : pv;
+                pos = x + 1;
+                break;
             }
-        }
-        bool moved = false;
-        for (; pos < n && !moved; ) {
-            // lane's column of this chunk, and the entries of k's lane there:
-            // the states before k in its lane, and k itself
-            const int j = pos + (lane >> 2);
-            const AW_GLOBAL Real *grow = alpha + (size_t)(ce - 1 - min(j, n - 1)) * RW;
-            Real gv[R];
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                if (r <= t.rk) gv[r] = grow[slot_pos(r, t.lk, R)];
-            // columns c and c + 8 together, so that their first fold follows
-            // at once; value 2c is column c's total, 2c + 1 its sum over the
-            // lanes before k's
-            float v[16];
-#pragma unroll
-            for (int c0 = 0; c0 < 8; c0 += CB / 2) {
-                if (pos + c0 >= n) {
-#pragma unroll
-                    for (int c = 0; c < CB; c++) v[2 * c0 + c] = 0.f;
-                    continue;
-                }
-                Real rv[CB][R];
-#pragma unroll
-                for (int c = 0; c < CB; c++)
-                    row_load<Real, R>(alpha, ce - 1 - min(pos + c0 + c / 2 + (c & 1) * 8, n - 1), rv[c]);
-#pragma unroll
-                for (int c = 0; c < CB; c += 2) {
-                    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-                    for (int r = 0; r < R; r++) {
-                        s0 += (float)rv[c][r] * tf[r];
-                        s1 += (float)rv[c + 1][r] * tf[r];
-                    }
-                    v[2 * (c0 + c / 2)] = fold32(s0, s1);
-                    v[2 * (c0 + c / 2) + 1] =
-                        fold32(lane < t.lk ? s0 : 0.f, lane < t.lk ? s1 : 0.f);
-                }
-            }
-            const float own = sum32(v), oth = dpp_r<DPP_QUAD_SWAP2>(own);
-            const float tot = (lane & 2) ? oth : own;
-            float below = (lane & 2) ? own : oth, at = 0.f;
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                if (r < t.rk) below += (float)gv[r] * tk[r];
-                else if (r == t.rk) at = (float)gv[r] * tk[r];
-            }
-            const float pick = bperm_r(uf, 4 * min(j, 63)) * tot, guard = tot * 0x1p-13f;
-            const bool stay = pick > below + guard && pick < below + at - guard;
-            unsigned long long odd = __ballot(j < n && !stay);
-            while (odd) {
-                const int x = pos + (((int)__ffsll((long long)odd) - 1) >> 2);
-                Real rv[R], tr[R];
-                int ti[R];
-                row_load<Real, R>(alpha, ce - 1 - x, rv);
-                slots_load<R>(info, lane, ti);
-                tb_weights<Real, R>(d, ti, t, tr);
-                const int kn = sample_state<Real, R>(rv, tr, S, readlane_d(uw, x));
-                if (kn != k) {
-                    k = kn;
-                    pv = lane >= x ? k : pv;
-                    pos = x + 1;
-                    moved = true;
-                    break;
-                }
-                odd &= ~(0xfull << (4 * (x - pos)));
-            }
-            if (!moved) pos += 16;
+            odd &= odd - 1;
         }
     }
     if (sw) {
         // the switch into block b (TransMatrixSwitch::get, trans.h:201-209)
         const int rs = cp(d.srcs)[2 * b], cs = cp(d.srcs)[2 * b + 1];
-        const AW_GLOBAL Real *cn = planes<Real>(d, b, RW);
-        const AW_GLOBAL int *detn = gp(d.ldet) + (size_t)b * RW;
+        const AW_GLOBAL int *detn = (const AW_GLOBAL int *)gp(d.ldet) + (size_t)b * RW;
         const int pk = lane_pos(k, R);
-        const Real rrk = cn[CRR * RW + pk], crk = cn[CCR * RW + pk];
-        Real rv[R], tr[R], dp[R];
-        int dt[R];
-        row_load<Real, R>(alpha, ce - n - 1, rv);
-        slots_load<R>(detn, lane, dt);
-        slots_load<R>(cn + CDP * RW, lane, dp);
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int s = lane * R + r;
-            // (-1 stays no state)
-            tr[r] = (s == cs) ? crk : (s == rs) ? rrk : ((dt[r] & ~DET_SHARED) == k ? dp[r] : Real(0));
+        const Real rrk = pl[CRR * RW + pk], crk = pl[CCR * RW + pk];
+        // (-1 stays no state)
+        auto weight = [&](int s, int dt, Real dp) {
+            return (s == cs) ? crk : (s == rs) ? rrk : ((dt & ~DET_SHARED) == k ? dp : Real(0));
+        };
+        const double u = readlane_d(uw, n);
+        const int j = gp(d.pred)[(size_t)b * RW + k];
+        bool sure = false;
+        if (j != (int)TB_NONE) {
+            // (in every lane, lane n has the column's values)
+            const int pj = lane_pos(j, R);
+            const double a0 = alpha[(size_t)c * RW + pj], a1 = alpha[(size_t)(c + 1) * RW + pk];
+            sure = !cut && tb_certain<Real>(a0, weight(j, detn[pj], pl[CDP * RW + pj]), a1 * norm,
+                                            emission(pk), u);
         }
-        k = sample_state<Real, R>(rv, tr, cp(d.soff)[b] - cp(d.soff)[b - 1], readlane_d(uw, n));
+        if (__ballot(sure) >> n & 1) {
+            k = j;
+        } else {
+            Real rv[R], tr[R], dp[R];
+            int dt[R];
+            row_load<Real, R>(alpha, ce - n - 1, rv);
+            slots_load<R>(detn, lane, dt);
+            slots_load<R>(pl + CDP * RW, lane, dp);
+#pragma unroll
+            for (int r = 0; r < R; r++) tr[r] = weight(lane * R + r, dt[r], dp[r]);
+            k = sample_state<Real, R>(rv, tr, cp(d.soff)[b] - cp(d.soff)[b - 1], u);
+        }
         pv = lane >= n ? k : pv;
     }
     return k;
 }
 
 // Sample columns hi, hi-1, .., lo given the state k at column hi+1 (block
-// blk), storing the samples in dst (nothing when dst is null).  With cmp the walk stops at the first column whose sample is the
+// blk), storing the samples in dst (nothing when dst is null).  With cmp the
+// walk stops at the first column whose sample is the
 // one already stored in dst (the chains have met: the rest is that path) and
 // returns it; else it returns -1, k being the state of column lo.  The
 // uniform of column col is u[L-1-col].  Called by the whole workgroup with

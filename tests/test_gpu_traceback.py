@@ -38,3 +38,23 @@ def test_walk_matches_oracle_and_untiled(aw, k, L, T, c):
             b.run(prec, tile)
             assert np.array_equal(b.path(0), whole), (prec, tile, warm)
     aw.delete_local_trees(tr)
+
+
+@pytest.mark.parametrize("k,L,T,c", [(4, 400, 20, 10), (8, 900, 20, 200), (24, 1200, 20, 50),
+                                     (60, 900, 28, 100), (100, 600, 20, 50)])
+def test_walk_over_tile_starts(aw, k, L, T, c):
+    """FP32 tables in forward tiles with short warm-ups and loose checks, so that
+    the columns at the tiles' starts (and where a re-run rejoins) do not follow
+    from the column stored before them: the thread is the sequential sample of
+    the table as it is stored."""
+    print("traceback of tiles k=%d L=%d T=%d c=%d" % (k, L, T, c), flush=True)
+    tr, seqs, inst, model = instance(aw, k, L, 40 + k, ntimes=T, c=c)
+    u = np.random.RandomState(L + 1).uniform(size=L)
+    b = aw.Batch()
+    b.add(tr, seqs, *model, k - 1, u)
+    b.upload()
+    for tile, warm, tol in ((40, 1, 10.0), (100, 2, 0.5), (300, 4, 1e-2)):
+        for tb in (0, 128):
+            b.run(1, tb, fw_tile=tile, fw_warm=warm, fw_tol=tol)
+            assert np.array_equal(b.path(0), inst.traceback(b.alpha(0), u)), (tile, warm, tol, tb)
+    aw.delete_local_trees(tr)
