@@ -50,6 +50,7 @@
 
 #include "engine.h"
 #include "forward.h"
+#include "host_stage.h"
 #include "kernel_util.h"
 #include "traceback.h"
 
@@ -927,29 +928,61 @@ int set_lds_limit(const void *kern, size_t sh)
     return 0;
 }
 
-// Pinned host memory in two halves that table rows pass through on their way
-// out, taken when the first table is copied out (a workspace batch: with its
-// streams).
-struct HostStage {
-    static constexpr size_t HALF = size_t(2) << 20;   // bytes; a row has at most 16 KB
-    char *p = nullptr;
-    hipEvent_t filled[2];
-    int ensure()
+namespace {
+std::mutex stage_mu;
+std::vector<HostStage *> &stage_pool()
+{
+    // never destroyed (see run_instance)
+    static auto *v = new std::vector<HostStage *>();
+    return *v;
+}
+void free_stage(HostStage *s)
+{
+    for (auto &e : s->filled) (void)hipEventDestroy(e);
+    if (s->dbuf) (void)hipFree(s->dbuf);
+    (void)hipHostFree(s->p);
+    delete s;
+}
+}  // namespace
+
+HostStage *take_stage()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     {
-        if (p) return 0;
-        for (auto &e : filled) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        HIP_OK(hipHostMalloc((void **)&p, 2 * HALF, hipHostMallocDefault));
-        return 0;
+        std::lock_guard<std::mutex> lk(stage_mu);
+        auto &v = stage_pool();
+        for (size_t i = 0; i < v.size(); i++)
+            if (v[i]->dev == dev) {
+                HostStage *s = v[i];
+                v.erase(v.begin() + i);
+                return s;
+            }
     }
-    double *half(int k) const { return reinterpret_cast<double *>(p + k * HALF); }
-    void release()
+    HostStage *s = new HostStage();
+    s->dev = dev;
+    hipError_t e = hipHostMalloc((void **)&s->p, 2 * HostStage::HALF, hipHostMallocDefault);
+    int k = 0;
+    for (; k < 2 && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->filled[k], hipEventDisableTiming);
+    if (e == hipSuccess) return s;
+    fprintf(stderr, "argweaver_amd: pinned staging memory: %s\n", hipGetErrorString(e));
+    if (s->p) (void)hipHostFree(s->p);
+    delete s;
+    return nullptr;
+}
+
+void give_stage(HostStage *s)
+{
+    s->trim();
     {
-        if (!p) return;
-        for (auto &e : filled) (void)hipEventDestroy(e);
-        (void)hipHostFree(p);
-        p = nullptr;
+        std::lock_guard<std::mutex> lk(stage_mu);
+        if (stage_pool().size() < STAGE_KEEP) {
+            stage_pool().push_back(s);
+            return;
+        }
     }
-};
+    free_stage(s);
+}
 
 struct Batch::Impl {
     std::vector<HostInstance> hosts;
@@ -964,9 +997,8 @@ struct Batch::Impl {
     std::vector<int> tlist0, tlist1;   // host tile lists of the two launches
     DevBuf in, work, tab, aux, vbuf, tiles, fwb;
     Arena arena;   // base == nullptr: buffers come from hipMalloc
-    std::vector<std::vector<float>> staged32;   // FP32 planes of host-prepared instances
     Streams st;
-    HostStage stage;
+    HostStage *stage = nullptr;   // a workspace batch's own
     DevInst *dD = nullptr;
     long long *d_coloff = nullptr;
     int *d_blkoff = nullptr, *d_voff = nullptr, *d_nvar = nullptr, *d_list = nullptr;
@@ -992,7 +1024,7 @@ struct Batch::Impl {
     ~Impl()
     {
         st.destroy();
-        stage.release();
+        if (stage) give_stage(stage);
         in.release();
         work.release();
         tab.release();
@@ -1028,7 +1060,8 @@ int Batch::init_streams()
 {
     if (ctx_init()) return 1;
     if (impl_->st.create()) return 1;
-    return impl_->arena.base ? impl_->stage.ensure() : 0;
+    if (impl_->arena.base && !impl_->stage) impl_->stage = take_stage();
+    return impl_->arena.base && !impl_->stage;
 }
 
 void Batch::clear()
@@ -1109,6 +1142,9 @@ int Batch::upload()
     m.soff.assign(n, {});
     m.lnl.assign(n, 0.0);
     m.nvar.assign(n, 0);
+    const StageUse use(m.stage);
+    if (!use.s) return 1;
+    Uploader up(*use.s, c.main);
     for (int pass = 0; pass < 2; pass++) {
         Plan p;
         p.base = pass ? m.in.p : nullptr;
@@ -1154,25 +1190,25 @@ int Batch::upload()
             d.seq = p.take<char>((size_t)d.nrows * L);
             d.u = p.take<double>(L);
             if (pass == 1) {
-                hipStream_t s = c.main;
-                HIP_OK(hipMemcpyAsync((void *)d.model, &hi.model, sizeof(Model), hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.parent, ft.parent.data(), sizeof(int) * B * N, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.c0, ft.child0.data(), sizeof(int) * B * N, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.c1, ft.child1.data(), sizeof(int) * B * N, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.age, ft.age.data(), sizeof(int) * B * N, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.map, ft.mapping.data(), sizeof(int) * B * N, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.spr, ft.spr.data(), sizeof(int) * 4 * B, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.bstart, ft.start.data(), sizeof(int) * B, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.blen, ft.len.data(), sizeof(int) * B, hipMemcpyHostToDevice, s));
-                HIP_OK(hipMemcpyAsync((void *)d.soff, m.soff[i].data(), sizeof(int) * (B + 1), hipMemcpyHostToDevice, s));
+                if (up.put((void *)d.model, &hi.model, sizeof(Model))) return 1;
+                if (up.put((void *)d.parent, ft.parent.data(), sizeof(int) * B * N)) return 1;
+                if (up.put((void *)d.c0, ft.child0.data(), sizeof(int) * B * N)) return 1;
+                if (up.put((void *)d.c1, ft.child1.data(), sizeof(int) * B * N)) return 1;
+                if (up.put((void *)d.age, ft.age.data(), sizeof(int) * B * N)) return 1;
+                if (up.put((void *)d.map, ft.mapping.data(), sizeof(int) * B * N)) return 1;
+                if (up.put((void *)d.spr, ft.spr.data(), sizeof(int) * 4 * B)) return 1;
+                if (up.put((void *)d.bstart, ft.start.data(), sizeof(int) * B)) return 1;
+                if (up.put((void *)d.blen, ft.len.data(), sizeof(int) * B)) return 1;
+                if (up.put((void *)d.soff, m.soff[i].data(), sizeof(int) * (B + 1))) return 1;
                 for (int r = 0; r < d.nrows; r++)
-                    HIP_OK(hipMemcpyAsync((char *)d.seq + (size_t)r * L, hi.rows[r], L, hipMemcpyHostToDevice, s));
+                    if (up.put((char *)d.seq + (size_t)r * L, hi.rows[r], L)) return 1;
                 if (!m.us[i].empty())
-                    HIP_OK(hipMemcpyAsync((void *)d.u, m.us[i].data(), sizeof(double) * L, hipMemcpyHostToDevice, s));
+                    if (up.put((void *)d.u, m.us[i].data(), sizeof(double) * L)) return 1;
             }
         }
         if (pass == 0 && m.in.ensure(p.used + 4096)) return 1;
     }
+    if (up.flush()) return 1;
     HIP_OK(hipStreamSynchronize(c.main));
     // host rows may be released now
     for (auto &hi : m.hosts) hi.rows.clear();
@@ -1700,36 +1736,24 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     }
     // host-prepared instances: their per-block inputs, column classes and
     // variant rows (the device kernels above skipped them)
-    m.staged32.clear();
-    for (int i = 0; i < n; i++) {
-        const HostPrep *hp = m.hosts[i].prep.get();
-        if (!hp) continue;
-        const DevInst &d = m.h[i];
-        const int B = d.B, RW = 64 * d.R, T1 = d.T - 1;
-        if (fp32) {
-            m.staged32.emplace_back(hp->planes.begin(), hp->planes.end());
-            HIP_OK(hipMemcpyAsync(d.lcoef32, m.staged32.back().data(),
-                                  sizeof(float) * hp->planes.size(), hipMemcpyHostToDevice, s));
-        } else {
-            HIP_OK(hipMemcpyAsync(d.lcoef, hp->planes.data(), sizeof(double) * hp->planes.size(),
-                                  hipMemcpyHostToDevice, s));
+    if (std::any_of(m.hosts.begin(), m.hosts.end(), [](const HostInstance &hi) { return hi.prep != nullptr; })) {
+        const StageUse use(m.stage);
+        if (!use.s) return 1;
+        Uploader up(*use.s, s);
+        const auto put = [&](auto *dst, const auto &v) { return up.put(dst, v.data(), sizeof(v[0]) * v.size()); };
+        std::vector<float> planes32;
+        for (int i = 0; i < n; i++) {
+            const HostPrep *hp = m.hosts[i].prep.get();
+            if (!hp) continue;
+            const DevInst &d = m.h[i];
+            if (fp32) planes32.assign(hp->planes.begin(), hp->planes.end());
+            if (fp32 ? put(d.lcoef32, planes32) : put(d.lcoef, hp->planes)) return 1;
+            if (put(d.linfo, hp->info) || put(d.ldet, hp->det) || put(d.tm, hp->tm) ||
+                put(d.tvec, hp->tvec) || put(d.srcs, hp->srcs) || put(d.lprior, hp->prior) ||
+                put(d.cls, hp->cls) || put(d.vemit, hp->vemit))
+                return 1;
         }
-        HIP_OK(hipMemcpyAsync(d.linfo, hp->info.data(), sizeof(int) * (size_t)B * RW,
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.ldet, hp->det.data(), sizeof(int) * (size_t)B * RW,
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.tm, hp->tm.data(), sizeof(double) * (size_t)B * T1 * T1,
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.tvec, hp->tvec.data(), sizeof(double) * hp->tvec.size(),
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.srcs, hp->srcs.data(), sizeof(int) * 2 * (size_t)B,
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.lprior, hp->prior.data(), sizeof(double) * RW,
-                              hipMemcpyHostToDevice, s));
-        HIP_OK(hipMemcpyAsync(d.cls, hp->cls.data(), sizeof(int) * d.L, hipMemcpyHostToDevice, s));
-        if (hp->nvar > 0)
-            HIP_OK(hipMemcpyAsync(d.vemit, hp->vemit.data(), sizeof(double) * hp->vemit.size(),
-                                  hipMemcpyHostToDevice, s));
+        if (up.flush()) return 1;
     }
     (void)hipEventRecord(c.ev[2], s);
     if (voff[n] > 0) {
@@ -1882,23 +1906,25 @@ int Batch::copy_alpha_range(int i, int c0, int c1, double *alpha) const
     // no table before a run, or only part of one after a run that failed
     const size_t bytes = (size_t)d.L * 64 * d.R * (fp32 ? sizeof(float) : sizeof(double));
     if (!d.alpha || (char *)d.alpha + bytes > m.tab.p + m.tab.cap) return 1;
-    if (m.stage.ensure()) return 1;
+    const StageUse use(m.stage);
+    if (!use.s) return 1;
+    const HostStage &stage = *use.s;
     const int pitch = *std::max_element(Sv.begin(), Sv.end());
     const int rows = (int)(HostStage::HALF / sizeof(double) / pitch);
     const auto fill = [&](int c, int half) {
         const int n = std::min(rows, c1 - c);
         hipLaunchKernelGGL(fp32 ? k_rows_out<float> : k_rows_out<double>, dim3((n + 3) / 4),
-                           dim3(256), 0, m.st.main, d.alpha, c, n, d.R, pitch, m.stage.half(half));
+                           dim3(256), 0, m.st.main, d.alpha, c, n, d.R, pitch, stage.half(half));
         HIP_OK(hipGetLastError());
-        HIP_OK(hipEventRecord(m.stage.filled[half], m.st.main));
+        HIP_OK(hipEventRecord(stage.filled[half], m.st.main));
         return 0;
     };
     int b = 0;
     if (fill(c0, 0)) return 1;
     for (int c = c0, half = 0; c < c1; c += rows, half ^= 1) {
         if (c + rows < c1 && fill(c + rows, half ^ 1)) return 1;
-        HIP_OK(hipEventSynchronize(m.stage.filled[half]));
-        const double *row = m.stage.half(half);
+        HIP_OK(hipEventSynchronize(stage.filled[half]));
+        const double *row = stage.half(half);
         for (int x = c; x < std::min(c + rows, c1); x++, row += pitch) {
             while (ft.start[b] + ft.len[b] <= x) b++;
             memcpy(alpha, row, sizeof(double) * Sv[b]);

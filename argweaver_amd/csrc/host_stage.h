@@ -1,0 +1,129 @@
+// host_stage.h -- pinned host memory that uploads and tables pass through.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdio>
+#include <cstring>
+
+namespace aw {
+
+#define STAGE_OK(x)                                                                      \
+    do {                                                                                 \
+        hipError_t e_ = (x);                                                             \
+        if (e_ != hipSuccess) {                                                          \
+            fprintf(stderr, "argweaver_amd: %s: %s\n", #x, hipGetErrorString(e_));      \
+            return 1;                                                                    \
+        }                                                                                \
+    } while (0)
+
+// Two halves of pinned memory with an event each, of one device, and device
+// memory for a call's arrays, kept up to DEV_KEEP bytes: allocating 36 MB, the
+// copies into pages not mapped yet and freeing it cost a call 2 ms.
+struct HostStage {
+    static constexpr size_t HALF = size_t(2) << 20;   // bytes; a table row has at most 16 KB
+    static constexpr size_t DEV_KEEP = size_t(64) << 20;
+    char *p = nullptr;
+    int dev = 0;
+    hipEvent_t filled[2];
+    char *dbuf = nullptr;
+    size_t dcap = 0;
+    // device memory of n bytes, null when there is none
+    char *device(size_t n)
+    {
+        if (n > dcap) {
+            if (dbuf) (void)hipFree(dbuf);
+            dcap = 0;
+            if (hipMalloc((void **)&dbuf, n) != hipSuccess) dbuf = nullptr;
+            else dcap = n;
+        }
+        return dbuf;
+    }
+    void trim()
+    {
+        if (dcap <= DEV_KEEP) return;
+        (void)hipFree(dbuf);
+        dbuf = nullptr;
+        dcap = 0;
+    }
+    double *half(int k) const { return reinterpret_cast<double *>(p + k * HALF); }
+};
+
+// A stage for the current device, and back (engine.hip).  Up to STAGE_KEEP stages
+// are kept for later calls of any thread, more are freed when given back; their
+// user has waited for the work on them.  Null when there is no memory.
+constexpr size_t STAGE_KEEP = 8;
+HostStage *take_stage();
+void give_stage(HostStage *s);
+
+// A stage while in use; `own` is one that the caller keeps, or null.
+struct StageUse {
+    HostStage *const own, *const s;
+    explicit StageUse(HostStage *own_ = nullptr) : own(own_), s(own_ ? own_ : take_stage()) {}
+    ~StageUse()
+    {
+        if (!own && s) give_stage(s);
+    }
+    StageUse(const StageUse &) = delete;
+    StageUse &operator=(const StageUse &) = delete;
+};
+
+// Host arrays on their way to the device.  A copy from pageable memory costs the
+// caller 5-50 us, however small (the rows of 100 sequences, 100 KB each: 45 us each);
+// put() gathers arrays in pinned memory, and what lies close together on the device
+// goes in one copy of up to 2 MB, beside which the next half is filled.  The
+// arrays may be released after put().
+class Uploader {
+public:
+    Uploader(HostStage &s, hipStream_t st) : s_(s), st_(st) {}
+    ~Uploader()
+    {
+        for (int k = 0; k < 2; k++)
+            if (busy_[k]) (void)hipEventSynchronize(s_.filled[k]);
+    }
+    int put(void *dst, const void *src, size_t n)
+    {
+        char *d = static_cast<char *>(dst);
+        const char *x = static_cast<const char *>(src);
+        while (n > 0) {
+            // gaps are alignment, and go along
+            if (base_ && (d < base_ + used_ || d >= base_ + used_ + 1024 || d >= base_ + HostStage::HALF))
+                if (flush()) return 1;
+            if (!base_) {
+                if (busy_[half_]) STAGE_OK(hipEventSynchronize(s_.filled[half_]));
+                busy_[half_] = false;
+                base_ = d;
+            }
+            const size_t off = d - base_, m = std::min(n, HostStage::HALF - off);
+            memcpy(s_.p + half_ * HostStage::HALF + off, x, m);
+            used_ = off + m;
+            d += m;
+            x += m;
+            n -= m;
+        }
+        return 0;
+    }
+    // sends what is gathered
+    int flush()
+    {
+        if (!base_) return 0;
+        STAGE_OK(hipMemcpyAsync(base_, s_.p + half_ * HostStage::HALF, used_, hipMemcpyHostToDevice, st_));
+        STAGE_OK(hipEventRecord(s_.filled[half_], st_));
+        busy_[half_] = true;
+        half_ ^= 1;
+        base_ = nullptr;
+        used_ = 0;
+        return 0;
+    }
+
+private:
+    HostStage &s_;
+    hipStream_t st_;
+    char *base_ = nullptr;   // device address of the half's first byte
+    size_t used_ = 0;
+    int half_ = 0;
+    bool busy_[2] = {false, false};
+};
+
+}  // namespace aw

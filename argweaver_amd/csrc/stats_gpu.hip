@@ -25,6 +25,7 @@
 
 #include "../../include/argweaver_amd.h"
 #include "aw_math.h"
+#include "host_stage.h"
 #include "local_trees.h"
 
 namespace aw {
@@ -195,20 +196,22 @@ void tree_heights(const FlatTrees &ft, std::vector<int> &height, std::vector<int
     });
 }
 
+// The device arrays of one call in one allocation: every take() before
+// allocate() sizes it, the same calls after it place the arrays.
 struct DevBufs {
-    std::vector<void *> ptrs;
-    ~DevBufs()
+    char *base = nullptr;
+    size_t used = 0;
+    int allocate(HostStage &s)
     {
-        for (void *p : ptrs) (void)hipFree(p);
+        base = s.device(used);
+        used = 0;
+        return base == nullptr;
     }
     template <class T>
-    int alloc(T *&p, size_t n)
+    void take(T *&p, size_t n)
     {
-        void *q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return 1;
-        ptrs.push_back(q);
-        p = static_cast<T *>(q);
-        return 0;
+        p = reinterpret_cast<T *>(base + used);
+        used += (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~size_t(255);
     }
 };
 
@@ -246,23 +249,40 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
     char *drows;
     double *dlk, *dpart;
     const int nwg = (L + 255) / 256;
-    if (m.alloc(dt, ntimes) || m.alloc(dp, (size_t)B * N) || m.alloc(dc0, (size_t)B * N) ||
-        m.alloc(dc1, (size_t)B * N) || m.alloc(dag, (size_t)B * N) || m.alloc(dh, (size_t)B * N) ||
-        m.alloc(dhm, B) || m.alloc(dbs, B + 1) || m.alloc(drows, (size_t)nseqs * L) ||
-        m.alloc(dinv, L) || m.alloc(dfirst, B) || m.alloc(dlk, L) || m.alloc(dpart, nwg)) {
+    const auto place = [&] {
+        m.take(dt, ntimes);
+        m.take(dp, (size_t)B * N);
+        m.take(dc0, (size_t)B * N);
+        m.take(dc1, (size_t)B * N);
+        m.take(dag, (size_t)B * N);
+        m.take(dh, (size_t)B * N);
+        m.take(dhm, B);
+        m.take(dbs, B + 1);
+        m.take(drows, (size_t)nseqs * L);
+        m.take(dinv, L);
+        m.take(dfirst, B);
+        m.take(dlk, L);
+        m.take(dpart, nwg);
+    };
+    place();
+    const StageUse use;
+    if (!use.s) return 1;
+    if (m.allocate(*use.s)) {
         fprintf(stderr, "argweaver_amd: awamd_arg_likelihood: device allocation failed\n");
         return 1;
     }
-    LNL_OK(hipMemcpy(dt, times, sizeof(double) * ntimes, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dp, ft.parent.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dc0, ft.child0.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dc1, ft.child1.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dag, ft.age.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dh, height.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dhm, hmax.data(), sizeof(int) * B, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dbs, bstart.data(), sizeof(int) * (B + 1), hipMemcpyHostToDevice));
+    place();
+    Uploader up(*use.s, 0);
+    const size_t nodes = sizeof(int) * B * N;
+    if (up.put(dt, times, sizeof(double) * ntimes) || up.put(dp, ft.parent.data(), nodes) ||
+        up.put(dc0, ft.child0.data(), nodes) || up.put(dc1, ft.child1.data(), nodes) ||
+        up.put(dag, ft.age.data(), nodes) || up.put(dh, height.data(), nodes) ||
+        up.put(dhm, hmax.data(), sizeof(int) * B) ||
+        up.put(dbs, bstart.data(), sizeof(int) * (B + 1)))
+        return 1;
     for (int j = 0; j < nseqs; j++)
-        LNL_OK(hipMemcpy(drows + (size_t)j * L, rowp[j], L, hipMemcpyHostToDevice));
+        if (up.put(drows + (size_t)j * L, rowp[j], L)) return 1;
+    if (up.flush()) return 1;
     a.times = dt; a.parent = dp; a.c0 = dc0; a.c1 = dc1; a.age = dag; a.height = dh;
     a.hmax = dhm; a.bstart = dbs; a.rows = drows; a.invariant = dinv; a.first = dfirst;
     a.lk = dlk; a.part = dpart;
@@ -280,13 +300,15 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
 }
 
 // log P(ARG) (calc_arg_prior, src/argweaver/total_prob.cpp:262-299): a
-// term per local tree, each on a thread of its own: the probability of the
+// term per local tree, each on a wave of its own: the probability of the
 // tree's recombination-free stretch and, when a tree follows, of the SPR
-// into it (calc_spr_prob, total_prob.cpp:210-257).
+// into it (calc_spr_prob, total_prob.cpp:210-257).  The sums over nodes and time
+// steps take a lane each (on one thread per tree, 0.50 ms for 100 haplotypes x
+// 100000 columns; 0.035 so).
 struct PriorArgs {
     int B, N;
     const Model *m;
-    const int *parent, *c0, *c1, *age;   // [B*N]
+    const int *parent, *age;             // [B*N]
     const int *spr;                      // [4B] the SPR into block b
     const int *len;                      // [B]
     const int *has_next;                 // [B] a block follows before the end
@@ -294,52 +316,61 @@ struct PriorArgs {
     double *part;                        // [ceil(B/256)]
 };
 
-__device__ double spr_logprob_dev(const TreeView &t, const Model &m, int rn, int rt, int ct,
-                                  double treelen)
+__device__ double wave_sum(double x)
 {
-    const int T = m.T;
-    const int root_age = t.age[t.root];
-    const double treelen_b = treelen + m.steps[root_age];
-    Lineages L;
-    count_lineages(t, T, L);
-    L.nr[root_age]--;
-    double lnl = 0.0;
-    const int k = rt;
-    lnl += log(L.nb[k] * m.steps[k] / (L.nr[k] * treelen_b));
-    const int broken_age = t.age[t.parent[rn]];
-    const int j = ct;
-    auto rate = [&](int i) {
-        const int nb = L.nb[i / 2] - int(i / 2 < broken_age);
-        return m.csteps[i] * nb / (2.0 * m.pop[i / 2]);
-    };
-    const int ncoals_j = L.nc[j] - int(j <= broken_age) - int(j == broken_age);
-    lnl -= log((double)ncoals_j);
-    if (j < T - 2) lnl += log(1.0 - exp(-rate(2 * j) - (j > k ? rate(2 * j - 1) : 0.0)));
-    for (int x = 2 * k; x < 2 * j - 1; x++) lnl -= rate(x);
-    return lnl;
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    return x;
 }
 
-__global__ __launch_bounds__(256) void k_prior_block(PriorArgs a)
+__global__ __launch_bounds__(64) void k_prior_block(PriorArgs a)
 {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= a.B) return;
-    const int N = a.N;
-    const int *par = a.parent + (size_t)b * N;
-    int root = 0;
-    while (par[root] != -1) root++;
-    const TreeView t{N, root, par, a.c0 + (size_t)b * N, a.c1 + (size_t)b * N,
-                     a.age + (size_t)b * N};
+    __shared__ int nb[MAXT], nr[MAXT], nc[MAXT];
+    const int b = blockIdx.x, lane = threadIdx.x, N = a.N;
+    const int *par = a.parent + (size_t)b * N, *age = a.age + (size_t)b * N;
     const Model &m = *a.m;
-    const double treelen = tree_length(t, m.times);
-    const double rr = fmax(m.rho * treelen, m.rho);
-    double v;
-    if (a.has_next[b]) {
-        const int *sp = a.spr + 4 * (size_t)(b + 1);
-        v = log(rr) - rr * a.len[b] + spr_logprob_dev(t, m, sp[0], sp[1], sp[3], treelen);
-    } else {
-        v = -rr * a.len[b];
+    const int T = m.T;
+    const bool spr = a.has_next[b];   // uniform over the wave
+    for (int i = lane; i < T; i += 64) nb[i] = nr[i] = nc[i] = 0;
+    __syncthreads();
+    // tree length without the basal stub; the lineage counts (count_lineages)
+    double len = 0.0;
+    int root = N;
+    for (int i = lane; i < N; i += 64) {
+        const int p = par[i], page = p == -1 ? T - 2 : age[p];
+        if (p == -1) root = min(root, i);
+        else len += m.times[page] - m.times[age[i]];
+        if (!spr) continue;
+        for (int j = age[i]; j < page; j++) {
+            atomicAdd(&nb[j], 1);
+            atomicAdd(&nr[j], 1);
+            atomicAdd(&nc[j], 1);
+        }
+        atomicAdd(&nr[page], 1);
+        atomicAdd(&nc[page], 1);
+        if (p == -1) atomicAdd(&nb[page], 1);
     }
-    a.term[b] = v;
+    for (int off = 32; off > 0; off >>= 1) root = min(root, __shfl_xor(root, off));
+    __syncthreads();
+    const double treelen = wave_sum(len), rr = fmax(m.rho * treelen, m.rho);
+    double v = -rr * a.len[b];
+    if (spr) {
+        const int *sp = a.spr + 4 * (size_t)(b + 1);
+        const int rn = sp[0], k = sp[1], j = sp[3];
+        const int root_age = age[root], broken_age = age[par[rn]];
+        const auto rate = [&](int i) {
+            const int n = (i / 2 == T - 1 ? 1 : nb[i / 2]) - int(i / 2 < broken_age);
+            return m.csteps[i] * n / (2.0 * m.pop[i / 2]);
+        };
+        // the coalescence rates passed on the way from k up to j
+        double passed = 0.0;
+        for (int x = 2 * k + lane; x < 2 * j - 1; x += 64) passed += rate(x);
+        v += log(rr) - wave_sum(passed);
+        v += log(nb[k] * m.steps[k] /
+                 ((nr[k] - int(k == root_age)) * (treelen + m.steps[root_age])));
+        v -= log((double)(nc[j] - int(j <= broken_age) - int(j == broken_age)));
+        if (j < T - 2) v += log(1.0 - exp(-rate(2 * j) - (j > k ? rate(2 * j - 1) : 0.0)));
+    }
+    if (lane == 0) a.term[b] = v;
 }
 
 __global__ __launch_bounds__(256) void k_sum_terms(const double *term, int n, double *part)
@@ -368,25 +399,36 @@ int arg_logprior_device(const ArgTrees &tr, const Model &model, double *out)
     }
     DevBufs m;
     Model *dm;
-    int *dp, *dc0, *dc1, *dag, *dspr, *dlen, *dnext;
+    int *dp, *dag, *dspr, *dlen, *dnext;
     double *dterm, *dpart;
     const int nwg = (B + 255) / 256;
-    if (m.alloc(dm, 1) || m.alloc(dp, (size_t)B * N) || m.alloc(dc0, (size_t)B * N) ||
-        m.alloc(dc1, (size_t)B * N) || m.alloc(dag, (size_t)B * N) || m.alloc(dspr, 4 * (size_t)B) ||
-        m.alloc(dlen, B) || m.alloc(dnext, B) || m.alloc(dterm, B) || m.alloc(dpart, nwg)) {
+    const auto place = [&] {
+        m.take(dm, 1);
+        m.take(dp, (size_t)B * N);
+        m.take(dag, (size_t)B * N);
+        m.take(dspr, 4 * (size_t)B);
+        m.take(dlen, B);
+        m.take(dnext, B);
+        m.take(dterm, B);
+        m.take(dpart, nwg);
+    };
+    place();
+    const StageUse use;
+    if (!use.s) return 1;
+    if (m.allocate(*use.s)) {
         fprintf(stderr, "argweaver_amd: awamd_arg_prior: device allocation failed\n");
         return 1;
     }
-    LNL_OK(hipMemcpy(dm, &model, sizeof(Model), hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dp, ft.parent.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dc0, ft.child0.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dc1, ft.child1.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dag, ft.age.data(), sizeof(int) * B * N, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dspr, ft.spr.data(), sizeof(int) * 4 * B, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dlen, ft.len.data(), sizeof(int) * B, hipMemcpyHostToDevice));
-    LNL_OK(hipMemcpy(dnext, has_next.data(), sizeof(int) * B, hipMemcpyHostToDevice));
-    PriorArgs a{B, N, dm, dp, dc0, dc1, dag, dspr, dlen, dnext, dterm, dpart};
-    hipLaunchKernelGGL(k_prior_block, dim3(nwg), dim3(256), 0, 0, a);
+    place();
+    Uploader up(*use.s, 0);
+    const size_t nodes = sizeof(int) * B * N;
+    if (up.put(dm, &model, sizeof(Model)) || up.put(dp, ft.parent.data(), nodes) ||
+        up.put(dag, ft.age.data(), nodes) || up.put(dspr, ft.spr.data(), sizeof(int) * 4 * B) ||
+        up.put(dlen, ft.len.data(), sizeof(int) * B) ||
+        up.put(dnext, has_next.data(), sizeof(int) * B) || up.flush())
+        return 1;
+    PriorArgs a{B, N, dm, dp, dag, dspr, dlen, dnext, dterm, dpart};
+    hipLaunchKernelGGL(k_prior_block, dim3(B), dim3(64), 0, 0, a);
     hipLaunchKernelGGL(k_sum_terms, dim3(nwg), dim3(256), 0, 0, (const double *)dterm, B, dpart);
     LNL_OK(hipGetLastError());
     std::vector<double> part(nwg);
