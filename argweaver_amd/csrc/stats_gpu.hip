@@ -44,8 +44,7 @@ struct LnlArgs {
     int B, N, L, nrows, nleaves;
     double mintime, mu;
     const double *times;            // [T]
-    const int *parent, *c0, *c1, *age, *height;   // [B*N]
-    const int *hmax;                // [B] largest node height of the tree
+    const int *parent, *c0, *c1, *age;            // [B*N]
     const int *bstart;              // [B+1] column of each tree's start, then L
     const char *rows;               // [nrows*L]: row j is leaf j's sequence
     int *invariant;                 // [L]
@@ -95,6 +94,7 @@ __global__ __launch_bounds__(64) void k_lnl_eval(LnlArgs a)
 {
     __shared__ double inner[LNL_MAXN][4];
     __shared__ double mut[LNL_MAXN], nomut[LNL_MAXN];
+    __shared__ int hg[LNL_MAXN];   // node heights: leaves 0, a node one more than its higher child
     const int c = blockIdx.x, lane = threadIdx.x;
     const int b = owner_block(a.bstart, a.B, c);
     // an invariant column other than its tree's first takes that one's value
@@ -102,10 +102,16 @@ __global__ __launch_bounds__(64) void k_lnl_eval(LnlArgs a)
     const int N = a.N;
     const int *par = a.parent + (size_t)b * N, *ch0 = a.c0 + (size_t)b * N;
     const int *ch1 = a.c1 + (size_t)b * N, *ag = a.age + (size_t)b * N;
-    const int *hg = a.height + (size_t)b * N;
     int root = -1;
+    for (int i = lane; i < N; i += 64) hg[i] = 0;
+    __syncthreads();
     for (int i = lane; i < N; i += 64) {
         const int p = par[i];
+        // every leaf raises its ancestors to their distance from it
+        if (ch0[i] == -1) {
+            int h = 1;
+            for (int q = p; q != -1 && h <= N; q = par[q]) atomicMax(&hg[q], h++);
+        }
         if (p == -1) {
             root = i;
             mut[i] = nomut[i] = 0.0;
@@ -118,7 +124,7 @@ __global__ __launch_bounds__(64) void k_lnl_eval(LnlArgs a)
     // the root's index from whichever lane found it
     for (int off = 32; off > 0; off >>= 1) root = max(root, __shfl_xor(root, off));
     __syncthreads();
-    const int H = a.hmax[b];
+    const int H = hg[root];
     for (int h = 0; h <= H; h++) {
         for (int i = lane; i < N; i += 64) {
             if (hg[i] != h) continue;
@@ -164,38 +170,6 @@ __global__ __launch_bounds__(256) void k_lnl_sum(LnlArgs a)
     if (threadIdx.x == 0) a.part[blockIdx.x] = s[0];
 }
 
-// node heights (leaves 0, a node one more than its higher child) of every
-// tree, and each tree's largest
-void tree_heights(const FlatTrees &ft, std::vector<int> &height, std::vector<int> &hmax)
-{
-    const int B = ft.nblocks, N = ft.nnodes;
-    height.assign((size_t)B * N, 0);
-    hmax.assign(B, 0);
-    parallel_ranges(B, [&](int lo, int hi) {
-        std::vector<int> pending(N);
-        std::vector<int> ready;
-        for (int b = lo; b < hi; b++) {
-            const int *par = &ft.parent[(size_t)b * N], *ch0 = &ft.child0[(size_t)b * N];
-            int *h = &height[(size_t)b * N];
-            ready.clear();
-            for (int i = 0; i < N; i++) {
-                pending[i] = ch0[i] == -1 ? 0 : 2;
-                if (!pending[i]) ready.push_back(i);
-            }
-            int top = 0;
-            for (size_t k = 0; k < ready.size(); k++) {
-                const int i = ready[k];
-                top = std::max(top, h[i]);
-                const int p = par[i];
-                if (p == -1) continue;
-                h[p] = std::max(h[p], h[i] + 1);
-                if (--pending[p] == 0) ready.push_back(p);
-            }
-            hmax[b] = top;
-        }
-    });
-}
-
 // The device arrays of one call in one allocation: every take() before
 // allocate() sizes it, the same calls after it place the arrays.
 struct DevBufs {
@@ -230,8 +204,6 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
         fprintf(stderr, "argweaver_amd: awamd_arg_likelihood: %d nodes (limit %d)\n", N, LNL_MAXN);
         return 1;
     }
-    std::vector<int> height, hmax;
-    tree_heights(ft, height, hmax);
     std::vector<int> bstart(B + 1);
     for (int b = 0; b < B; b++) bstart[b] = ft.start[b];
     bstart[B] = L;
@@ -245,7 +217,7 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
     a.mintime = times[1] * .1;
     a.mu = mu;
     double *dt;
-    int *dp, *dc0, *dc1, *dag, *dh, *dhm, *dbs, *dinv, *dfirst;
+    int *dp, *dc0, *dc1, *dag, *dbs, *dinv, *dfirst;
     char *drows;
     double *dlk, *dpart;
     const int nwg = (L + 255) / 256;
@@ -255,8 +227,6 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
         m.take(dc0, (size_t)B * N);
         m.take(dc1, (size_t)B * N);
         m.take(dag, (size_t)B * N);
-        m.take(dh, (size_t)B * N);
-        m.take(dhm, B);
         m.take(dbs, B + 1);
         m.take(drows, (size_t)nseqs * L);
         m.take(dinv, L);
@@ -276,15 +246,13 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
     const size_t nodes = sizeof(int) * B * N;
     if (up.put(dt, times, sizeof(double) * ntimes) || up.put(dp, ft.parent.data(), nodes) ||
         up.put(dc0, ft.child0.data(), nodes) || up.put(dc1, ft.child1.data(), nodes) ||
-        up.put(dag, ft.age.data(), nodes) || up.put(dh, height.data(), nodes) ||
-        up.put(dhm, hmax.data(), sizeof(int) * B) ||
+        up.put(dag, ft.age.data(), nodes) ||
         up.put(dbs, bstart.data(), sizeof(int) * (B + 1)))
         return 1;
     for (int j = 0; j < nseqs; j++)
         if (up.put(drows + (size_t)j * L, rowp[j], L)) return 1;
     if (up.flush()) return 1;
-    a.times = dt; a.parent = dp; a.c0 = dc0; a.c1 = dc1; a.age = dag; a.height = dh;
-    a.hmax = dhm; a.bstart = dbs; a.rows = drows; a.invariant = dinv; a.first = dfirst;
+    a.times = dt; a.parent = dp; a.c0 = dc0; a.c1 = dc1; a.age = dag; a.bstart = dbs; a.rows = drows; a.invariant = dinv; a.first = dfirst;
     a.lk = dlk; a.part = dpart;
     hipLaunchKernelGGL(k_lnl_class, dim3(nwg), dim3(256), 0, 0, a);
     hipLaunchKernelGGL(k_lnl_first, dim3((B + 255) / 256), dim3(256), 0, 0, a);
