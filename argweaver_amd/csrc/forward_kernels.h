@@ -36,11 +36,52 @@ namespace aw {
 // us per column at R = 1 / 2 / 4 / 6 / 8 / 12 / 16 states per lane, one
 // instance on MI355X, switches included: FP32 0.30 0.31 0.35 0.40 0.45 0.53
 // 0.74 (one wave, 16-lane-group copies, readlane product: 0.93 0.82 0.79 0.88
-// 0.99 1.24 1.82); FP64 0.36 0.35 0.38 0.42 0.46 0.64 2.1 (1.15 0.95 1.05
+// 0.99 1.24 1.82); FP64 0.36 0.35 0.37 0.42 0.46 0.62 1.5 (1.15 0.95 1.05
 // 1.12 1.30 1.67 2.74).  Both waves run the columns between two events (block
 // ends, variant columns, windows of 64) in a loop of their own: with the tests
 // for events in every column it was 0.44 0.41 0.39 0.45 0.52 0.59 0.83.
 constexpr int FW_THREADS = 128;
+
+// The 0/1 factors of a lane's R states: keep(x, r) is x times factor r, add(acc,
+// x, r) is acc plus that.  A product where the factor has the table's type, a
+// select (the same value) where it is a float beside doubles, and where even
+// those would spill, one bit a state, spread over a mask for every use (open():
+// once a scan, or the compiler would keep the spread masks in registers).
+template <class Real, int R>
+struct FwFactors {
+    using Fac = std::conditional_t<(sizeof(Real) * R <= 64), Real, float>;
+    Fac f[R];
+    __device__ __forceinline__ void set(int r, bool on) { f[r] = on ? Fac(1) : Fac(0); }
+    __device__ __forceinline__ const FwFactors &open() const { return *this; }
+    __device__ __forceinline__ Real keep(Real x, int r) const
+    {
+        if constexpr (sizeof(Real) == sizeof(Fac)) return x * f[r];
+        else return (f[r] != Fac(0)) ? x : Real(0);
+    }
+    __device__ __forceinline__ Real add(Real acc, Real x, int r) const
+    {
+        if constexpr (sizeof(Real) == sizeof(Fac)) return fma(x, f[r], acc);
+        else return acc + ((f[r] != Fac(0)) ? x : Real(0));
+    }
+};
+template <class Real, int R>
+struct FwBits {
+    unsigned m = 0;
+    __device__ __forceinline__ void set(int r, bool on) { m |= on ? 1u << r : 0u; }
+    __device__ __forceinline__ FwBits open() const
+    {
+        FwBits x = *this;
+        asm volatile("" : "+v"(x.m));
+        return x;
+    }
+    __device__ __forceinline__ Real keep(Real x, int r) const
+    {
+        const int k = (int)(m << (31 - r)) >> 31;
+        if constexpr (sizeof(Real) == 4) return __int_as_float(__float_as_int(x) & k);
+        else return __hiloint2double(__double2hiint(x) & k, __double2loint(x) & k);
+    }
+    __device__ __forceinline__ Real add(Real acc, Real x, int r) const { return acc + keep(x, r); }
+};
 
 // Per block, each lane of the lanes wave keeps in registers the factor planes
 // of its R states, two 0/1 factors per state (not the first / not the last
@@ -48,33 +89,18 @@ constexpr int FW_THREADS = 128;
 // products from the lane's start / end (whether the carry reaches the state),
 // and whether the lane holds a branch start / end (the carry stops there), and
 // the state's time; padding states use time bin 31, whose term is 0, so they
-// come out 0 with no mask.  The 0/1 factors have the table's type, so that
-// applying one is one instruction; in FP64 with more than 8 states per lane
-// they are floats applied as selects, for their registers.
+// come out 0 with no mask.  The 0/1 factors (FwFactors, FwBits) take a register
+// or two a state, or a bit: with 16 states per lane in FP64 the products take 2.1
+// us per column and the bits 1.5, with 32 in FP32 3.9 (spilled) and 2.2; with 12 in
+// FP64 the bits cost 5 %.
 template <class Real, int R>
 struct FwLane {
     Real cf[R], cd[R], cg[R], ck[R], cj[R], ce[R];
-    using Fac = std::conditional_t<(sizeof(Real) * R <= 64), Real, float>;
-    Fac nf[R], nl[R], ff[R], fl[R];
+    std::conditional_t<(sizeof(Real) * R >= 128), FwBits<Real, R>, FwFactors<Real, R>> nf, nl, ff, fl;
     const AW_LDS Real *tf[R];   // the handed-back term of the state's time
     Real m1, m2;
     int K;           // carry steps: lanes a branch of the block spans
 };
-
-// x times a 0/1 factor m, and acc + x * m: a product where the factor has the
-// table's type, a select (the same value) where it is a float beside doubles
-template <class Real, class F>
-__device__ __forceinline__ Real keep(Real x, F m)
-{
-    if constexpr (sizeof(Real) == sizeof(F)) return x * m;
-    else return (m != F(0)) ? x : Real(0);
-}
-template <class Real, class F>
-__device__ __forceinline__ Real add_kept(Real acc, Real x, F m)
-{
-    if constexpr (sizeof(Real) == sizeof(F)) return fma(x, m, acc);
-    else return acc + ((m != F(0)) ? x : Real(0));
-}
 
 // Per-time sums are accumulated in GCOPY copies of the 32 time bins, copy
 // lane % 16 at GP[a * GCOPY + copy].  LDS takes sixteen consecutive lanes of
@@ -218,19 +244,20 @@ __device__ __forceinline__ void fw_block(const DevInst &d, int b, const Real *tv
     fw_plane<Real, R>(d, b, CJ, fl.cj);
     fw_plane<Real, R>(d, b, CE, fl.ce);
     bool first = false, last = false;
-    using Fac = typename FwLane<Real, R>::Fac;
-    Fac f1 = 1, f2 = 1;
+    bool f1 = true, f2 = true;
+    fl.nf = fl.nl = fl.ff = fl.fl = {};
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        fl.nf[r] = (info[r] & INFO_FIRST) ? Fac(0) : Fac(1);
-        fl.nl[r] = (info[r] & INFO_LAST) ? Fac(0) : Fac(1);
-        fl.ff[r] = f1 *= fl.nf[r];
+        f1 &= !(info[r] & INFO_FIRST);
+        fl.nf.set(r, !(info[r] & INFO_FIRST));
+        fl.nl.set(r, !(info[r] & INFO_LAST));
+        fl.ff.set(r, f1);
         fl.tf[r] = (const AW_LDS Real *)tv + (info[r] & INFO_TIME);
         first |= (info[r] & INFO_FIRST) != 0;
         last |= (info[r] & INFO_LAST) != 0;
     }
 #pragma unroll
-    for (int r = R - 1; r >= 0; r--) fl.fl[r] = f2 *= fl.nl[r];
+    for (int r = R - 1; r >= 0; r--) fl.fl.set(r, f2 &= !(info[r] & INFO_LAST));
     fl.m1 = first ? Real(0) : Real(1);
     fl.m2 = last ? Real(0) : Real(1);
     // the carry crosses lanes without a branch start (end): more steps than
@@ -570,11 +597,12 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
     auto scan = [&](Real (&same)[R]) {
         Real P[R], Q[R];
         Real p = Real(0), q = Real(0);
+        const auto &nf = fl.nf.open(), &nl = fl.nl.open(), &ff = fl.ff.open(), &fe = fl.fl.open();
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int t = R - 1 - r;
-            P[r] = keep(p, fl.nf[r]);
-            Q[t] = keep(q, fl.nl[t]);
+            P[r] = nf.keep(p, r);
+            Q[t] = nl.keep(q, t);
             p = fma(fl.cf[r], v[r], P[r]);
             q = fma(fl.cd[t], v[t], Q[t]);
         }
@@ -590,7 +618,7 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
         y2 = dpp_r<DPP_WAVE_SHL1>(y2);
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const Real pr = add_kept(P[r], y1, fl.ff[r]), qr = add_kept(Q[r], y2, fl.fl[r]);
+            const Real pr = ff.add(P[r], y1, r), qr = fe.add(Q[r], y2, r);
             // the last slot of a lane adds its two products in the other order
             // in FP32
             const Real two = (sizeof(Real) == 8 || r < R - 1) ? fma(fl.cg[r], pr, fl.ck[r] * qr)

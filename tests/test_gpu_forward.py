@@ -69,3 +69,8 @@ def test_table_copied_in_pieces(aw, prec):
         part = b.alpha_range(0, c0, c1, per_col)
         assert np.array_equal(part, whole[off[c0]:off[c1]])
     aw.delete_local_trees(tr)
+
+
+def test_forward_tables_of_the_largest_blocks(aw):
+    """32 states per lane: blocks of more than 1024 states."""
+    test_forward_tables(aw, 128, 150, 20, 100)
