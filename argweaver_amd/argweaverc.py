@@ -896,8 +896,8 @@ class Batch(object):
 
     def set_traceback(self, warm=256, options=3):
         """Traceback tiles of later runs: the speculative chain's warm-up
-        columns and the options per tile (1..4); the thread does not depend
-        on them."""
+        columns; options (1..4) is checked and has no effect.  The thread does
+        not depend on them."""
         if awamd_batch_set_traceback(self.ptr, int(warm), int(options)) != 0:
             raise ValueError("traceback warm-up / options out of range")
 

@@ -4,10 +4,11 @@
 // whose inputs (local trees, sequences, uniforms) are resident in HBM.
 //
 //   k_classify_b   one lane per column: masked / invariant / variant
-//   k_scan_b       one workgroup per instance: variant-column numbering
+//   k_scan_b       one workgroup per instance: variant-column numbering, the
+//                  mutation probabilities of branches by their times
 //   k_prep_b       one workgroup per local-tree block: state space, lineage
 //                  counts, TransMatrix vectors and tables, the switch matrix
-//                  from the previous block, emission terms, first-column
+//                  from the previous block, invariant emissions, first-column
 //                  prior, and the per-state coefficient planes of the
 //                  lane-run layout (engine.h)
 //   k_var_emit_b   one wave per variant column: Felsenstein partials and the
@@ -1446,8 +1447,10 @@ int Batch::tune_forward(const int *tiles, const int *warms, int ncand, double to
     return best;
 }
 
-// FP32 forward column cost (us) by states per lane: medians of the tiles of
-// the 256-instance batch (20 time points) on MI355X.  Small R pays for a
+// FP32 forward column cost (us) by states per lane that tiles are planned with:
+// medians of the tiles of the 256-instance batch (20 time points) on MI355X with
+// one wave per tile.  With two a column takes 40-45 % of it at every R, which
+// leaves the tiles' proportions, and the plan defines the FP32 tables.  Small R pays for a
 // longer carry chain of the same-branch scan, so the cost is nearly flat up
 // to R = 6.
 constexpr double FW_CREF = 0.94;

@@ -779,7 +779,7 @@ __device__ __forceinline__ void fw_instance(const DevInst d, void *lds, const Fw
 // profiles report the main forward launch on its own).  BIG: the instances
 // with 32 states per lane (blocks of 1025-2048 states) run in a symbol of
 // their own, launched over the same tiles, so that their register demand
-// (spilled to AGPRs and scratch) does not weigh on the others.
+// (AGPRs, in FP64 scratch) does not weigh on the others.
 template <class Real, int NT1, bool REDO, bool BIG>
 __global__ __launch_bounds__(FW_THREADS)
 void k_fw_all(const DevInst *__restrict__ D, const FwTile *__restrict__ tiles,

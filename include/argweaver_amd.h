@@ -364,7 +364,7 @@ LocalTrees *awamd_add_thread(LocalTrees *trees, int ntimes, const int *path, int
  * forward and traceback for all instances.  precision 0: FP64 forward table
  * (the drop-in arithmetic); precision 1: FP32 table and recursion with
  * per-column rescaling, FP64 normalisers, log-likelihood and traceback CDF.
- * The forward runs one wave per instance; the traceback runs in tiles of
+ * The forward runs one workgroup per instance; the traceback runs in tiles of
  * tile_cols columns (0: one tile per instance) with fix-up passes.
  * stats[9]: prep, emit, forward, traceback and total ms, W, variant columns,
  * traceback fix-up passes and re-sampled columns. */
@@ -398,10 +398,9 @@ int awamd_batch_run_opts(void *batch, int precision, int tile_cols, int tracebac
 int awamd_batch_run_ex(void *batch, int precision, int tile_cols, int traceback, int fixup,
                        int fw_tile, int fw_warm, double fw_tol, double *stats);
 /* Traceback tiles of later runs: warm-up columns of a tile's speculative
- * chain (default 256) and options per tile, 1 .. 4 (default 3: the
- * speculative chain and chains from the neighbouring states of its branch;
- * a tile no option fits is re-run).  The sampled thread is the same for
- * every setting.  0 on success, -1 for a value out of range. */
+ * chain (default 256).  options, 1 .. 4, is checked and has no effect (an
+ * earlier traceback kept that many chains per tile; a tile whose chain does not
+ * fit is re-run).  The sampled thread is the same for every setting.  0 on success, -1 for a value out of range. */
 int awamd_batch_set_traceback(void *batch, int warm, int options);
 /* Traceback tile length of the instances whose FP32 forward tiles are
  * re-run (their traceback runs after the forward: shorter tiles spread it
