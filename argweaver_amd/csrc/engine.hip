@@ -1002,6 +1002,7 @@ struct Batch::Impl {
     HostStage *stage = nullptr;   // a workspace batch's own
     DevInst *dD = nullptr;
     long long *d_coloff = nullptr;
+    double *d_lnl = nullptr;   // [n] the instances' log-likelihoods
     int *d_blkoff = nullptr, *d_voff = nullptr, *d_nvar = nullptr, *d_list = nullptr;
     // traceback tiles: start / end states of their chains, re-run lists and
     // results
@@ -1669,7 +1670,6 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
             d.norms = p.take<double>(L);
             d.cut = p.take<unsigned>(L / 32 + 1);
             d.path = p.take<int>(L);
-            d.lnl = p.take<double>(1);
         }
         if (pass == 0 && m.work.ensure(p.used + 4096)) return 1;
     }
@@ -1693,8 +1693,10 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         m.d_voff = p.take<int>(n + 1);
         m.d_nvar = p.take<int>(n);
         m.d_list = p.take<int>(n);
+        m.d_lnl = p.take<double>(n);
         if (pass == 0 && m.aux.ensure(p.used + 4096)) return 1;
     }
+    for (int i = 0; i < n; i++) m.h[i].lnl = m.d_lnl + i;
 
     (void)hipEventRecord(c.ev[0], s);
     HIP_OK(hipMemcpyAsync(m.d_coloff, coloff.data(), sizeof(long long) * (n + 1), hipMemcpyHostToDevice, s));
@@ -1846,8 +1848,8 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         }
     }
     (void)hipEventRecord(c.ev[5], s);
-    for (int i = 0; i < n; i++)
-        HIP_OK(hipMemcpyAsync(&m.lnl[i], m.h[i].lnl, sizeof(double), hipMemcpyDeviceToHost, s));
+    // side by side, so that they come in one copy (256 copies took 3.4 ms)
+    HIP_OK(hipMemcpyAsync(m.lnl.data(), m.d_lnl, sizeof(double) * n, hipMemcpyDeviceToHost, s));
     HIP_OK(hipStreamSynchronize(s));
     m.prec_done = opt.prec;
     float ms;
