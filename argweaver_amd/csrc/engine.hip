@@ -1483,46 +1483,17 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
     Streams &c = m.st;
     hipStream_t s = c.main;
     const size_t rsz = fp32 ? sizeof(float) : sizeof(double);
-    std::vector<FwTile> tl;
-    std::vector<int> next;   // tile index of the following tile of its instance, -1 for none
-    int nslot = 0;
+    FwPlan plan;
     const int C0 = (fp32 && opt.fw_tile > 0) ? opt.fw_tile : 0;
     const int W = std::max(opt.fw_warm, 1);
     for (int i : order) {
-        const int L = m.h[i].L;
         // tiles of C0 columns at a column cost of FW_CREF us; an instance
         // whose columns cost more gets proportionally shorter tiles, so that
         // the tiles of every instance take about the same time
         const int C = C0 ? std::max(W + W / 4, (int)(C0 * FW_CREF / fw_cost_model(m.h[i].R))) : 0;
-        if (!C || L <= C || C <= W) {
-            tl.push_back(FwTile{i, 0, 0, L, 0, -1, -1});
-            next.push_back(-1);
-            continue;
-        }
-        // tile 0: [0, C); then tiles of C - W stored columns after a warm-up
-        // of W columns
-        const int F = C - W;
-        int s0 = 0, e0 = C, prev = -1;
-        while (true) {
-            const bool last = e0 >= L;
-            const int slot = last ? -1 : nslot++;
-            FwTile t;
-            t.inst = i;
-            t.cs = s0;
-            t.c1 = std::min(e0, L);
-            t.c0 = s0 == 0 ? 0 : s0 - W;
-            t.mode = s0 == 0 ? 0 : 1;
-            t.bin = prev;
-            t.bout = slot;
-            if (!next.empty() && prev >= 0) next.back() = (int)tl.size();
-            tl.push_back(t);
-            next.push_back(-1);
-            if (last) break;
-            prev = slot;
-            s0 = e0;
-            e0 = s0 + F;
-        }
+        plan.add(i, m.h[i].L, m.h[i].R, C, W);
     }
+    const std::vector<FwTile> &tl = plan.tiles;
     const int nt = (int)tl.size();
     rs.fw_tiles = nt;
     for (int pass = 0; pass < 2; pass++) {
@@ -1530,8 +1501,8 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
         p.base = pass ? m.fwb.p : nullptr;
         m.d_fwt = p.take<FwTile>(nt);
         m.d_fwre = p.take<FwTile>(nt);
-        m.d_bnd = p.take<char>((size_t)std::max(nslot, 1) * BND_STRIDE * rsz);
-        m.d_bnorm = p.take<double>(std::max(nslot, 1));
+        m.d_bnd = p.take<char>((size_t)plan.units * BND_UNIT * rsz);
+        m.d_bnorm = p.take<double>(plan.units);
         m.d_fidx = p.take<int>(nt);
         m.d_fflag = p.take<int>(nt);
         if (pass == 0 && m.fwb.ensure(p.used + 4096)) return 1;
@@ -1556,9 +1527,7 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
     (void)hipEventRecord(c.ev[7], s);
     if (m.any_big) HIP_OK(hipStreamSynchronize(c.side));
     // tiles whose start is to be checked: those with a boundary slot in
-    std::vector<int> chk;
-    for (int k = 0; k < nt; k++)
-        if (tl[k].bin >= 0) chk.push_back(k);
+    std::vector<int> chk = plan.started();
     std::vector<int> flags;
     bool first = true;
     while (!chk.empty()) {
@@ -1581,13 +1550,7 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
         }
         if (redo.empty()) break;
         // re-run from the boundary column, then check the tiles after them
-        std::vector<FwTile> sub;
-        for (int k : redo) {
-            FwTile &t = tl[k];
-            t.mode = 2;
-            t.c0 = t.cs;
-            sub.push_back(t);
-        }
+        const std::vector<FwTile> sub = plan.rerun(redo);
         rs.fw_reruns += (int)redo.size();
         if (trace_tiles()) {
             for (int k : redo)
@@ -1597,7 +1560,6 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
         // the tile list keeps every tile's index for the checks; the re-run
         // tiles are launched from a list of their own
         const int nr = (int)sub.size();
-        HIP_OK(hipMemcpyAsync(m.d_fwt, tl.data(), sizeof(FwTile) * nt, hipMemcpyHostToDevice, s));
         HIP_OK(hipMemcpyAsync(m.d_fwre, sub.data(), sizeof(FwTile) * nr, hipMemcpyHostToDevice, s));
         if (launch_fw<float, false>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, shf, s, t1max,
                                     opt.fw_tol, m.d_fflag))
@@ -1605,14 +1567,12 @@ static int forward_stage(Batch::Impl &m, bool fp32, const BatchOptions &opt,
         if (m.any_big && launch_fw<float, true>(m.dD, m.d_fwre, nr, m.d_bnd, m.d_bnorm, m.shf_big,
                                                 s, t1max, opt.fw_tol, m.d_fflag))
             return 1;
-        // a tile that rejoined its stored columns kept its boundary column;
-        // the tile after one that ran to its end is checked again
         std::vector<int> early(nr);
         HIP_OK(hipMemcpyAsync(early.data(), m.d_fflag, sizeof(int) * nr, hipMemcpyDeviceToHost, s));
         HIP_OK(hipStreamSynchronize(s));
-        chk.clear();
-        for (int x = 0; x < nr; x++)
-            if (!early[x] && next[redo[x]] >= 0) chk.push_back(next[redo[x]]);
+        chk = plan.finished(redo, sub, early);
+        if (!chk.empty())
+            HIP_OK(hipMemcpyAsync(m.d_fwt, tl.data(), sizeof(FwTile) * nt, hipMemcpyHostToDevice, s));
         if (trace_tiles()) {
             for (int x = 0; x < nr; x++)
                 fprintf(stderr, "  inst %d tile [%d, %d): %s %d\n", sub[x].inst, sub[x].cs,

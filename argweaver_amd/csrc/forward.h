@@ -4,23 +4,9 @@
 #include <hip/hip_runtime.h>
 
 #include "engine.h"
+#include "fw_plan.h"
 
 namespace aw {
-
-// A forward tile: columns [c0, c1) of an instance computed by one workgroup.
-// mode 0 starts from the prior at column 0.  mode 1 starts at c0 from a
-// uniform vector and stores nothing before cs (a warm-up: the filter
-// forgets its start).  mode 2 starts at c0 from the column held in boundary
-// slot bin (written by the tile before).  A tile with bout >= 0 also
-// computes column c1 into boundary slot bout, for the check of the next
-// tile's start.
-struct FwTile {
-    int inst;
-    int c0, cs, c1;
-    int mode;
-    int bout, bin;
-};
-constexpr int BND_STRIDE = 64 * 32;   // Reals per boundary slot (the largest row)
 
 // LDS bytes of the forward kernel for R states per lane
 size_t fw_lds_bytes(bool fp32, int R);

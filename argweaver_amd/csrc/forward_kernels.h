@@ -459,7 +459,7 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
         if (REDO) ev = min(ev, chk);
         if (col == sp.c0) ev = col;
         AW_GLOBAL Real *row = col < sp.c1 ? alpha + (size_t)col * RW
-                                           : bnd + (size_t)sp.bout * BND_STRIDE;
+                                           : bnd + (size_t)sp.bout * BND_UNIT;
         for (;; col++, row += RW) {
             fw_barrier();
             Real x[R];
@@ -523,7 +523,8 @@ __device__ __forceinline__ void fw_sums(const DevInst &d, FwShared<Real, R> &sh,
         }
     }
     if (sp.bout >= 0 && !rejoined && lane == (col & 63)) bnorm[sp.bout] = (double)nw;
-    // the first column's own normaliser
+    // the first column's own normaliser (bnorm's slot: no tile of this launch
+    // writes it, see FwPlan)
     if (sp.c0 >= sp.cs && sp.c0 < sp.c1 && lane == 0) {
         if (sp.c0 == 0 && L > 1) norms[0] = 1.0;
         if (REDO && sp.mode == 2) norms[sp.c0] = bnorm[sp.bin];
@@ -577,7 +578,7 @@ __device__ __forceinline__ void fw_lanes(const DevInst &d, FwShared<Real, R> &sh
 #pragma unroll
         for (int r = 0; r < R; r++) v[r] = (lane * R + r < S) ? Real(1) : Real(0);
     } else {
-        const AW_GLOBAL Real *src = bnd + (size_t)sp.bin * BND_STRIDE;
+        const AW_GLOBAL Real *src = bnd + (size_t)sp.bin * BND_UNIT;
         slots_load<R>(src, lane, v);
     }
 
@@ -823,7 +824,7 @@ __global__ __launch_bounds__(64) void k_fw_check(const DevInst *__restrict__ D,
     const DevInst &d = D[t.inst];
     const int RW = 64 * d.R, lane = threadIdx.x;
     const Real *a = (const Real *)d.alpha + (size_t)t.cs * RW;
-    const Real *q = bnd + (size_t)t.bin * BND_STRIDE;
+    const Real *q = bnd + (size_t)t.bin * BND_UNIT;
     double dmax = 0.0, amax = 0.0;
     for (int x = lane; x < RW; x += 64) {
         dmax = fmax(dmax, fabs((double)a[x] - (double)q[x]));
