@@ -822,11 +822,13 @@ __global__ __launch_bounds__(256) void k_rows_out(const void *alpha, int c0, int
 // (stream synchronisation), never by a stream waiting on an event.
 struct Streams {
     bool init = false;
+    int dev = 0;   // theirs
     hipStream_t main = nullptr, side = nullptr;
     hipEvent_t ev[10];
     int create()
     {
         if (init) return 0;
+        HIP_OK(hipGetDevice(&dev));
         HIP_OK(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
         HIP_OK(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
         for (auto &e : ev) HIP_OK(hipEventCreate(&e));
@@ -1139,6 +1141,7 @@ int Batch::upload()
     Impl &m = *impl_;
     if (m.st.create()) return 1;
     Streams &c = m.st;
+    const OnDevice on(c.dev);
     const int n = (int)m.hosts.size();
     m.h.assign(n, DevInst{});
     m.soff.assign(n, {});
@@ -1401,6 +1404,7 @@ int Batch::tune_tiles(Precision prec, const int *cand, int ncand, double *ms_out
     if (run(opt)) return -1;
     Impl &m = *impl_;
     Streams &c = m.st;
+    const OnDevice on(c.dev);
     const bool fp32 = prec == Precision::FP32;
     int best = cand[0];
     float best_ms = 0;
@@ -1592,6 +1596,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     Impl &m = *impl_;
     if (!m.uploaded && upload()) return 1;
     Streams &c = m.st;
+    const OnDevice on(c.dev);
     const int n = (int)m.hosts.size();
     hipStream_t s = c.main;
     const bool fp32 = opt.prec == Precision::FP32;
@@ -1775,6 +1780,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         if (launch_chains(m, fp32, &done, 0, c.side)) return 1;
         if (opt.fixup)
             helper = std::thread([&] {
+                const OnDevice side(c.dev);
                 rc_side = resolve_tiles(m, fp32, rs_side, c.side, &done, 1);
                 (void)hipEventRecord(c.ev[8], c.side);
             });
@@ -1871,6 +1877,7 @@ int Batch::copy_alpha_range(int i, int c0, int c1, double *alpha) const
     // no table before a run, or only part of one after a run that failed
     const size_t bytes = (size_t)d.L * 64 * d.R * (fp32 ? sizeof(float) : sizeof(double));
     if (!d.alpha || (char *)d.alpha + bytes > m.tab.p + m.tab.cap) return 1;
+    const OnDevice on(m.st.dev);
     const StageUse use(m.stage);
     if (!use.s) return 1;
     const HostStage &stage = *use.s;

@@ -18,6 +18,25 @@ namespace aw {
         }                                                                                \
     } while (0)
 
+// Makes a device current while it lives: streams, events and memory of one
+// device are used together, whichever the caller has current.
+class OnDevice {
+public:
+    explicit OnDevice(int dev)
+    {
+        if (hipGetDevice(&was_) != hipSuccess || was_ == dev || hipSetDevice(dev) != hipSuccess) was_ = -1;
+    }
+    ~OnDevice()
+    {
+        if (was_ >= 0) (void)hipSetDevice(was_);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+
+private:
+    int was_ = -1;
+};
+
 // Two halves of pinned memory with an event each, of one device, and device
 // memory for a call's arrays, kept up to DEV_KEEP bytes: allocating 36 MB, the
 // copies into pages not mapped yet and freeing it cost a call 2 ms.

@@ -1,0 +1,6 @@
+"""Host side of copies and device memory, against a HIP runtime in host memory."""
+from native_check import run_check
+
+
+def test_batch_used_with_another_device_current(tmp_path):
+    run_check(tmp_path, "check_batch_device", library=True)
