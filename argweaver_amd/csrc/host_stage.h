@@ -95,6 +95,7 @@ struct StageUse {
 // arrays may be released after put().
 class Uploader {
 public:
+    static constexpr size_t ALIGN = 256;   // of the arrays put (Plan, DevBufs)
     Uploader(HostStage &s, hipStream_t st) : s_(s), st_(st) {}
     ~Uploader()
     {
@@ -106,8 +107,8 @@ public:
         char *d = static_cast<char *>(dst);
         const char *x = static_cast<const char *>(src);
         while (n > 0) {
-            // gaps are alignment, and go along
-            if (base_ && (d < base_ + used_ || d >= base_ + used_ + 1024 || d >= base_ + HostStage::HALF))
+            // gaps less than the 256 bytes that arrays are aligned to hold nothing, and go along
+            if (base_ && (d < base_ + used_ || d >= base_ + used_ + ALIGN || d >= base_ + HostStage::HALF))
                 if (flush()) return 1;
             if (!base_) {
                 if (busy_[half_]) STAGE_OK(hipEventSynchronize(s_.filled[half_]));

@@ -28,7 +28,7 @@ struct Event {
 
 inline int device = 0;
 inline int live_events = 0;
-inline int kernels = 0;
+inline int kernels = 0, copies = 0;
 inline int good_events = -1, good_launches = -1;   // calls that still succeed, -1: all
 inline size_t device_bytes = 0, device_limit = size_t(1) << 40;
 inline std::map<void *, size_t> allocated;
@@ -74,6 +74,7 @@ hipError_t hipGetLastError(void)
     fake::last = hipSuccess;
     return e;
 }
+const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "an error of the check's runtime"; }
 
 hipError_t hipMalloc(void **p, size_t n)
 {
@@ -94,6 +95,7 @@ hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
+    fake::copies++;
     return memcpy(d, s, n), hipSuccess;
 }
 

@@ -4,3 +4,7 @@ from native_check import run_check
 
 def test_batch_used_with_another_device_current(tmp_path):
     run_check(tmp_path, "check_batch_device", library=True)
+
+
+def test_uploads_leave_what_lies_between(tmp_path):
+    run_check(tmp_path, "check_uploader", library=True)
