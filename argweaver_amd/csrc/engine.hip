@@ -965,10 +965,14 @@ HostStage *take_stage()
     HostStage *s = new HostStage();
     s->dev = dev;
     hipError_t e = hipHostMalloc((void **)&s->p, 2 * HostStage::HALF, hipHostMallocDefault);
-    int k = 0;
-    for (; k < 2 && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->filled[k], hipEventDisableTiming);
+    int events = 0;
+    while (e == hipSuccess && events < 2) {
+        e = hipEventCreateWithFlags(&s->filled[events], hipEventDisableTiming);
+        if (e == hipSuccess) events++;
+    }
     if (e == hipSuccess) return s;
     fprintf(stderr, "argweaver_amd: pinned staging memory: %s\n", hipGetErrorString(e));
+    while (events > 0) (void)hipEventDestroy(s->filled[--events]);
     if (s->p) (void)hipHostFree(s->p);
     delete s;
     return nullptr;

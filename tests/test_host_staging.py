@@ -8,3 +8,7 @@ def test_batch_used_with_another_device_current(tmp_path):
 
 def test_uploads_leave_what_lies_between(tmp_path):
     run_check(tmp_path, "check_uploader", library=True)
+
+
+def test_staging_memory_not_available(tmp_path):
+    run_check(tmp_path, "check_stage_pool", library=True)
