@@ -1895,19 +1895,25 @@ int Batch::copy_alpha_range(int i, int c0, int c1, double *alpha) const
         HIP_OK(hipEventRecord(stage.filled[half], m.st.main));
         return 0;
     };
-    int b = 0;
-    if (fill(c0, 0)) return 1;
-    for (int c = c0, half = 0; c < c1; c += rows, half ^= 1) {
-        if (c + rows < c1 && fill(c + rows, half ^ 1)) return 1;
-        HIP_OK(hipEventSynchronize(stage.filled[half]));
-        const double *row = stage.half(half);
-        for (int x = c; x < std::min(c + rows, c1); x++, row += pitch) {
-            while (ft.start[b] + ft.len[b] <= x) b++;
-            memcpy(alpha, row, sizeof(double) * Sv[b]);
-            alpha += Sv[b];
+    const auto copy = [&] {
+        int b = 0;
+        if (fill(c0, 0)) return 1;
+        for (int c = c0, half = 0; c < c1; c += rows, half ^= 1) {
+            if (c + rows < c1 && fill(c + rows, half ^ 1)) return 1;
+            HIP_OK(hipEventSynchronize(stage.filled[half]));
+            const double *row = stage.half(half);
+            for (int x = c; x < std::min(c + rows, c1); x++, row += pitch) {
+                while (ft.start[b] + ft.len[b] <= x) b++;
+                memcpy(alpha, row, sizeof(double) * Sv[b]);
+                alpha += Sv[b];
+            }
         }
-    }
-    return 0;
+        return 0;
+    };
+    if (!copy()) return 0;
+    // a kernel may still write to the staging memory, which is given back
+    (void)hipStreamSynchronize(m.st.main);
+    return 1;
 }
 
 int Batch::copy_alpha(int i, double *alpha) const

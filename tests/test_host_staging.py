@@ -12,3 +12,7 @@ def test_uploads_leave_what_lies_between(tmp_path):
 
 def test_staging_memory_not_available(tmp_path):
     run_check(tmp_path, "check_stage_pool", library=True)
+
+
+def test_table_copy_that_fails(tmp_path):
+    run_check(tmp_path, "check_table_error", library=True)
