@@ -21,9 +21,10 @@ int main()
         REQUIRE(fake::pending() == 0);
     }
     fake::good_launches = -1;
+    const std::vector<double> before = table;
     std::fill(table.begin(), table.end(), 1.0);
     REQUIRE(awamd_batch_alpha(b, 0, table.data()) == 0);
-    for (double x : table) REQUIRE(x == 0.0);
+    REQUIRE(table == before);
     awamd_batch_free(b);
     printf("ok\n");
 }
