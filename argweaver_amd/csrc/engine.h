@@ -248,6 +248,9 @@ int run_instance(const HostInstance &hi, const double *u, int *path, double *alp
 // states per block); else 1, with the reason in msg.
 int instance_supported(const HostInstance &hi, std::string *msg = nullptr);
 
+// Device bytes of an instance's arrays in a batch, with nvar variant columns.
+size_t instance_bytes(const HostInstance &hi, Precision prec, int nvar);
+
 // Bytes of the fixed per-GPU workspace of run_instance_noalloc.
 constexpr size_t kNoAllocBytes = size_t(64) << 20;
 

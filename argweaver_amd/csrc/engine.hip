@@ -1137,6 +1137,94 @@ int Batch::add(HostInstance &&hin, const double *u, const double *prior)
     return (int)m.hosts.size() - 1;
 }
 
+// an instance's sizes, Sv its states per block
+static int shape_instance(const HostInstance &hi, const std::vector<int> &Sv, DevInst &d)
+{
+    const FlatTrees &ft = hi.ft;
+    d.hostprep = hi.prep ? 1 : 0;
+    d.last_state = hi.last_state;
+    d.T = hi.model.T; d.N = ft.nnodes; d.B = ft.nblocks; d.L = ft.seqlen;
+    d.nrows = (int)hi.rows.size();
+    d.Smax = 1;
+    for (int S : Sv) d.Smax = std::max(d.Smax, S);
+    d.R = lanes_per_state_r(d.Smax);
+    if (d.R > 0) return 0;
+    fprintf(stderr, "argweaver_amd: %d states per block exceed the %d of one wave\n", d.Smax,
+            64 * RVALS[NRV - 1]);
+    return 1;
+}
+
+// An instance's device arrays: what is uploaded, what a run fills, its forward
+// table, and its variant rows, whose number a run finds.  instance_bytes adds
+// the same plans up.
+static void plan_inputs(Plan &p, DevInst &d)
+{
+    const int B = d.B, N = d.N, L = d.L;
+    d.model = p.take<Model>(1);
+    d.parent = p.take<int>((size_t)B * N);
+    d.c0 = p.take<int>((size_t)B * N);
+    d.c1 = p.take<int>((size_t)B * N);
+    d.age = p.take<int>((size_t)B * N);
+    d.map = p.take<int>((size_t)B * N);
+    d.spr = p.take<int>(4 * (size_t)B);
+    d.bstart = p.take<int>(B);
+    d.blen = p.take<int>(B);
+    d.soff = p.take<int>(B + 1);
+    d.seq = p.take<char>((size_t)d.nrows * L);
+    d.u = p.take<double>(L);
+}
+
+static void plan_work(Plan &p, DevInst &d, bool fp32)
+{
+    const int B = d.B, N = d.N, L = d.L, T1 = d.T - 1, RW = 64 * d.R;
+    d.vflag = p.take<int>(L);
+    d.cls = p.take<int>(L);
+    d.vcol = p.take<int>(L);
+    d.order = p.take<int>((size_t)B * N);
+    d.roots = p.take<int>(B);
+    d.pmut = p.take<double>(mut_entry(d.T + 1, 0, d.T));
+    d.tm = p.take<double>((size_t)B * T1 * T1);
+    d.tvec = p.take<double>((size_t)B * time_vecs(T1));
+    d.srcs = p.take<int>(2 * (size_t)B);
+    d.linfo = p.take<int>((size_t)B * RW);
+    // coefficient planes in the run's precision only
+    d.fp32 = fp32 ? 1 : 0;
+    d.lcoef = fp32 ? nullptr : p.take<double>((size_t)B * NCOEF * RW);
+    d.lcoef32 = fp32 ? p.take<float>((size_t)B * NCOEF * RW) : nullptr;
+    d.ldet = p.take<int>((size_t)B * RW);
+    d.pred = p.take<unsigned short>((size_t)B * RW);
+    d.lprior = p.take<double>(RW);
+    d.norms = p.take<double>(L);
+    d.cut = p.take<unsigned>(L / 32 + 1);
+    d.path = p.take<int>(L);
+}
+
+static void plan_table(Plan &p, DevInst &d)
+{
+    d.alpha = p.take<char>((size_t)d.L * 64 * d.R * (d.fp32 ? sizeof(float) : sizeof(double)));
+}
+
+static void plan_variants(Plan &p, DevInst &d)
+{
+    d.vemit = p.take<double>((size_t)std::max(d.nvar, 1) * 64 * d.R);
+}
+
+size_t instance_bytes(const HostInstance &hi, Precision prec, int nvar)
+{
+    DevInst d{};
+    std::vector<int> Sv;
+    if (hi.prep) Sv = hi.prep->S;
+    else instance_states(hi.ft, hi.model.T, &Sv);
+    if (shape_instance(hi, Sv, d)) return 0;
+    d.nvar = nvar;
+    Plan p;
+    plan_inputs(p, d);
+    plan_work(p, d, prec == Precision::FP32);
+    plan_table(p, d);
+    plan_variants(p, d);
+    return p.used;
+}
+
 // Inputs: trees, sequences, uniforms and the model of every instance.
 int Batch::upload()
 {
@@ -1170,34 +1258,11 @@ int Batch::upload()
                 }
                 std::vector<int> &so = m.soff[i];
                 so.assign(B + 1, 0);
-                int Smax = 1;
-                for (int b = 0; b < B; b++) {
-                    so[b + 1] = so[b] + m.Sv[i][b];
-                    Smax = std::max(Smax, m.Sv[i][b]);
-                }
-                const int R = lanes_per_state_r(Smax);
-                if (R < 0) {
-                    fprintf(stderr, "argweaver_amd: %d states per block exceed the %d of one wave\n",
-                            Smax, 64 * RVALS[NRV - 1]);
-                    return 1;
-                }
-                d.hostprep = hi.prep ? 1 : 0;
-                d.last_state = hi.last_state;
-                d.T = T; d.N = N; d.B = B; d.L = L; d.nrows = (int)hi.rows.size();
-                d.Smax = Smax; d.W = m.W[i]; d.R = R;
+                for (int b = 0; b < B; b++) so[b + 1] = so[b] + m.Sv[i][b];
+                if (shape_instance(hi, m.Sv[i], d)) return 1;
+                d.W = m.W[i];
             }
-            d.model = p.take<Model>(1);
-            d.parent = p.take<int>((size_t)B * N);
-            d.c0 = p.take<int>((size_t)B * N);
-            d.c1 = p.take<int>((size_t)B * N);
-            d.age = p.take<int>((size_t)B * N);
-            d.map = p.take<int>((size_t)B * N);
-            d.spr = p.take<int>(4 * (size_t)B);
-            d.bstart = p.take<int>(B);
-            d.blen = p.take<int>(B);
-            d.soff = p.take<int>(B + 1);
-            d.seq = p.take<char>((size_t)d.nrows * L);
-            d.u = p.take<double>(L);
+            plan_inputs(p, d);
             if (pass == 1) {
                 if (up.put((void *)d.model, &hi.model, sizeof(Model))) return 1;
                 if (up.put((void *)d.parent, ft.parent.data(), sizeof(int) * B * N)) return 1;
@@ -1604,7 +1669,6 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     const int n = (int)m.hosts.size();
     hipStream_t s = c.main;
     const bool fp32 = opt.prec == Precision::FP32;
-    const size_t rsz = fp32 ? sizeof(float) : sizeof(double);
 
     std::vector<long long> coloff(n + 1, 0);
     std::vector<int> blkoff(n + 1, 0);
@@ -1616,40 +1680,14 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
     for (int pass = 0; pass < 2; pass++) {
         Plan p;
         p.base = pass ? m.work.p : nullptr;
-        for (int i = 0; i < n; i++) {
-            DevInst &d = m.h[i];
-            const int B = d.B, N = d.N, L = d.L, T1 = d.T - 1, RW = 64 * d.R;
-            d.vflag = p.take<int>(L);
-            d.cls = p.take<int>(L);
-            d.vcol = p.take<int>(L);
-            d.order = p.take<int>((size_t)B * N);
-            d.roots = p.take<int>(B);
-            d.pmut = p.take<double>(mut_entry(d.T + 1, 0, d.T));
-            d.tm = p.take<double>((size_t)B * T1 * T1);
-            d.tvec = p.take<double>((size_t)B * time_vecs(T1));
-            d.srcs = p.take<int>(2 * (size_t)B);
-            d.linfo = p.take<int>((size_t)B * RW);
-            // coefficient planes in the run's precision only
-            d.fp32 = fp32 ? 1 : 0;
-            d.lcoef = fp32 ? nullptr : p.take<double>((size_t)B * NCOEF * RW);
-            d.lcoef32 = fp32 ? p.take<float>((size_t)B * NCOEF * RW) : nullptr;
-            d.ldet = p.take<int>((size_t)B * RW);
-            d.pred = p.take<unsigned short>((size_t)B * RW);
-            d.lprior = p.take<double>(RW);
-            d.norms = p.take<double>(L);
-            d.cut = p.take<unsigned>(L / 32 + 1);
-            d.path = p.take<int>(L);
-        }
+        for (int i = 0; i < n; i++) plan_work(p, m.h[i], fp32);
         if (pass == 0 && m.work.ensure(p.used + 4096)) return 1;
     }
     // forward tables
     for (int pass = 0; pass < 2; pass++) {
         Plan p;
         p.base = pass ? m.tab.p : nullptr;
-        for (int i = 0; i < n; i++) {
-            DevInst &d = m.h[i];
-            d.alpha = p.take<char>((size_t)d.L * 64 * d.R * rsz);
-        }
+        for (int i = 0; i < n; i++) plan_table(p, m.h[i]);
         if (pass == 0 && m.tab.ensure(p.used + 4096)) return 1;
     }
     // auxiliary arrays
@@ -1687,7 +1725,7 @@ int Batch::run(const BatchOptions &opt, RunStats *st)
         p.base = pass ? m.vbuf.p : nullptr;
         for (int i = 0; i < n; i++) {
             m.h[i].nvar = m.nvar[i];
-            m.h[i].vemit = p.take<double>((size_t)std::max(m.nvar[i], 1) * 64 * m.h[i].R);
+            plan_variants(p, m.h[i]);
             voff[i + 1] = voff[i] + m.nvar[i];
         }
         if (pass == 0 && m.vbuf.ensure(p.used + 4096)) return 1;

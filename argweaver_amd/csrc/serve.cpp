@@ -33,29 +33,13 @@ Server::~Server()
 
 double Server::now() const { return wall_seconds() - t0_; }
 
-// Mirrors the device arrays Batch::run allocates for one instance: the
-// forward table, the lane-run planes of every block, the variant rows (the
-// variant columns are counted here on the host), the per-block transition
-// tables and the per-column arrays.
+// The arrays of the instance's own (instance_bytes; the variant columns are
+// counted here on the host) and a share of a batch's tile lists.
 size_t Server::footprint(const HostInstance &hi, Precision prec)
 {
-    const FlatTrees &ft = hi.ft;
-    const int T = hi.model.T, T1 = T - 1, B = ft.nblocks, N = ft.nnodes, L = ft.seqlen;
-    std::vector<int> Sv;
-    instance_states(ft, T, &Sv);
-    int Smax = 1;
-    for (int S : Sv) Smax = std::max(Smax, S);
-    // states per lane as the kernels round it (1, 2, 4, 6, 8, 12, 16)
-    size_t R = 16;
-    for (int r : {1, 2, 4, 6, 8, 12, 16})
-        if (64 * r >= Smax) {
-            R = r;
-            break;
-        }
-    const size_t RW = 64 * R;
-    long long nvar = 0;
+    int nvar = 0;
     if (!hi.rows.empty()) {
-        for (int c = 0; c < L; c++) {
+        for (int c = 0; c < hi.ft.seqlen; c++) {
             const char x = hi.rows[0][c];
             for (size_t r = 1; r < hi.rows.size(); r++)
                 if (hi.rows[r][c] != x) {
@@ -64,14 +48,7 @@ size_t Server::footprint(const HostInstance &hi, Precision prec)
                 }
         }
     }
-    const size_t rsz = prec == Precision::FP32 ? 4 : 8;
-    size_t b = (size_t)L * RW * rsz;                          // forward table
-    b += (size_t)B * RW * (NCOEF * rsz + 4 + 4 + 2);          // planes, info, targets, sources
-    b += (size_t)std::max<long long>(nvar, 1) * RW * 8;        // variant rows
-    b += (size_t)B * ((size_t)T1 * T1 + time_vecs(T1)) * 8;    // transition tables
-    b += (size_t)B * N * (5 * 4 + 4) + (size_t)B * 12;         // trees, pruning
-    b += (size_t)L * (3 * 4 + 8 + 4 + 8 + hi.rows.size()) + L / 8;   // columns, uniforms, sequences
-    return b + (size_t)16 * 4096;
+    return instance_bytes(hi, prec, nvar) + (size_t)16 * 4096;
 }
 
 int Server::submit(const HostInstance &hi, const double *u)

@@ -7,12 +7,16 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
 #include <vector>
+
+using std::max;   // as hipcc's headers have them
+using std::min;
 
 namespace fake {
 

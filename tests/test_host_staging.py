@@ -16,3 +16,7 @@ def test_staging_memory_not_available(tmp_path):
 
 def test_table_copy_that_fails(tmp_path):
     run_check(tmp_path, "check_table_error", library=True)
+
+
+def test_server_estimate_covers_a_batch(tmp_path):
+    run_check(tmp_path, "check_footprint", library=True)
