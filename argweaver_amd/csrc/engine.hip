@@ -881,7 +881,7 @@ struct DevBuf {
         if (p) HIP_OK(hipFree(p));
         p = nullptr;
         cap = 0;
-        HIP_OK(hipMalloc(&p, n));
+        HIP_OK(device_malloc((void **)&p, n));
         cap = n;
         return 0;
     }
@@ -989,6 +989,22 @@ void give_stage(HostStage *s)
         }
     }
     free_stage(s);
+}
+
+size_t idle_stage_bytes()
+{
+    std::lock_guard<std::mutex> lk(stage_mu);
+    size_t n = 0;
+    for (const HostStage *s : stage_pool()) n += s->dcap;
+    return n;
+}
+
+bool free_idle_stage_memory()
+{
+    std::lock_guard<std::mutex> lk(stage_mu);
+    bool any = false;
+    for (HostStage *s : stage_pool()) any |= s->drop();
+    return any;
 }
 
 struct Batch::Impl {

@@ -37,6 +37,21 @@ private:
     int was_ = -1;
 };
 
+// The pool's device memory that no call uses, in bytes, and its release
+// (engine.hip): true if there was any.  A device allocation that finds no memory
+// releases it and tries again.
+size_t idle_stage_bytes();
+bool free_idle_stage_memory();
+
+// hipMalloc, with the pool's idle memory given up where memory is short
+inline hipError_t device_malloc(void **p, size_t n)
+{
+    hipError_t e = hipMalloc(p, n);
+    if (e == hipSuccess || !free_idle_stage_memory()) return e;
+    (void)hipGetLastError();   // of the first try
+    return hipMalloc(p, n);
+}
+
 // Two halves of pinned memory with an event each, of one device, and device
 // memory for a call's arrays, kept up to DEV_KEEP bytes: allocating 36 MB, the
 // copies into pages not mapped yet and freeing it cost a call 2 ms.
@@ -52,19 +67,24 @@ struct HostStage {
     char *device(size_t n)
     {
         if (n > dcap) {
-            if (dbuf) (void)hipFree(dbuf);
-            dcap = 0;
-            if (hipMalloc((void **)&dbuf, n) != hipSuccess) dbuf = nullptr;
+            drop();
+            if (device_malloc((void **)&dbuf, n) != hipSuccess) dbuf = nullptr;
             else dcap = n;
         }
         return dbuf;
     }
-    void trim()
+    // gives the device memory back; true if there was any
+    bool drop()
     {
-        if (dcap <= DEV_KEEP) return;
-        (void)hipFree(dbuf);
+        const bool any = dbuf != nullptr;
+        if (any) (void)hipFree(dbuf);
         dbuf = nullptr;
         dcap = 0;
+        return any;
+    }
+    void trim()
+    {
+        if (dcap > DEV_KEEP) drop();
     }
     double *half(int k) const { return reinterpret_cast<double *>(p + k * HALF); }
 };

@@ -5,6 +5,8 @@
 #include <chrono>
 #include <cstdio>
 
+#include "host_stage.h"
+
 namespace aw {
 
 static double wall_seconds()
@@ -49,6 +51,11 @@ size_t Server::footprint(const HostInstance &hi, Precision prec)
         }
     }
     return instance_bytes(hi, prec, nvar) + (size_t)16 * 4096;
+}
+
+size_t Server::share(const ServeOptions &opt)
+{
+    return (opt.hbm_budget - std::min(opt.hbm_budget, idle_stage_bytes())) / opt.drivers;
 }
 
 int Server::submit(const HostInstance &hi, const double *u)
@@ -105,7 +112,6 @@ void Server::worker(int index)
     // run side by side on the device
     Batch batch;
     batch.set_concurrent(true);
-    const size_t budget = opt_.hbm_budget / opt_.drivers;
     std::vector<Request *> mine;
     while (true) {
         {
@@ -114,6 +120,7 @@ void Server::worker(int index)
             if (queue_.empty()) return;   // stopping, nothing left
             // admission in arrival order while the batch fits the budget
             size_t taken = 0;
+            const size_t budget = share(opt_);
             while (!queue_.empty() && (int)mine.size() < opt_.max_batch) {
                 const size_t b = queue_.front()->bytes;
                 if (!mine.empty() && taken + b > budget) break;

@@ -64,6 +64,9 @@ public:
     double now() const;
     // Device bytes a request needs while it runs (the admission estimate).
     static size_t footprint(const HostInstance &hi, Precision prec);
+    // A driver's share of the budget, less the device memory that the staging pool
+    // holds (released only when an allocation finds none).
+    static size_t share(const ServeOptions &opt);
 
 private:
     struct Request {

@@ -20,3 +20,7 @@ def test_table_copy_that_fails(tmp_path):
 
 def test_server_estimate_covers_a_batch(tmp_path):
     run_check(tmp_path, "check_footprint", library=True)
+
+
+def test_idle_device_memory_is_given_up(tmp_path):
+    run_check(tmp_path, "check_pool_memory", library=True)
