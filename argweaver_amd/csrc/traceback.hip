@@ -148,16 +148,8 @@ __device__ __forceinline__ Target<Real> tb_target(const DevInst &d, int b, int k
     const int c = info_age(info), a = min(lane & 31, T1 - 1);
     const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * TT;
     const AW_GLOBAL double *vec = gp(d.tvec) + (size_t)b * time_vecs(T1);
-    // lanes 32 on: the same-branch entry (TransMatrix::get_time, trans.h:89-128;
-    // with the youngest age of a thread inside a subtree)
-    const int mina = (int)vec[tv_minage(T1)];
-    const AW_GLOBAL double *X = vec + tv_x(T1) + t.time;
-    const double ct = c > 0 ? X[(c - 1) * T1] : 0.0;
     const double other = tm[a * T1 + t.time];
-    double same = fma(vec[TV_D * T1 + a] * vec[TV_E * T1 + t.time],
-                      vec[TV_Y * T1 + t.time] - ct, 2 * other) +
-                  (a == t.time ? vec[TV_NORECOMBS * T1 + a] : 0.0);
-    if (a < mina || t.time < mina) same = 0.0;
+    const double same = same_entry(vec, T1, a, t.time, c, other);   // lanes 32 on
     t.tab = (Real)(lane < 32 ? other : same);
     return t;
 }
