@@ -20,8 +20,14 @@
 // the forward recursion computed the next column's entry from: entry * normaliser
 // / emission.  The state j assumed for the column has the share entry *
 // weight of it; the sums below j are unknown, but lie between 0 and the rest, so
-// a uniform that is off both ends by more than that (and 2^-13, sixty times
-// the bound on the FP32 recursion's rounding) picks j wherever j stands.
+// a uniform that is off both ends by more than that and a guard of 2^-13 picks j
+// wherever j stands.  The guard covers the FP32 recursion's rounding: its terms are
+// all positive (and its planes normal numbers), and with n = T-1 time bins an entry
+// passes at most n + 6 roundings (units of 2^-24) in the same-branch sum (planes 2,
+// running sum and carry n + 1, products 3) or 13 in the other-branch product, 3 from
+// there to the column, 3 through scale and normaliser, 1 in the row before, and 2 in
+// the products that are sampled from: n + 15, so that the guard is 60 times the bound
+// at 20 time points and 44 times at 32.
 // Only the other columns, about twice the share that is not j's, are sampled from
 // their rows, with the FP64 cumulative sums; so are those whose next column
 // was not computed from the stored one (DevInst::cut).  The columns at switches go
