@@ -393,6 +393,22 @@ def mcmc_rethread_fp32(A, seed, log, k=100, L=500000, nsteps=3):
                 fp32_error=err, arg_likelihood=lik)
 
 
+def short(x):
+    """A result with its numbers to nine digits (the line has to stay short, see trace_points)."""
+    if isinstance(x, dict):
+        return {k: short(v) for k, v in x.items()}
+    if isinstance(x, (list, tuple)):
+        return [short(v) for v in x]
+    return float("%.9g" % x) if isinstance(x, float) else x
+
+
+def trace_points(nsteps, n=4):
+    """The steps of a chain whose statistics go into the result line: n of them,
+    evenly spread, the last one included (every step's would take 22 KB at 100 steps
+    of four chains, more than a record of the line keeps)."""
+    return sorted({max(0, round(nsteps * i / n) - 1) for i in range(1, n + 1)}) if nsteps else []
+
+
 def mcmc_batched_chains(A, seed, log, nchains=4, k=100, L=500000, steps=100):
     """Config 5 as batched FP32 chains: nchains independent chains, each a
     k=100, 500k-column ARG simulated from its own seed under the same N(t).
@@ -403,8 +419,8 @@ def mcmc_batched_chains(A, seed, log, nchains=4, k=100, L=500000, steps=100):
     k-1, k-2, ..., so steps = k is one sweep re-threading every leaf of
     every chain.  Reports the time per step, the aggregate column-states/s,
     each chain's recombination count (local trees - 1), log P(seqs | ARG) and
-    log P(ARG) (computed on the device, outside the step's time) after every
-    step, and
+    log P(ARG) (computed on the device after every step, outside its time) at
+    the steps trace_points gives, and
     its log P(seqs | ARG) and log P(ARG) on the host before and after."""
     times = np.array(A.get_time_points(20, 200e3), np.float64)
     pops, rho, mu = mcmc_model(seed)
@@ -458,13 +474,16 @@ def mcmc_batched_chains(A, seed, log, nchains=4, k=100, L=500000, steps=100):
     for tr, _ in chains:
         A.delete_local_trees(tr)
     sps = float(np.mean(secs[1:])) if steps > 1 else secs[0]
+    shown = trace_points(steps)
     out = dict(chains=nchains, k=k, columns=L, steps=steps,
                leaves_rethreaded_per_chain=steps, seconds_per_step=sps,
                host_ms_per_step=float(np.mean(host_ms[1:] or host_ms)),
                batch_run_ms_per_step=float(np.mean(gpu_ms[1:] or gpu_ms)),
                column_states_per_s=float(np.mean(Ws[1:] or Ws)) / sps,
-               recombinations_trace=trace, log_likelihood_trace=lik_trace,
-               log_prior_trace=prior_trace,
+               trace_steps=[j + 1 for j in shown],
+               recombinations_trace=[trace[j] for j in shown],
+               log_likelihood_trace=[lik_trace[j] for j in shown],
+               log_prior_trace=[prior_trace[j] for j in shown],
                log_likelihood_device_vs_host_end=[
                    abs(lik_trace[-1][c] - stats1[c][0]) / abs(stats1[c][0]) for c in range(nchains)],
                log_likelihood_start=[x[0] for x in stats0], log_likelihood_end=[x[0] for x in stats1],
@@ -786,7 +805,7 @@ def main():
         "roofline": roofline,
         "cpu_baseline": cpu,
     }
-    out.update(extra)
+    out.update(short(extra))
     print(json.dumps(out))
 
 
