@@ -126,16 +126,18 @@ __host__ __device__ inline int tv_minage(int T1) { return TV_N * T1; }
 __host__ __device__ inline int tv_x(int T1) { return TV_N * T1 + 1; }
 __host__ __device__ inline int time_vecs(int T1) { return tv_x(T1) + T1 * T1; }
 // that entry (TransMatrix::get_time, trans.h:89-128, with the youngest age m of a
-// thread inside a subtree) for a branch of age c, from the block's terms and other =
-// P_other(a -> b)
+// thread inside a subtree) for a branch of age c, from the block's terms; other:
+// where P_other(a -> b) is
 template <class P>
-__host__ __device__ inline double same_entry(P vec, int T1, int a, int b, int c, double other)
+__host__ __device__ inline double same_entry(P vec, int T1, int a, int b, int c, P other)
 {
     const int mina = (int)vec[tv_minage(T1)];
-    const double ct = c > 0 ? vec[tv_x(T1) + (c - 1) * T1 + b] : 0.0;
-    const double same = fma(vec[TV_D * T1 + a] * vec[TV_E * T1 + b], vec[TV_Y * T1 + b] - ct, 2 * other) +
-                        (a == b ? vec[TV_NORECOMBS * T1 + a] : 0.0);
-    return a < mina || b < mina ? 0.0 : same;
+    const P X = vec + tv_x(T1) + b;
+    const double ct = c > 0 ? X[(c - 1) * T1] : 0.0;
+    double same = fma(vec[TV_D * T1 + a] * vec[TV_E * T1 + b], vec[TV_Y * T1 + b] - ct, 2 * *other) +
+                  (a == b ? vec[TV_NORECOMBS * T1 + a] : 0.0);
+    if (a < mina || b < mina) same = 0.0;
+    return same;
 }
 
 enum class Precision { FP64 = 0, FP32 = 1 };

@@ -154,9 +154,9 @@ __device__ __forceinline__ Target<Real> tb_target(const DevInst &d, int b, int k
     const int c = info_age(info), a = min(lane & 31, T1 - 1);
     const AW_GLOBAL double *tm = gp(d.tm) + (size_t)b * TT;
     const AW_GLOBAL double *vec = gp(d.tvec) + (size_t)b * time_vecs(T1);
-    const double other = tm[a * T1 + t.time];
-    const double same = same_entry(vec, T1, a, t.time, c, other);   // lanes 32 on
-    t.tab = (Real)(lane < 32 ? other : same);
+    const AW_GLOBAL double *other = tm + (a * T1 + t.time);
+    const double same = same_entry(vec, T1, a, t.time, c, other);
+    t.tab = (Real)(lane < 32 ? *other : same);
     return t;
 }
 

@@ -52,15 +52,15 @@ int main()
                             const auto X = [&](int x) { return x >= 0 && x < t ? vec[tv_x(T1) + x * T1 + t] : 0.0; };
                             const double M = 2 * fabs(other) + DE * (2 * vec[TV_Y * T1 + t] + 2 * X(t - 1) + X(c - 1)) +
                                              (a == t ? vec[TV_NORECOMBS * T1 + a] : 0.0);
-                            const double got = same_entry(vec, T1, a, t, c, other);
+                            const double got = same_entry(vec, T1, a, t, c, &tm[a * T1 + t]);
                             REQUIRE(fabs(got - (other + add)) <= 64 * 2.3e-16 * M);
                             entries++;
                         }
                     // no way from or to an age that no thread has
                     for (int a = 0; a < (int)vec[tv_minage(T1)]; a++)
                         for (int t = 0; t < T1; t++)
-                            REQUIRE(same_entry(vec, T1, a, t, 0, tm[a * T1 + t]) == 0.0 &&
-                                    same_entry(vec, T1, t, a, 0, tm[t * T1 + a]) == 0.0);
+                            REQUIRE(same_entry(vec, T1, a, t, 0, &tm[a * T1 + t]) == 0.0 &&
+                                    same_entry(vec, T1, t, a, 0, &tm[t * T1 + a]) == 0.0);
                 }
             }
     printf("%ld entries, %ld blocks of an age above 0\n", entries, aged);
