@@ -18,8 +18,9 @@ namespace aw {
 // Everything one threading instance keeps in HBM.  POD; an array of these
 // lives in device memory and every kernel finds its instance through it.
 //
-// Lane-run layout.  The HMM kernels run one 64-lane wave per instance (or
-// per traceback tile); lane l owns the R consecutive states l*R .. l*R+R-1
+// Lane-run layout.  Each wave of the HMM kernels that works on a column (one
+// of the two of a forward tile, every one of the 16 or 8 of a traceback tile) has
+// its states spread over 64 lanes; lane l owns the R consecutive states l*R .. l*R+R-1
 // of the node-major state order, so the states of one branch sit in one
 // lane or in neighbouring lanes.  Every per-state array is stored
 // transposed (lane_pos) in rows of RW = 64*R entries: the slots of a lane are
@@ -186,8 +187,8 @@ struct BatchOptions {
     bool traceback = true;
     bool fixup = true;       // false: speculative paths only (diagnostics)
     // FP32 forward tiles: long instances are split into tiles (counting the
-    // warm-up) of fw_tile columns at a column cost of 0.94 us, scaled by
-    // the column cost of the instance's states per lane, that run
+    // warm-up) of fw_tile columns, scaled by the planned column cost of the
+    // instance's states per lane (fw_cost_model, engine.hip), that run
     // concurrently; a tile after the first starts fw_warm columns early
     // from a uniform vector, and its start is checked against the column
     // the tile before computes (relative tolerance fw_tol), a tile that

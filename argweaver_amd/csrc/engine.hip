@@ -1539,10 +1539,10 @@ int Batch::tune_forward(const int *tiles, const int *warms, int ncand, double to
 
 // FP32 forward column cost (us) by states per lane that tiles are planned with:
 // medians of the tiles of the 256-instance batch (20 time points) on MI355X with
-// one wave per tile.  With two a column takes 40-45 % of it at every R, which
-// leaves the tiles' proportions, and the plan defines the FP32 tables.  Small R pays for a
-// longer carry chain of the same-branch scan, so the cost is nearly flat up
-// to R = 6.
+// one wave per tile.  With two a column takes 33 % of it at R = 2, 38-41 % at 4 to
+// 12 and 46 % at 16, so that an instance's tiles end up to a fifth apart from those of
+// another R; the plan stays, because it defines the FP32 tables.  Small R pays for a
+// longer carry chain of the same-branch scan, so the cost is nearly flat up to R = 6.
 constexpr double FW_CREF = 0.94;
 inline double fw_cost_model(int R)
 {

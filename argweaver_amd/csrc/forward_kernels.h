@@ -28,7 +28,7 @@ namespace aw {
 //
 // The lanes wave runs its scan while the sums wave works.  The kernel is bound
 // by the latency of that chain: hand over, atomics, their sums, the product,
-// hand back, about 900 cycles at 8 FP32 states per lane.  One wave doing both
+// hand back, about 990 cycles at 8 FP32 states per lane.  One wave doing both
 // is bound by its instruction issue (a dependent instruction every 8 cycles, an
 // independent one every 5); four waves sharing the slots out lost more to
 // atomics from several waves meeting in LDS than they gained.

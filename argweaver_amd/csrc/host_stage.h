@@ -4,19 +4,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdio>
 #include <cstring>
 
-namespace aw {
+#include "hip_check.h"
 
-#define STAGE_OK(x)                                                                      \
-    do {                                                                                 \
-        hipError_t e_ = (x);                                                             \
-        if (e_ != hipSuccess) {                                                          \
-            fprintf(stderr, "argweaver_amd: %s: %s\n", #x, hipGetErrorString(e_));      \
-            return 1;                                                                    \
-        }                                                                                \
-    } while (0)
+namespace aw {
 
 // Makes a device current while it lives: streams, events and memory of one
 // device are used together, whichever the caller has current.
@@ -131,7 +123,7 @@ public:
             if (base_ && (d < base_ + used_ || d >= base_ + used_ + ALIGN || d >= base_ + HostStage::HALF))
                 if (flush()) return 1;
             if (!base_) {
-                if (busy_[half_]) STAGE_OK(hipEventSynchronize(s_.filled[half_]));
+                if (busy_[half_]) HIP_OK(hipEventSynchronize(s_.filled[half_]));
                 busy_[half_] = false;
                 base_ = d;
             }
@@ -148,8 +140,8 @@ public:
     int flush()
     {
         if (!base_) return 0;
-        STAGE_OK(hipMemcpyAsync(base_, s_.p + half_ * HostStage::HALF, used_, hipMemcpyHostToDevice, st_));
-        STAGE_OK(hipEventRecord(s_.filled[half_], st_));
+        HIP_OK(hipMemcpyAsync(base_, s_.p + half_ * HostStage::HALF, used_, hipMemcpyHostToDevice, st_));
+        HIP_OK(hipEventRecord(s_.filled[half_], st_));
         busy_[half_] = true;
         half_ ^= 1;
         base_ = nullptr;

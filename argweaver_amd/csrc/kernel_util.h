@@ -4,21 +4,10 @@
 
 #include <hip/hip_runtime.h>
 
-#include <cstdio>
-
 #include "engine.h"
+#include "hip_check.h"
 
 namespace aw {
-
-#define HIP_OK(x)                                                                       \
-    do {                                                                                \
-        hipError_t e_ = (x);                                                            \
-        if (e_ != hipSuccess) {                                                         \
-            fprintf(stderr, "argweaver_amd: HIP error %s at %s:%d\n", hipGetErrorString(e_), \
-                    __FILE__, __LINE__);                                                \
-            return 1;                                                                   \
-        }                                                                               \
-    } while (0)
 
 // Pointers read out of DevInst are generic; accesses through them compile to
 // flat instructions, which count against the LDS wait counter too, so every
@@ -60,8 +49,7 @@ __device__ inline int find_owner(PT off, int n, X x)
 // shifts) or outside its 16-lane row (row shifts) receives 0.
 
 constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114,
-              DPP_ROW_SHR8 = 0x118, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138,
-              DPP_QUAD_SWAP1 = 0xB1;   // quad_perm [1,0,3,2]: lanes 2k and 2k+1 swap
+              DPP_ROW_SHR8 = 0x118, DPP_WAVE_SHL1 = 0x130, DPP_WAVE_SHR1 = 0x138;
 
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int x)

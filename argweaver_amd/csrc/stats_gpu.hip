@@ -31,17 +31,8 @@
 namespace aw {
 namespace {
 
-#define LNL_OK(x)                                                                        \
-    do {                                                                                 \
-        hipError_t e_ = (x);                                                             \
-        if (e_ != hipSuccess) {                                                          \
-            fprintf(stderr, "argweaver_amd: %s: %s\n", #x, hipGetErrorString(e_));      \
-            return 1;                                                                    \
-        }                                                                                \
-    } while (0)
-
 struct LnlArgs {
-    int B, N, L, nrows, nleaves;
+    int B, N, L, nrows;
     double mintime, mu;
     const double *times;            // [T]
     const int *parent, *c0, *c1, *age;            // [B*N]
@@ -213,7 +204,7 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
 
     DevBufs m;
     LnlArgs a{};
-    a.B = B; a.N = N; a.L = L; a.nrows = nseqs; a.nleaves = tr.num_leaves();
+    a.B = B; a.N = N; a.L = L; a.nrows = nseqs;
     a.mintime = times[1] * .1;
     a.mu = mu;
     double *dt;
@@ -258,9 +249,9 @@ int arg_loglik_device(const ArgTrees &tr, const double *times, int ntimes, doubl
     hipLaunchKernelGGL(k_lnl_first, dim3((B + 255) / 256), dim3(256), 0, 0, a);
     hipLaunchKernelGGL(k_lnl_eval, dim3(L), dim3(64), 0, 0, a);
     hipLaunchKernelGGL(k_lnl_sum, dim3(nwg), dim3(256), 0, 0, a);
-    LNL_OK(hipGetLastError());
+    HIP_OK(hipGetLastError());
     std::vector<double> part(nwg);
-    LNL_OK(hipMemcpy(part.data(), dpart, sizeof(double) * nwg, hipMemcpyDeviceToHost));
+    HIP_OK(hipMemcpy(part.data(), dpart, sizeof(double) * nwg, hipMemcpyDeviceToHost));
     double s = 0.0;
     for (double x : part) s += x;
     *out = s;
@@ -398,9 +389,9 @@ int arg_logprior_device(const ArgTrees &tr, const Model &model, double *out)
     PriorArgs a{B, N, dm, dp, dag, dspr, dlen, dnext, dterm, dpart};
     hipLaunchKernelGGL(k_prior_block, dim3(B), dim3(64), 0, 0, a);
     hipLaunchKernelGGL(k_sum_terms, dim3(nwg), dim3(256), 0, 0, (const double *)dterm, B, dpart);
-    LNL_OK(hipGetLastError());
+    HIP_OK(hipGetLastError());
     std::vector<double> part(nwg);
-    LNL_OK(hipMemcpy(part.data(), dpart, sizeof(double) * nwg, hipMemcpyDeviceToHost));
+    HIP_OK(hipMemcpy(part.data(), dpart, sizeof(double) * nwg, hipMemcpyDeviceToHost));
     double s = 0.0;
     for (double x : part) s += x;
     *out = s;

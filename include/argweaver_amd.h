@@ -385,8 +385,8 @@ int awamd_batch_run_opts(void *batch, int precision, int tile_cols, int tracebac
                          double *stats);
 /* as awamd_batch_run_opts, with FP32 forward tiles: long instances run as
  * concurrent tiles of fw_tile columns (0: off; FP64 runs ignore it) scaled
- * by 0.94 us over the column cost of the instance's states per lane (so
- * that all tiles take about as long); a tile after the first starts fw_warm
+ * by a planned column cost of the instance's states per lane (so that all
+ * tiles take about as long); a tile after the first starts fw_warm
  * columns early
  * (<= 0: 25000) from a uniform vector, its first stored column is checked
  * against the column computed by the tile before at relative tolerance
@@ -400,7 +400,8 @@ int awamd_batch_run_ex(void *batch, int precision, int tile_cols, int traceback,
 /* Traceback tiles of later runs: warm-up columns of a tile's speculative
  * chain (default 256).  options, 1 .. 4, is checked and has no effect (an
  * earlier traceback kept that many chains per tile; a tile whose chain does not
- * fit is re-run).  The sampled thread is the same for every setting.  0 on success, -1 for a value out of range. */
+ * fit is re-run).  The sampled thread is the same for every setting.  0 on
+ * success, -1 for a value out of range. */
 int awamd_batch_set_traceback(void *batch, int warm, int options);
 /* Traceback tile length of the instances whose FP32 forward tiles are
  * re-run (their traceback runs after the forward: shorter tiles spread it
